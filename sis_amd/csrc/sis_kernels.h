@@ -1005,7 +1005,7 @@ __device__ __forceinline__ void mc_one_component(const Params &P, const Ptrs &D,
   }
   int *sg = seg + gr * SEGCAP;
   if (n <= MCL_PAIRS) {   // small component: one lane, same result
-    if (threadIdx.x == 0 && !mc_component_lane(D, P.N, r, r, root, sg, n, beta, seed, step))
+    if (threadIdx.x == 0 && !mc_component_lane(D, P.max_bp_per_nt, P.N, r, root, sg, n, beta, seed, step))
       mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
     return;
   }
@@ -1023,7 +1023,7 @@ __global__ void __launch_bounds__(64) k_mc_wave(Params P, Ptrs D, int *seg_n, in
   const int64_t step = step_dev ? *step_dev : step0;   // graph replays read the step from the device
   size_t gr = (size_t)r * P.N + root;
   if (!has_exc[gr]) return;
-  __shared__ int ws[MCB_LDS];
+  __shared__ __align__(16) int ws[MCB_LDS];
   mc_one_component(P, D, r, root, seg_n, seg, ecT, seed, step, huge, ws);
 }
 
@@ -1035,7 +1035,7 @@ __global__ void __launch_bounds__(64) k_mc_list(Params P, Ptrs D, int *seg_n, in
                                                 const int64_t *step_dev) {
   const int64_t step = step_dev ? *step_dev : step0;
   const int n = exc_list[0];
-  __shared__ int ws[MCB_LDS];
+  __shared__ __align__(16) int ws[MCB_LDS];
   for (int k = blockIdx.x; k < n; k += gridDim.x) {
     const int gr = exc_list[1 + k];
     const int r = gr / P.N, root = gr - r * P.N;

@@ -65,480 +65,404 @@ __device__ __forceinline__ int below(unsigned long long m) {
 // Orders LDS writes of this wave before its later LDS reads of other lanes' words.
 __device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront"); }
 
-// The Monte Carlo loop of mc_component_wave over its pair slots (IT chunks
-// of 64) and distinct nucleotides (ND chunks of 64), then the write-back of
-// the deleted pairs.  Uniform arguments; all 64 lanes call it.
-template <int IT, int ND>
-__device__ __forceinline__ bool mcg_sweep(const Params &P, const Ptrs &D, int rk, int root, int n, int nn,
-                                          double beta, uint64_t seed, int64_t step, int *sseq, const int (&gb)[IT],
-                                          const int (&ia)[IT], const int (&ib)[IT], const double (&en)[IT],
-                                          bool (&alive)[IT], const int (&nid)[ND], int (&ncnt)[ND]) {
-  constexpr int NP = 64 * IT;
-  const int L = lane_id();
-  // ---- the Monte Carlo loop.  Draws come from a window of 64 counters,
-  // lane i holding draw w0 + i and its logarithm (for the Metropolis test,
-  // log u < dE beta, the same test as u < exp(dE beta)); the window moves
-  // on when an iteration could run past it.
-  uint32_t draw = 0, w0 = 0;
-  double wu = philox_u(seed, rk, step, root, (uint32_t)L), wl = log(wu);
-  // draws above one half: the swap target of a two-pair sequence is 1 there
-  unsigned long long g2 = __ballot(wu > 0.5);
-  const int nchunk_nodes = (nn + 63) / 64;
-  const int nchunk_items = (n + 63) / 64;
-  // live pairs, one 64-bit mask per chunk of pair slots
-  unsigned long long live[IT];
-#pragma unroll
-  for (int k = 0; k < IT; k++) live[k] = __ballot(alive[k]);
-  for (int iter = 0; iter < 4 * NP + 4; iter++) {
-    // active nucleotides (count > 0) in ascending id order
-    int nact = 0;
-    unsigned long long am[ND];
-#pragma unroll
-    for (int q = 0; q < ND; q++) {
-      am[q] = (q < nchunk_nodes) ? __ballot(ncnt[q] > 0) : 0ull;
-      nact += __popcll(am[q]);
-    }
-    if (nact == 0) break;
-    if (draw + 1 > w0 + 64u) {   // the pick draw must be in the window
-      w0 = draw;
-      wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
-      wl = log(wu);
-      g2 = __ballot(wu > 0.5);
-    }
-    const int pick = bcast((int)ceil(wu * nact), (int)(draw - w0));   // 1..nact
-    // the pick-th active nucleotide: its chunk (scalar prefix counts),
-    // then the lane whose prefix count of active lanes is pick - 1
-    int want = pick - 1;
-    unsigned long long amq = am[0];
-    int nidq = nid[0];
-    {
-      int acc = 0;
-      bool found = false;
-#pragma unroll
-      for (int q = 0; q < ND; q++) {
-        const int pc = __popcll(am[q]);
-        const bool here = !found && acc + pc >= pick;
-        want = here ? pick - acc - 1 : want;
-        amq = here ? am[q] : amq;
-        nidq = here ? nid[q] : nidq;
-        found = found || here;
-        acc += pc;
-      }
-    }
-    const int ntd = bcast(nidq, __builtin_ctzll(__ballot(below(amq) == want) & amq));
-    // formed pairs of ntd in list order
-    unsigned long long sm[IT];
-    int ns = 0;
-#pragma unroll
-    for (int k = 0; k < IT; k++) {
-      sm[k] = (k < nchunk_items) ? ((__ballot(ia[k] == ntd) | __ballot(ib[k] == ntd)) & live[k]) : 0ull;
-      ns += __popcll(sm[k]);
-    }
-    if (ns == 0) return false;
-    if (ns > 64) ns = 64;
-    // energy of pair slot `slot` (wave-uniform)
-    auto ene_of = [&](int slot) {
-      const int k = slot >> 6;
-      double x = en[0];
-#pragma unroll
-      for (int kk = 1; kk < IT; kk++) x = (kk == k) ? en[kk] : x;
-      return bcast(x, slot & 63);
-    };
-    int del;
-    if (ns == 2) {
-      // two pairs: the swap sweep leaves them reversed exactly when both
-      // swap draws fall on the same side of one half
-      if (draw + 4u > w0 + 64u) {
-        w0 = draw;
-        wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
-        wl = log(wu);
-        g2 = __ballot(wu > 0.5);
-      }
-      const int o = (int)(draw - w0);
-      int la = -1, lb = -1;
-#pragma unroll
-      for (int k = IT - 1; k >= 0; k--)
-        if (sm[k]) la = 64 * k + __builtin_ctzll(sm[k]);
-#pragma unroll
-      for (int k = 0; k < IT; k++)
-        if (sm[k]) lb = 64 * k + 63 - __builtin_clzll(sm[k]);
-      const unsigned t = (unsigned)(g2 >> (o + 1)) & 3u;
-      const bool flip = t == 0u || t == 3u;
-      const int s0 = flip ? lb : la, s1 = flip ? la : lb;
-      const double e0 = ene_of(s0), w = bcast(wl, o + 3);
-      const int k1 = s1 >> 6;
-      double e1v = en[0];
-#pragma unroll
-      for (int kk = 1; kk < IT; kk++) e1v = (kk == k1) ? en[kk] : e1v;
-      const bool accd = (__ballot(w < (e1v - e0) * beta) >> (s1 & 63)) & 1ull;
-      del = accd ? s1 : s0;
-    } else if (ns <= 8) {
-      // short sequence: kept in scalar registers, entry m in bits
-      // 8m..8m+7 (slots < 256); the window holds the 2 ns draws
-      uint64_t sp = 0;
-      int m = 0;
-#pragma unroll
-      for (int k = 0; k < IT; k++)
-        for (unsigned long long mk = sm[k]; mk; mk &= mk - 1) {
-          sp |= (uint64_t)(64 * k + __builtin_ctzll(mk)) << (8 * m);
-          m++;
-        }
-      if (draw + 2u * (uint32_t)ns > w0 + 64u) {
-        w0 = draw;
-        wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
-        wl = log(wu);
-        g2 = __ballot(wu > 0.5);
-      }
-      const int o = (int)(draw - w0);
-      // swap target of a shuffle draw held by this lane
-      const int swv = (int)ceil(wu * ns) - 1;
-      // reference shuffle: for i = 1..n swap(i, ceil(rnd*n))
-      for (int i = 0; i < ns; i++) {
-        const int sw = bcast(swv, o + 1 + i);
-        const uint64_t x = ((sp >> (8 * i)) ^ (sp >> (8 * sw))) & 0xffull;   // swap entries i and sw
-        sp ^= (x << (8 * i)) | (x << (8 * sw));
-      }
-      // Metropolis sweep on the energies of the sequence's pairs
-      del = (int)(sp & 0xffull);
-      double edel = ene_of(del);
-      for (int i = 1; i < ns; i++) {
-        const int si = (int)((sp >> (8 * i)) & 0xffull);
-        const double ej = ene_of(si);
-        if (bcast(wl, o + ns + i) < (ej - edel) * beta) { del = si; edel = ej; }
-      }
-    } else {
-      // long sequence: entry m in lane m (through LDS)
-#pragma unroll
-      for (int k = 0, m0 = 0; k < IT; k++) {
-        const int m = m0 + below(sm[k]);
-        if (((sm[k] >> L) & 1ull) && m < 64) sseq[m] = 64 * k + L;
-        m0 += __popcll(sm[k]);
-      }
-      wave_lds_fence();
-      int seqv = L < ns ? sseq[L] : 0;
-      // draws used: 1 (pick) + ns (shuffle) + ns - 1 (Metropolis) = 2 ns;
-      // a window holding all of them starts at this iteration's pick draw
-      const bool fits = 2 * ns <= 64;
-      if (fits && draw + 2u * (uint32_t)ns > w0 + 64u) {
-        w0 = draw;
-        wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
-        wl = log(wu);
-        g2 = __ballot(wu > 0.5);
-      }
-      const int o = (int)(draw - w0);
-      // u and log u of the draw `k` places after the pick draw
-      auto du = [&](int k) { return fits ? bcast(wu, o + k) : philox_u(seed, rk, step, root, draw + (uint32_t)k); };
-      auto dlog = [&](int k) { return fits ? bcast(wl, o + k) : log(philox_u(seed, rk, step, root, draw + (uint32_t)k)); };
-      // swap targets of the shuffle, lane i holding the i-th
-      const int swl = fits ? (int)ceil(__shfl(wu, (o + 1 + L) & 63) * ns) - 1 : 0;
-      for (int i = 0; i < ns; i++) {
-        const int sw = fits ? bcast(swl, i) : (int)ceil(du(1 + i) * ns) - 1;
-        const int ti = bcast(seqv, i), ts = bcast(seqv, sw);
-        seqv = setlane(seqv, ts, i);
-        seqv = setlane(seqv, ti, sw);
-      }
-      del = bcast(seqv, 0);
-      double edel = ene_of(del);
-      for (int i = 1; i < ns; i++) {
-        const int si = bcast(seqv, i);
-        const double ej = ene_of(si);
-        if (dlog(ns + i) < (ej - edel) * beta) { del = si; edel = ej; }
-      }
-    }
-    draw += 2u * (uint32_t)ns;
-    // delete: pair slot del, decrement its two nucleotides
-    const int dk = del >> 6, dl = del & 63;
-    int xa = ia[0], xb = ib[0];
-#pragma unroll
-    for (int k = 1; k < IT; k++) {
-      xa = (k == dk) ? ia[k] : xa;
-      xb = (k == dk) ? ib[k] : xb;
-    }
-    const int da = bcast(xa, dl), db = bcast(xb, dl);
-#pragma unroll
-    for (int k = 0; k < IT; k++)
-      if (k == dk) live[k] &= ~(1ull << dl);
-#pragma unroll
-    for (int q = 0; q < ND; q++) ncnt[q] -= (nid[q] == da) + (nid[q] == db);
-  }
-#pragma unroll
-  for (int k = 0; k < IT; k++) alive[k] = (live[k] >> L) & 1ull;
-  // write back the pairs deleted here
-#pragma unroll
-  for (int k = 0; k < IT; k++) {
-    const int t = L + 64 * k;
-    if (t < n && !alive[k]) D.bp_status[gb[k]] = 0;
-  }
-  return true;
+// Prefix sum, minimum and maximum over the 64 lanes by DPP row shifts and
+// row broadcasts: register traffic, no LDS round trip.
+template <typename F>
+__device__ __forceinline__ int wave_scan(int v, int id, F f) {
+  v = f(v, __builtin_amdgcn_update_dpp(id, v, 0x111, 0xf, 0xf, false));   // row_shr:1
+  v = f(v, __builtin_amdgcn_update_dpp(id, v, 0x112, 0xf, 0xf, false));   // row_shr:2
+  v = f(v, __builtin_amdgcn_update_dpp(id, v, 0x114, 0xf, 0xf, false));   // row_shr:4
+  v = f(v, __builtin_amdgcn_update_dpp(id, v, 0x118, 0xf, 0xf, false));   // row_shr:8
+  v = f(v, __builtin_amdgcn_update_dpp(id, v, 0x142, 0xa, 0xf, false));   // row_bcast:15
+  return f(v, __builtin_amdgcn_update_dpp(id, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
+}
+__device__ __forceinline__ int wave_min(int v) {
+  return bcast(wave_scan(v, 0x7fffffff, [](int a, int b) { return a < b ? a : b; }), 63);
+}
+__device__ __forceinline__ int wave_max(int v) {
+  return bcast(wave_scan(v, (int)0x80000000, [](int a, int b) { return a > b ? a : b; }), 63);
 }
 
-// Resolve the component whose formed pairs are seg[0..n) (candidate ids,
-// any order).  Must be called by all 64 lanes of a wave with uniform
-// arguments; ws is mcw_lds(IT) ints of LDS private to the wave.  Returns
-// false if the component exceeds the capacity of 64*IT pairs.  The result
-// does not depend on IT (same draws, same decisions).  r indexes the per-replica
-// arrays; rk keys the random stream.
-// Layout: pair slot t (candidate-id order) lives in lane t % 64, chunk
-// t / 64; nucleotide slot u (ascending id) in lane u % 64, chunk u / 64;
-// the pair sequence of one iteration holds entry m in lane m.
-template <int IT = MCW_ITEMS, int ND = MCW_NODES>
-__device__ __forceinline__ bool mc_component_wave(const Params &P, const Ptrs &D, int r, int rk, int root,
-                                                  const int *seg, int n, double beta, uint64_t seed,
-                                                  int64_t step, int *ws) {
-  constexpr int NONE = 0x7fffffff;
-  constexpr int NP = 64 * IT, NE = 2 * NP;
-  static_assert(NP <= 256, "pair slots are packed in 8 bits");
+// Ranks of the values v[k] (where ok[k]) among the distinct values held by
+// the wave, ascending; returns how many distinct ones there are, or -1 when
+// they span more than the 2,048 bits of the bitmap (bm, pre: 64 ints of LDS
+// each).  A bit per value, a prefix count over the 64 words and two LDS
+// reads a value: a few hundred cycles whatever the number of values, where
+// comparing each with all others took thousands.
+template <int K>
+__device__ __forceinline__ int wave_rank(const int (&v)[K], const bool (&ok)[K], int *bm, int *pre, int (&rank)[K]) {
   const int L = lane_id();
-  const int N = P.N;
-  // uniform by contract; said so to the compiler, so that loop counters
-  // and lane indices stay scalar
-  n = __builtin_amdgcn_readfirstlane(n);
-  root = __builtin_amdgcn_readfirstlane(root);
-  if (n > NP) return false;
-  const int nc = 2 * n;
-  int *sraw = ws, *ssort = ws + NP, *send = ws + 2 * NP, *sflag = ws + 2 * NP + NE, *sseq = ws + 2 * NP + 2 * NE;
-  // ---- pairs in candidate-id order (= reference list order): rank by
-  // comparing against all ids (4 per LDS read), then scatter by rank
-  const int n4 = (n + 3) & ~3;
-  int raw[IT];
+  int lo = 0x7fffffff, hi = -1;
 #pragma unroll
-  for (int k = 0; k < IT; k++) {
-    const int t = L + 64 * k;
-    raw[k] = t < n ? seg[t] : NONE;
-    if (t < n4) sraw[t] = raw[k];
-  }
-  wave_lds_fence();
-  int rank[IT] = {};
-  for (int j = 0; j < n4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(sraw + j);
-#pragma unroll
-    for (int k = 0; k < IT; k++)
-      rank[k] += (v.x < raw[k]) + (v.y < raw[k]) + (v.z < raw[k]) + (v.w < raw[k]);
-  }
-#pragma unroll
-  for (int k = 0; k < IT; k++)
-    if (L + 64 * k < n) ssort[rank[k]] = raw[k];
-  wave_lds_fence();
-  int gb[IT], ia[IT], ib[IT];
-  double en[IT];
-  bool alive[IT];
-  bool bad = false;
-#pragma unroll
-  for (int k = 0; k < IT; k++) {
-    const int t = L + 64 * k;
-    alive[k] = t < n;
-    gb[k] = NONE;
-    ia[k] = ib[k] = -1;
-    en[k] = 0.0;
-    if (alive[k]) {
-      gb[k] = ssort[t];
-      const int *mp = D.bp_mp + (size_t)gb[k] * 8;
-      ia[k] = mp[0] - 1;
-      ib[k] = mp[1] - 1;
-      en[k] = D.ene_bp[gb[k]];
-      bad = bad || ia[k] < 0 || ia[k] >= N || ib[k] < 0 || ib[k] >= N;
+  for (int k = 0; k < K; k++)
+    if (ok[k]) {
+      lo = v[k] < lo ? v[k] : lo;
+      hi = v[k] > hi ? v[k] : hi;
     }
-  }
-  // a candidate naming a bead outside the system means corrupted MC state:
-  // report it (flags[7]) instead of indexing with it
-  if (__ballot(bad)) {
-    if (L == 0) D.flags[7] = 1;
-    return true;
-  }
-  // ---- distinct nucleotides in ascending id order, with their counts.
-  // Endpoint c = 2t (+1) is nucleotide a (b) of pair slot t.
-  const int nc4 = (nc + 3) & ~3;
+  lo = wave_min(lo);
+  hi = wave_max(hi);
+  if (hi - lo >= 2048) return -1;
+  bm[L] = 0;
+  wave_lds_fence();
 #pragma unroll
-  for (int k = 0; k < IT; k++) {
+  for (int k = 0; k < K; k++)
+    if (ok[k]) atomicOr(&bm[(v[k] - lo) >> 5], 1 << ((v[k] - lo) & 31));
+  wave_lds_fence();
+  const int c = __popc((unsigned)bm[L]);
+  const int inc = wave_scan(c, 0, [](int a, int b) { return a + b; });
+  pre[L] = inc - c;
+  wave_lds_fence();
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    const int d = ok[k] ? v[k] - lo : 0;
+    rank[k] = pre[d >> 5] + __popc((unsigned)bm[d >> 5] & ((1u << (d & 31)) - 1u));
+  }
+  wave_lds_fence();
+  return bcast(inc, 63);
+}
+
+// wave_rank for values of any span (a component between chains whose beads
+// are numbered far apart): every value compared with all `nv` (value k of
+// lane L is number L + 64 k; all: nv rounded up to 4 ints of LDS, first: as
+// many).  Kept rolled: a launch meets this code cold, and the fetch of an
+// unrolled body took longer than the loop (17,000 cycles against 25,000 for
+// a 26-pair component).
+template <int K>
+__device__ __forceinline__ int wave_rank_any(const int (&v)[K], int nv, int *all, int *first, int (&rank)[K]) {
+  constexpr int NONE = 0x7fffffff;
+  const int L = lane_id();
+  const int n4 = (nv + 3) & ~3;
+  bool f[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
     const int t = L + 64 * k;
-    if (t < n) {
-      send[2 * t] = ia[k];
-      send[2 * t + 1] = ib[k];
-    } else if (2 * t < nc4) {
-      send[2 * t] = NONE;
-      send[2 * t + 1] = NONE;
-    }
+    f[k] = t < nv;
+    rank[k] = 0;
+    if (t < n4) all[t] = t < nv ? v[k] : NONE;
   }
   wave_lds_fence();
-  // first occurrence of each endpoint value
-  int ev[ND];
-  bool first[ND];
+  for (int j = 0; j < nv; j++) {
+    const int x = all[j];
 #pragma unroll
-  for (int q = 0; q < ND; q++) {
-    const int c = L + 64 * q;
-    ev[q] = c < nc ? send[c] : NONE;
-    first[q] = c < nc;
+    for (int k = 0; k < K; k++)
+      if (j < L + 64 * k && x == v[k]) f[k] = false;
   }
-  for (int j = 0; j < nc4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(send + j);
-#pragma unroll
-    for (int q = 0; q < ND; q++) {
-      const int c = L + 64 * q;
-      if ((j < c && v.x == ev[q]) || (j + 1 < c && v.y == ev[q]) || (j + 2 < c && v.z == ev[q]) ||
-          (j + 3 < c && v.w == ev[q]))
-        first[q] = false;
-    }
-  }
-#pragma unroll
-  for (int q = 0; q < ND; q++) {
-    const int c = L + 64 * q;
-    if (c < nc4) sflag[c] = first[q] ? ev[q] : NONE;   // first occurrences only
-  }
-  wave_lds_fence();
-  // rank among distinct values, then scatter
   int nn = 0;
 #pragma unroll
-  for (int q = 0; q < ND; q++) nn += __popcll(__ballot(first[q]));
-  int urank[ND] = {};
-  for (int j = 0; j < nc4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(sflag + j);
-#pragma unroll
-    for (int q = 0; q < ND; q++)
-      urank[q] += (v.x < ev[q]) + (v.y < ev[q]) + (v.z < ev[q]) + (v.w < ev[q]);
+  for (int k = 0; k < K; k++) {
+    const int t = L + 64 * k;
+    if (t < n4) first[t] = f[k] ? v[k] : NONE;
+    nn += __popcll(__ballot(f[k]));
   }
-#pragma unroll
-  for (int q = 0; q < ND; q++)
-    if (first[q]) send[urank[q]] = ev[q];   // endpoints no longer needed
   wave_lds_fence();
-  int nid[ND], ncnt[ND];
+  for (int j = 0; j < nv; j++) {
+    const int x = first[j];
 #pragma unroll
-  for (int q = 0; q < ND; q++) {
-    const int u = L + 64 * q;
-    nid[q] = u < nn ? send[u] : NONE;
-    ncnt[q] = u < nn ? D.nt_cnt[(size_t)r * N + nid[q]] : 0;
+    for (int k = 0; k < K; k++) rank[k] += x < v[k];
   }
-  // the sweep runs over as few nucleotide chunks as the component needs:
-  // two for at most 128 distinct nucleotides (nearly all components), four
-  // for at most 256
-  if (ND > 2 && nn <= 128) {
-    const int nid2[2] = {nid[0], nid[1]};
-    int ncnt2[2] = {ncnt[0], ncnt[1]};
-    return mcg_sweep<IT, 2>(P, D, rk, root, n, nn, beta, seed, step, sseq, gb, ia, ib, en, alive, nid2, ncnt2);
-  }
-  if (ND > 4 && nn <= 256) {
-    const int nid4[4] = {nid[0], nid[1], nid[2], nid[3]};
-    int ncnt4[4] = {ncnt[0], ncnt[1], ncnt[2], ncnt[3]};
-    return mcg_sweep<IT, 4>(P, D, rk, root, n, nn, beta, seed, step, sseq, gb, ia, ib, en, alive, nid4, ncnt4);
-  }
-  return mcg_sweep<IT, ND>(P, D, rk, root, n, nn, beta, seed, step, sseq, gb, ia, ib, en, alive, nid, ncnt);
+  wave_lds_fence();
+  return nn;
 }
 
-// ---------------------------------------------------------------------
-// The same sweep for a component of at most 64 pairs (the usual size),
-// with one pair per lane and the bookkeeping in scalar registers: the live
-// pairs are a 64-bit mask, the nucleotides two slots per lane, the sequence
-// of up to 8 pairs held as a 4-bit permutation of their ranks.  A single
-// wavefront runs this serially, so its cost is the latency of its chain of
-// lane reads and ballots (each about 25-30 cycles on gfx950); the common
-// two-pair case resolves its swap sweep from one ballot of the block of
-// draws taken at each refill.  Draws and decisions are those of
-// mc_component_wave.  Returns false (having written nothing) if the
-// component is larger, a nucleotide has more than 8 formed pairs, or the
-// state is inconsistent; the caller then runs the general form from the
-// start, which reproduces the same result.
-__device__ __forceinline__ bool mc_component_wave64(const Params &P, const Ptrs &D, int r, int rk, int root,
-                                                    const int *seg, int n, double beta, uint64_t seed, int64_t step,
-                                                    int *ws) {
-  constexpr int NONE = 0x7fffffff;
+// The pick among nact active nucleotides, ceil(u nact) - 1, with the draw
+// of lane o (wu, its upper 32 bits wh): floor(u nact) unless the product is
+// a whole number, which the upper 32 bits exclude except next to one.
+__device__ __forceinline__ int mc_pick(unsigned wh, double wu, int nact, int o) {
+  const uint64_t pr = (uint64_t)(unsigned)bcast((int)wh, o) * (unsigned)nact;
+  if ((unsigned)pr - 2u <= 0xffffffe0u - (unsigned)nact) return (int)(pr >> 32);
+  return bcast((int)ceil(wu * nact), o) - 1;
+}
+
+// The Monte Carlo loop of mc_component_wave over its pair slots (IT chunks
+// of 64: endpoints ua, ub as nucleotide slots, energies en) and nucleotides
+// (ND chunks of 64: excess counts cnt).  live: the pairs left at the end.
+// Uniform arguments; all 64 lanes call it.
+//
+// One deletion is a chain of dependent scalar and lane operations, and its
+// latency is the kernel's time, so as little as possible stays on the
+// chain.  Most nucleotides of a large component have two pairs, and for
+// those every nucleotide's lane works out beforehand which of its two it
+// would delete with the draws to come: the two pairs (F, G: slot << 9 |
+// other nucleotide) and the Metropolis argument D = dE beta change only when
+// the nucleotide itself loses its third pair.  The chain is then: count of
+// active nucleotides, pick (mc_pick: a 32-bit multiply for an FP64 product,
+// ceiling and conversion), the lane of the picked bit, its answer, the
+// partner's count.  With wave_rank for the two sorts of the set-up (each
+// took a loop over all pairs) a step of 256 replicas of 128 nt went from
+// 85 to 75 us.
+template <int IT, int ND>
+__device__ __forceinline__ bool mc_sweep(int max_bp, int rk, int root, int n, double beta, uint64_t seed, int64_t step,
+                                         int *ws, const int (&ua)[IT], const int (&ub)[IT], const double (&en)[IT],
+                                         const int (&cnt)[ND], unsigned long long (&live)[IT]) {
+  static_assert(ND <= 8, "excess counts are packed in bytes");
   const int L = lane_id();
-  const int N = P.N;
-  n = __builtin_amdgcn_readfirstlane(n);
-  root = __builtin_amdgcn_readfirstlane(root);
-  if (n > 64) return false;
-  int *sraw = ws, *ssort = ws + 64, *send = ws + 128, *sflag = ws + 256;   // 384 ints
-  // ---- pairs in candidate-id order: rank by comparison, scatter
-  const int n4 = (n + 3) & ~3;
-  const int raw = L < n ? seg[L] : NONE;
-  if (L < n4) sraw[L] = raw;
-  wave_lds_fence();
-  int rank = 0;
-  for (int j = 0; j < n4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(sraw + j);
-    rank += (v.x < raw) + (v.y < raw) + (v.z < raw) + (v.w < raw);
-  }
-  if (L < n) ssort[rank] = raw;
-  wave_lds_fence();
-  int gb = NONE, ia = -1, ib = -1;
-  double en = 0.0;
-  bool bad = false;
-  if (L < n) {
-    gb = ssort[L];
-    const int *mp = D.bp_mp + (size_t)gb * 8;
-    ia = mp[0] - 1;
-    ib = mp[1] - 1;
-    en = D.ene_bp[gb];
-    bad = ia < 0 || ia >= N || ib < 0 || ib >= N;
-  }
-  if (__ballot(bad)) return false;
-  // ---- distinct nucleotides in ascending id order (slots L and 64 + L)
-  const int nc = 2 * n, nc4 = (nc + 3) & ~3;
-  if (L < n) {
-    send[2 * L] = ia;
-    send[2 * L + 1] = ib;
-  } else if (2 * L < nc4) {
-    send[2 * L] = NONE;
-    send[2 * L + 1] = NONE;
+  const int c2 = 2 - max_bp;   // excess count of a nucleotide with two pairs
+  int *sseq = ws, *sfirst = ws + 64 + 128 * IT, *slast = sfirst + 64 * ND;
+  double *sen = reinterpret_cast<double *>(ws + 64);
+  // ---- first and last pair of every nucleotide
+#pragma unroll
+  for (int q = 0; q < ND; q++) {
+    sfirst[L + 64 * q] = 0x7fffffff;
+    slast[L + 64 * q] = -1;
   }
   wave_lds_fence();
-  const int c1 = 64 + L;
-  const int ev0 = L < nc ? send[L] : NONE, ev1 = c1 < nc ? send[c1] : NONE;
-  bool f0 = L < nc, f1 = c1 < nc;
-  for (int j = 0; j < nc4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(send + j);
-    if ((j < L && v.x == ev0) || (j + 1 < L && v.y == ev0) || (j + 2 < L && v.z == ev0) || (j + 3 < L && v.w == ev0))
-      f0 = false;
-    if ((j < c1 && v.x == ev1) || (j + 1 < c1 && v.y == ev1) || (j + 2 < c1 && v.z == ev1) ||
-        (j + 3 < c1 && v.w == ev1))
-      f1 = false;
-  }
-  if (L < nc4) sflag[L] = f0 ? ev0 : NONE;
-  if (c1 < nc4) sflag[c1] = f1 ? ev1 : NONE;
-  wave_lds_fence();
-  const int nn = __popcll(__ballot(f0)) + __popcll(__ballot(f1));
-  int u0 = 0, u1 = 0;
-  for (int j = 0; j < nc4; j += 4) {
-    const int4 v = *reinterpret_cast<const int4 *>(sflag + j);
-    u0 += (v.x < ev0) + (v.y < ev0) + (v.z < ev0) + (v.w < ev0);
-    u1 += (v.x < ev1) + (v.y < ev1) + (v.z < ev1) + (v.w < ev1);
-  }
-  if (f0) send[u0] = ev0;
-  if (f1) send[u1] = ev1;
-  wave_lds_fence();
-  const int nid0 = L < nn ? send[L] : NONE, nid1 = c1 < nn ? send[c1] : NONE;
-  int cnt0 = L < nn ? D.nt_cnt[(size_t)r * N + nid0] : 0;
-  int cnt1 = c1 < nn ? D.nt_cnt[(size_t)r * N + nid1] : 0;
-  // ---- the sweep
-  unsigned long long live = __ballot(L < n);
-  uint32_t draw = 0, w0 = 0;
-  double wu = philox_u(seed, rk, step, root, (uint32_t)L), wl = log(wu);
-  // draws above one half: the swap target of a two-pair sequence is 1 there
-  unsigned long long g2 = __ballot(wu > 0.5);
-  for (int iter = 0; iter < 4 * 64 + 4; iter++) {
-    const unsigned long long a0 = __ballot(cnt0 > 0), a1 = __ballot(cnt1 > 0);
-    const int p0 = __popcll(a0), nact = p0 + __popcll(a1);
-    if (nact == 0) break;
-    if (draw + 1 > w0 + 64u) {
-      w0 = draw;
-      wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
-      wl = log(wu);
-      g2 = __ballot(wu > 0.5);
+#pragma unroll
+  for (int k = 0; k < IT; k++) {
+    const int t = L + 64 * k;
+    live[k] = __ballot(t < n);
+    if (t < n) {
+      sen[t] = en[k];
+      atomicMin(&sfirst[ua[k]], t << 9 | ub[k]);
+      atomicMax(&slast[ua[k]], t << 9 | ub[k]);
+      atomicMin(&sfirst[ub[k]], t << 9 | ua[k]);
+      atomicMax(&slast[ub[k]], t << 9 | ua[k]);
     }
-    const int pick = bcast((int)ceil(wu * nact), (int)(draw - w0));   // 1..nact
-    const bool upper = pick > p0;
-    const unsigned long long am = upper ? a1 : a0;
-    const int want = upper ? pick - p0 - 1 : pick - 1;
-    const int ln = __builtin_ctzll(__ballot(below(am) == want) & am);
-    const int ntd = bcast(upper ? nid1 : nid0, ln);
-    const unsigned long long sm = (__ballot(ia == ntd) | __ballot(ib == ntd)) & live;
-    const int ns = __popcll(sm);
-    if (ns == 0 || ns > 8) return false;
-    if (draw + 2u * (uint32_t)ns > w0 + 64u) {
+  }
+  wave_lds_fence();
+  int F[ND], G[ND];
+  double D[ND];
+  unsigned long long am[ND];   // active nucleotides (excess > 0)
+  unsigned c0 = 0, c1 = 0;     // their excess (at most 255), a byte for each chunk
+#pragma unroll
+  for (int q = 0; q < ND; q++) {
+    const unsigned e = cnt[q] > 0 ? (unsigned)cnt[q] << (8 * (q & 3)) : 0u;
+    if (q < 4) c0 |= e; else c1 |= e;
+    F[q] = G[q] = -1;
+    D[q] = 0.0;
+    am[q] = __ballot(cnt[q] > 0);
+    if (cnt[q] > 0 && cnt[q] == c2) {
+      F[q] = sfirst[L + 64 * q];
+      G[q] = slast[L + 64 * q];
+      D[q] = (sen[G[q] >> 9] - sen[F[q] >> 9]) * beta;
+    }
+  }
+  wave_lds_fence();
+  // energy of pair slot `slot` (wave-uniform)
+  auto ene_of = [&](int slot) {
+    double x = en[0];
+#pragma unroll
+    for (int k = 1; k < IT; k++) x = (slot >> 6) == k ? en[k] : x;
+    return bcast(x, slot & 63);
+  };
+  // the other nucleotide of pair slot `slot` of nucleotide x
+  auto partner_of = [&](int slot, int x) {
+    int a = ua[0], b = ub[0];
+#pragma unroll
+    for (int k = 1; k < IT; k++) {
+      a = (slot >> 6) == k ? ua[k] : a;
+      b = (slot >> 6) == k ? ub[k] : b;
+    }
+    return bcast(a, slot & 63) + bcast(b, slot & 63) - x;
+  };
+  // nucleotide x loses a pair: no longer active, or down to its last two
+  // pairs, where its answer is worked out
+  auto lose_one = [&](int x) {
+    const int sh = 8 * ((x >> 6) & 3);
+    const bool hi = ND > 4 && x >= 256;
+    const int was = (bcast((int)(hi ? c1 : c0), x & 63) >> sh) & 255;
+    if (was == 0) return;
+    const unsigned one = L == (x & 63) ? 1u << sh : 0u;
+    if (hi) c1 -= one; else c0 -= one;
+    const int c = was - 1;
+    if (c == 0) {
+#pragma unroll
+      for (int q = 0; q < ND; q++)
+        if ((x >> 6) == q) am[q] &= ~(1ull << (x & 63));
+    } else if (c == c2) {
+      int la = -1, lb = -1;
+#pragma unroll
+      for (int k = 0; k < IT; k++) {
+        const unsigned long long m = (__ballot(ua[k] == x) | __ballot(ub[k] == x)) & live[k];
+        if (m) {
+          if (la < 0) la = 64 * k + __builtin_ctzll(m);
+          lb = 64 * k + 63 - __builtin_clzll(m);
+        }
+      }
+      if (la < 0) return;   // counts and pairs disagree: the pick finds it
+      const int f = la << 9 | partner_of(la, x), g = lb << 9 | partner_of(lb, x);
+      const double d = (ene_of(lb) - ene_of(la)) * beta;
+#pragma unroll
+      for (int q = 0; q < ND; q++) {
+        const bool me = L + 64 * q == x;
+        F[q] = me ? f : F[q];
+        G[q] = me ? g : G[q];
+        D[q] = me ? d : D[q];
+      }
+    }
+  };
+  // ---- draws: a window of 64 counters, lane i holding draw w0 + i, its
+  // logarithm (Metropolis test: log u < dE beta) and its upper 32 bits;
+  // g2: draws above one half (the swap target of a two-pair sequence)
+  uint32_t draw = 0, w0 = (uint32_t)-64;
+  double wu = 0.0, wl = 0.0;
+  unsigned wh = 0;
+  unsigned long long g2 = 0;
+  for (;;) {
+    int pc[ND], nact = 0;
+#pragma unroll
+    for (int q = 0; q < ND; q++) {
+      pc[q] = __popcll(am[q]);
+      nact += pc[q];
+    }
+    if (nact == 0) return true;
+    if ((int)(draw - w0) > 64 - 16) {   // the window holds any sequence of up to eight pairs
       w0 = draw;
       wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
       wl = log(wu);
+      wh = (unsigned)(wu * 4294967296.0);
       g2 = __ballot(wu > 0.5);
     }
     const int o = (int)(draw - w0);
+    // what every nucleotide with two pairs would delete: the swap sweep
+    // leaves its pairs reversed exactly when both swap draws fall on the
+    // same side of one half; then one Metropolis test
+    const unsigned t2 = (unsigned)(g2 >> (o + 1)) & 3u;
+    const bool flip = t2 == 0u || t2 == 3u;
+    // in list order the first goes when w >= D; reversed, when D < -w: the
+    // same comparison with the double below -w (w < 0)
+    const long long wb = __double_as_longlong(bcast(wl, o + 3));
+    const double w = __longlong_as_double(flip ? (wb ^ (1ll << 63)) - 1 : wb);
+    int R[ND];
+#pragma unroll
+    for (int q = 0; q < ND; q++) R[q] = D[q] <= w ? F[q] : G[q];
+    int want = mc_pick(wh, wu, nact, o);
+    unsigned long long amq = am[0];
+    int base = 0;
+#pragma unroll
+    for (int q = 1; q < ND; q++) {
+      const bool next = base == 64 * (q - 1) && want >= pc[q - 1];
+      want = next ? want - pc[q - 1] : want;
+      amq = next ? am[q] : amq;
+      base = next ? 64 * q : base;
+    }
+    int Rq = R[0];
+#pragma unroll
+    for (int q = 1; q < ND; q++) Rq = base == 64 * q ? R[q] : Rq;
+    const int ln = __builtin_ctzll(__ballot(below(amq) == want) & amq);
+    const int ntd = base + ln;
+    int got = bcast(Rq, ln);
+    int ns = 2;
+    if (got < 0) {
+      // three pairs or more: ntd's pairs in list order
+      unsigned long long sm[IT];
+      ns = 0;
+#pragma unroll
+      for (int k = 0; k < IT; k++) {
+        sm[k] = (__ballot(ua[k] == ntd) | __ballot(ub[k] == ntd)) & live[k];
+        ns += __popcll(sm[k]);
+      }
+      if (ns == 0) return false;
+      if (ns > 64) ns = 64;
+      // draws used: 1 (pick) + ns (shuffle) + ns - 1 (Metropolis) = 2 ns
+      int del;
+      if (ns <= 8) {
+        // short sequence: kept in scalar registers, entry m in bits
+        // 8m..8m+7 (slots < 256)
+        uint64_t sp = 0;
+        int m = 0;
+#pragma unroll
+        for (int k = 0; k < IT; k++)
+          for (unsigned long long mk = sm[k]; mk; mk &= mk - 1) {
+            sp |= (uint64_t)(64 * k + __builtin_ctzll(mk)) << (8 * m);
+            m++;
+          }
+        const int swv = 8 * ((int)ceil(wu * ns) - 1);
+        // reference shuffle: for i = 1..n swap(i, ceil(rnd*n))
+        for (int i = 0; i < 8 * ns; i += 8) {
+          const int sw = bcast(swv, o + 1 + (i >> 3));
+          const uint64_t x = ((sp >> i) ^ (sp >> sw)) & 0xffull;   // swap entries i and sw
+          sp ^= (x << i) | (x << sw);
+        }
+        // Metropolis sweep on the energies of the sequence's pairs
+        del = (int)(sp & 0xffull);
+        double edel = ene_of(del);
+        for (int i = 1; i < ns; i++) {
+          const int si = (int)((sp >> (8 * i)) & 0xffull);
+          const double ej = ene_of(si);
+          if (bcast(wl, o + ns + i) < (ej - edel) * beta) { del = si; edel = ej; }
+        }
+      } else {
+        // long sequence: entry m in lane m (through LDS)
+#pragma unroll
+        for (int k = 0, m0 = 0; k < IT; k++) {
+          const int m = m0 + below(sm[k]);
+          if (((sm[k] >> L) & 1ull) && m < 64) sseq[m] = 64 * k + L;
+          m0 += __popcll(sm[k]);
+        }
+        wave_lds_fence();
+        int seqv = L < ns ? sseq[L] : 0;
+        // lane i: the i-th swap target, and the logarithm of the draw that
+        // decides on entry i
+        const double us = philox_u(seed, rk, step, root, draw + 1u + (uint32_t)L);
+        const double ul = log(philox_u(seed, rk, step, root, draw + (uint32_t)(ns + L)));
+        const int swl = (int)ceil(us * ns) - 1;
+        for (int i = 0; i < ns; i++) {
+          const int sw = bcast(swl, i);
+          const int ti = bcast(seqv, i), ts = bcast(seqv, sw);
+          seqv = setlane(seqv, ts, i);
+          seqv = setlane(seqv, ti, sw);
+        }
+        del = bcast(seqv, 0);
+        double edel = ene_of(del);
+        for (int i = 1; i < ns; i++) {
+          const int si = bcast(seqv, i);
+          const double ej = ene_of(si);
+          if (bcast(ul, i) < (ej - edel) * beta) { del = si; edel = ej; }
+        }
+        wave_lds_fence();
+      }
+      got = del << 9 | partner_of(del, ntd);
+    }
+    draw += 2u * (uint32_t)ns;
+    const int del = got >> 9, other = got & 511;
+#pragma unroll
+    for (int k = 0; k < IT; k++)
+      if ((del >> 6) == k) live[k] &= ~(1ull << (del & 63));
+    lose_one(ntd);
+    lose_one(other);
+  }
+}
+
+// The same loop for components of at most 64 pairs and 128 nucleotides, one
+// pair and two nucleotides a lane: the live pairs are one 64-bit mask, and
+// a sequence of up to 8 pairs a 4-bit permutation of their ranks.  These
+// components are short and dense (three pairs a nucleotide and more), where
+// a deletion's time is the number of instructions on it, so nothing is
+// worked out ahead: 1,250 cycles a deletion (34 deletions of a 40-pair
+// component in 42,000) against 2,000 for the loop above and 1,700 with the
+// FP64 pick.  Its loops stay rolled: unrolled ones gained 5% on such a
+// component and lost 30% on one of five pairs, to instruction fetch.
+// Returns false if a nucleotide has more than 8 formed
+// pairs or the state is inconsistent (the caller then runs the general loop
+// from the start, which gives the same result).
+__device__ __forceinline__ bool mc_sweep64(int rk, int root, int n, double beta, uint64_t seed, int64_t step,
+                                           int ua, int ub, double en, int cnt0, int cnt1, unsigned long long &live) {
+  const int L = lane_id();
+  live = __ballot(L < n);
+  uint32_t draw = 0, w0 = (uint32_t)-64;
+  double wu = 0.0, wl = 0.0;
+  unsigned wh = 0;
+  unsigned long long g2 = 0;
+  for (;;) {
+    const unsigned long long a0 = __ballot(cnt0 > 0), a1 = __ballot(cnt1 > 0);
+    const int p0 = __popcll(a0), nact = p0 + __popcll(a1);
+    if (nact == 0) return true;
+    if ((int)(draw - w0) > 64 - 16) {   // the window holds any sequence of up to eight pairs
+      w0 = draw;
+      wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
+      wl = log(wu);
+      wh = (unsigned)(wu * 4294967296.0);
+      g2 = __ballot(wu > 0.5);
+    }
+    const int o = (int)(draw - w0);
+    const int want0 = mc_pick(wh, wu, nact, o);
+    const bool upper = want0 >= p0;
+    const unsigned long long am = upper ? a1 : a0;
+    const int want = upper ? want0 - p0 : want0;
+    const int ntd = __builtin_ctzll(__ballot(below(am) == want) & am) + (upper ? 64 : 0);
+    const unsigned long long sm = (__ballot(ua == ntd) | __ballot(ub == ntd)) & live;
+    const int ns = __popcll(sm);
+    if (ns == 0 || ns > 8) return false;
     int del;
     if (ns == 2) {
       // two pairs: the swap sweep leaves them reversed exactly when both
@@ -551,14 +475,14 @@ __device__ __forceinline__ bool mc_component_wave64(const Params &P, const Ptrs 
       const bool acc = (__ballot(w < (en - e0) * beta) >> s1) & 1ull;
       del = acc ? s1 : s0;
     } else {
-      const int swv = (int)ceil(wu * ns) - 1;
       // ntd's pairs in list order are the set bits of sm in lane order (rank
       // 0..ns-1); perm holds the rank at each sequence slot, 4 bits a slot
+      const int swv = 4 * ((int)ceil(wu * ns) - 1);
       uint32_t perm = 0x76543210u;
       for (int i = 0; i < ns; i++) {
         const int sw = bcast(swv, o + 1 + i);
-        const uint32_t x = ((perm >> (4 * i)) ^ (perm >> (4 * sw))) & 15u;
-        perm ^= (x << (4 * i)) | (x << (4 * sw));
+        const uint32_t x = ((perm >> (4 * i)) ^ (perm >> sw)) & 15u;
+        perm ^= (x << (4 * i)) | (x << sw);
       }
       const int rkl = below(sm);
       del = __builtin_ctzll(__ballot(rkl == (int)(perm & 15u)) & sm);
@@ -571,171 +495,168 @@ __device__ __forceinline__ bool mc_component_wave64(const Params &P, const Ptrs 
     }
     draw += 2u * (uint32_t)ns;
     live &= ~(1ull << del);
-    const int da = bcast(ia, del), db = bcast(ib, del);
-    cnt0 -= (nid0 == da) + (nid0 == db);
-    cnt1 -= (nid1 == da) + (nid1 == db);
+    const int da = bcast(ua, del), db = bcast(ub, del);
+    cnt0 -= (L == da) + (L == db);
+    cnt1 -= (L + 64 == da) + (L + 64 == db);
   }
-  if (L < n && !((live >> L) & 1ull)) D.bp_status[gb] = 0;
+}
+
+// Resolve the component whose formed pairs are seg[0..n) (candidate ids,
+// any order).  Must be called by all 64 lanes of a wave with uniform
+// arguments; ws is mcw_lds(IT) ints of LDS private to the wave (8-byte
+// aligned).  Returns false if the component exceeds the capacity of 64*IT
+// pairs or its state is inconsistent, having written nothing.  The result
+// does not depend on IT (same draws, same decisions).  r indexes the
+// per-replica arrays; rk keys the random stream.
+// Layout: pair slot t (candidate-id order) lives in lane t % 64, chunk
+// t / 64; nucleotide slot u (ascending id) in lane u % 64, chunk u / 64;
+// the pair sequence of one iteration holds entry m in lane m.
+template <int IT = MCW_ITEMS, int ND = MCW_NODES>
+__device__ __forceinline__ bool mc_component_wave(const Params &P, const Ptrs &D, int r, int rk, int root,
+                                                  const int *seg, int n, double beta, uint64_t seed,
+                                                  int64_t step, int *ws) {
+  constexpr int NONE = 0x7fffffff;
+  constexpr int NP = 64 * IT;
+  static_assert(NP <= 256 && ND <= 8 && ND == 2 * IT, "pair slots are packed in 8 bits, nucleotide slots in 9");
+  const int L = lane_id();
+  const int N = P.N;
+  // uniform by contract; said so to the compiler, so that loop counters
+  // and lane indices stay scalar
+  n = __builtin_amdgcn_readfirstlane(n);
+  root = __builtin_amdgcn_readfirstlane(root);
+  if (n > NP) return false;
+  // ---- pairs in candidate-id order (= reference list order)
+  int *ssort = ws + 128;   // after the two 64-word arrays of wave_rank, inside its any-span arrays
+  int raw[IT], rank[IT];
+  bool ok[IT];
+#pragma unroll
+  for (int k = 0; k < IT; k++) {
+    const int t = L + 64 * k;
+    ok[k] = t < n;
+    raw[k] = ok[k] ? seg[t] : NONE;
+  }
+  if (wave_rank(raw, ok, ws, ws + 64, rank) < 0) wave_rank_any(raw, n, ws, ws + NP, rank);
+#pragma unroll
+  for (int k = 0; k < IT; k++)
+    if (ok[k]) ssort[rank[k]] = raw[k];
+  wave_lds_fence();
+  int gb[IT], ua[IT], ub[IT], e2[2 * IT], u2[2 * IT];
+  bool ok2[2 * IT];
+  double en[IT];
+  bool bad = false;
+#pragma unroll
+  for (int k = 0; k < IT; k++) {
+    gb[k] = ok[k] ? ssort[L + 64 * k] : NONE;
+    e2[2 * k] = e2[2 * k + 1] = -1;
+    ok2[2 * k] = ok2[2 * k + 1] = ok[k];
+    en[k] = 0.0;
+    if (ok[k]) {
+      const int *mp = D.bp_mp + (size_t)gb[k] * 8;
+      e2[2 * k] = mp[0] - 1;
+      e2[2 * k + 1] = mp[1] - 1;
+      en[k] = D.ene_bp[gb[k]];
+      bad = bad || e2[2 * k] < 0 || e2[2 * k] >= N || e2[2 * k + 1] < 0 || e2[2 * k + 1] >= N;
+    }
+  }
+  wave_lds_fence();
+  // a candidate naming a bead outside the system means corrupted MC state:
+  // report it (flags[7]) instead of indexing with it
+  if (__ballot(bad)) {
+    if (L == 0) D.flags[7] = 1;
+    return true;
+  }
+  // ---- distinct nucleotides in ascending id order, with their counts
+  int *snode = ws + 128;
+  int nn = wave_rank(e2, ok2, ws, ws + 64, u2);
+  if (nn < 0) {
+    // endpoint number L + 64 j of lane L in wave_rank_any's numbering:
+    // pairs of chunk k first by their lower, then their upper nucleotide
+    int v[2 * IT], w[2 * IT];
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+      v[k] = ok[k] ? e2[2 * k] : N;      // slots beyond n hold one value
+      v[IT + k] = ok[k] ? e2[2 * k + 1] : N;   // above every bead id
+    }
+    nn = wave_rank_any(v, 2 * NP, ws + 64, ws + 64 + 2 * NP, w) - (n < NP ? 1 : 0);
+#pragma unroll
+    for (int k = 0; k < IT; k++) {
+      u2[2 * k] = w[k];
+      u2[2 * k + 1] = w[IT + k];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 2 * IT; j++)
+    if (ok2[j]) snode[u2[j]] = e2[j];   // equal values write the same word
+  wave_lds_fence();
+  int cnt[ND];
+#pragma unroll
+  for (int q = 0; q < ND; q++) {
+    const int u = L + 64 * q;
+    cnt[q] = u < nn ? D.nt_cnt[(size_t)r * N + snode[u]] : 0;
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int k = 0; k < IT; k++) {
+    ua[k] = ok[k] ? u2[2 * k] : -1;
+    ub[k] = ok[k] ? u2[2 * k + 1] : -1;
+  }
+  unsigned long long live[IT];
+  // two nucleotide chunks do for nearly all components of up to 128 pairs
+  bool done = false;
+  if constexpr (IT == 1) done = mc_sweep64(rk, root, n, beta, seed, step, ua[0], ub[0], en[0], cnt[0], cnt[1], live[0]);
+  if (done) {
+  } else if (ND == 4 && nn <= 128) {
+    const int c[2] = {cnt[0], cnt[1]};
+    done = mc_sweep<IT, 2>(P.max_bp_per_nt, rk, root, n, beta, seed, step, ws, ua, ub, en, c, live);
+  } else {
+    done = mc_sweep<IT, ND>(P.max_bp_per_nt, rk, root, n, beta, seed, step, ws, ua, ub, en, cnt, live);
+  }
+  if (!done) return false;
+  // write back the pairs deleted here
+#pragma unroll
+  for (int k = 0; k < IT; k++)
+    if (ok[k] && !((live[k] >> L) & 1ull)) D.bp_status[gb[k]] = 0;
   return true;
 }
 
-// The wavefront forms by size: 64 pairs or fewer in the scalar form, up
-// to 64 * MCW_ITEMS in the general one (also the fallback of the scalar
-// form).  ws holds MCW_LDS ints.
+// The wavefront forms by size: one pair per lane up to 64 pairs, MCW_ITEMS
+// above.  ws holds MCW_LDS ints.
 __device__ __forceinline__ bool mc_component_wave_any(const Params &P, const Ptrs &D, int r, int rk, int root,
                                                       const int *seg, int n, double beta, uint64_t seed,
                                                       int64_t step, int *ws) {
-  if (n <= 64 && mc_component_wave64(P, D, r, rk, root, seg, n, beta, seed, step, ws)) return true;
+  if (n <= 64) return mc_component_wave<1, 2>(P, D, r, rk, root, seg, n, beta, seed, step, ws);
   return mc_component_wave(P, D, r, rk, root, seg, n, beta, seed, step, ws);
 }
 
 // ---------------------------------------------------------------------
-// The same algorithm for a component of at most MCL_PAIRS pairs, run by
-// one lane with everything in registers: arrays are read through unrolled
-// selects and the pair sequence is packed in 4-bit fields, so no per-lane
-// array is indexed dynamically.  The draws (seed, rk, step, root, 0, 1, ...)
-// and every decision are those of mc_component_wave, so the two give
-// identical results; many small components resolve in parallel, one per
-// lane.  Returns false if the component is too large or inconsistent.
-constexpr int MCL_PAIRS = 4;
+// A component of two pairs (the usual smallest one) by one lane: with one
+// pair allowed per nucleotide they share the only nucleotide in excess, so
+// its pick is certain and one deletion resolves it, by the draws the sweep
+// would use (1 and 2: swaps, 3: Metropolis).  Draws and decision are those
+// of mc_component_wave; many such components resolve in parallel, one per
+// lane.  Returns false for any other component or an inconsistent one.
+constexpr int MCL_PAIRS = 2;
 
-template <int M>
-__device__ __forceinline__ int sel_i(const int (&a)[M], int i) {
-  int v = a[0];
-#pragma unroll
-  for (int k = 1; k < M; k++) v = (i == k) ? a[k] : v;
-  return v;
-}
-template <int M>
-__device__ __forceinline__ double sel_d(const double (&a)[M], int i) {
-  double v = a[0];
-#pragma unroll
-  for (int k = 1; k < M; k++) v = (i == k) ? a[k] : v;
-  return v;
-}
-
-__device__ __forceinline__ bool mc_component_lane(const Ptrs &D, int N, int r, int rk, int root, const int *seg,
+__device__ __forceinline__ bool mc_component_lane(const Ptrs &D, int max_bp, int N, int rk, int root, const int *seg,
                                                   int n, double beta, uint64_t seed, int64_t step) {
-  constexpr int M = MCL_PAIRS, M2 = 2 * MCL_PAIRS;
-  constexpr int NONE = 0x7fffffff;
-  if (n > M) return false;
-  // candidate ids in ascending order (= list order)
-  int raw[M], g[M];
-#pragma unroll
-  for (int j = 0; j < M; j++) raw[j] = j < n ? seg[j] : NONE;
-#pragma unroll
-  for (int p = 0; p < M; p++) g[p] = NONE;
-#pragma unroll
-  for (int i = 0; i < M; i++) {
-    int rank = 0;
-#pragma unroll
-    for (int j = 0; j < M; j++) rank += raw[j] < raw[i] ? 1 : 0;
-#pragma unroll
-    for (int p = 0; p < M; p++)
-      if (i < n && rank == p) g[p] = raw[i];
-  }
-  int pa[M], pb[M];
-  double en[M];
-  bool bad = false;
-#pragma unroll
-  for (int j = 0; j < M; j++) {
-    pa[j] = pb[j] = -1;
-    en[j] = 0.0;
-    if (j < n) {
-      const int *mp = D.bp_mp + (size_t)g[j] * 8;
-      pa[j] = mp[0] - 1;
-      pb[j] = mp[1] - 1;
-      en[j] = D.ene_bp[g[j]];
-      bad = bad || pa[j] < 0 || pa[j] >= N || pb[j] < 0 || pb[j] >= N;
-    }
-  }
-  if (bad) {
+  if (n != 2 || max_bp != 1) return false;
+  const int g0 = seg[0], g1 = seg[1];
+  const int a = g0 < g1 ? g0 : g1, b = g0 < g1 ? g1 : g0;
+  const int *ma = D.bp_mp + (size_t)a * 8, *mb = D.bp_mp + (size_t)b * 8;
+  const int a0 = ma[0], a1 = ma[1], b0 = mb[0], b1 = mb[1];
+  if (a0 < 1 || a0 > N || a1 < 1 || a1 > N || b0 < 1 || b0 > N || b1 < 1 || b1 > N) {
     D.flags[7] = 1;
     return true;
   }
-  // distinct nucleotides in ascending id order, with their counts
-  int e[M2];
-#pragma unroll
-  for (int j = 0; j < M; j++) {
-    e[2 * j] = j < n ? pa[j] : NONE;
-    e[2 * j + 1] = j < n ? pb[j] : NONE;
-  }
-  bool first[M2];
-#pragma unroll
-  for (int k = 0; k < M2; k++) {
-    bool f = e[k] != NONE;
-#pragma unroll
-    for (int j = 0; j < M2; j++)
-      if (j < k && e[j] == e[k]) f = false;
-    first[k] = f;
-  }
-  int node[M2], cnt[M2];
-#pragma unroll
-  for (int q = 0; q < M2; q++) node[q] = NONE;
-#pragma unroll
-  for (int k = 0; k < M2; k++) {
-    int ur = 0;
-#pragma unroll
-    for (int j = 0; j < M2; j++) ur += (first[j] && e[j] < e[k]) ? 1 : 0;
-#pragma unroll
-    for (int q = 0; q < M2; q++)
-      if (first[k] && ur == q) node[q] = e[k];
-  }
-#pragma unroll
-  for (int q = 0; q < M2; q++) cnt[q] = node[q] != NONE ? D.nt_cnt[(size_t)r * N + node[q]] : 0;
-  // the Monte Carlo loop
-  uint32_t alive = (n >= 32) ? 0xffffffffu : ((1u << n) - 1u);
-  uint32_t draw = 0;
-  for (int iter = 0; iter < 4 * M + 4; iter++) {
-    int nact = 0;
-#pragma unroll
-    for (int q = 0; q < M2; q++) nact += cnt[q] > 0 ? 1 : 0;
-    if (nact == 0) break;
-    const int pick = (int)ceil(philox_u(seed, rk, step, root, draw++) * nact);   // 1..nact
-    int ntd = -1, acc = 0;
-#pragma unroll
-    for (int q = 0; q < M2; q++)
-      if (cnt[q] > 0) {
-        acc++;
-        if (acc == pick) ntd = node[q];
-      }
-    // formed pairs of ntd in list order, packed 4 bits each
-    uint32_t seqp = 0;
-    int ns = 0;
-#pragma unroll
-    for (int j = 0; j < M; j++)
-      if (((alive >> j) & 1u) && (pa[j] == ntd || pb[j] == ntd)) {
-        seqp |= (uint32_t)j << (4 * ns);
-        ns++;
-      }
-    if (ns == 0) return false;
-    // reference shuffle: for i = 1..n swap(i, ceil(rnd*n))
-    for (int i = 0; i < ns; i++) {
-      const int sw = (int)ceil(philox_u(seed, rk, step, root, draw++) * ns) - 1;
-      const uint32_t ti = (seqp >> (4 * i)) & 15u, ts = (seqp >> (4 * sw)) & 15u;
-      seqp = (seqp & ~(15u << (4 * i))) | (ts << (4 * i));
-      seqp = (seqp & ~(15u << (4 * sw))) | (ti << (4 * sw));
-    }
-    // Metropolis sweep on the energies
-    int del = (int)(seqp & 15u);
-    double edel = sel_d(en, del);
-    for (int i = 1; i < ns; i++) {
-      const int j = (int)((seqp >> (4 * i)) & 15u);
-      const double ej = sel_d(en, j);
-      if (log(philox_u(seed, rk, step, root, draw++)) < (ej - edel) * beta) {
-        del = j;
-        edel = ej;
-      }
-    }
-    alive &= ~(1u << del);
-    const int da = sel_i(pa, del), db = sel_i(pb, del);
-#pragma unroll
-    for (int q = 0; q < M2; q++)
-      if (node[q] == da || node[q] == db) cnt[q] -= 1;
-  }
-#pragma unroll
-  for (int j = 0; j < M; j++)
-    if (j < n && !((alive >> j) & 1u)) D.bp_status[g[j]] = 0;
+  if ((a0 == b0) + (a0 == b1) + (a1 == b0) + (a1 == b1) != 1) return false;
+  const bool h1 = philox_u(seed, rk, step, root, 1u) > 0.5, h2 = philox_u(seed, rk, step, root, 2u) > 0.5;
+  const double w = log(philox_u(seed, rk, step, root, 3u));
+  const double ea = D.ene_bp[a], eb = D.ene_bp[b];
+  // both swap draws on the same side of one half: the pairs are reversed
+  const bool flip = h1 == h2;
+  const double e0 = flip ? eb : ea, e1 = flip ? ea : eb;
+  const bool second = w < (e1 - e0) * beta;
+  D.bp_status[second == flip ? a : b] = 0;
   return true;
 }
 

@@ -89,7 +89,7 @@ template <typename T, int LPB, int B>
 __global__ void __launch_bounds__(B) k_persistent(Params P, Ptrs D, PersArgs A) {
   __shared__ double s1[B / LPB], s2[B / LPB];
   __shared__ int s_exit, s_big;
-  __shared__ int s_mcws[(B / 64) * MCW_LDS];   // wave MC scratch, one slice per wave
+  __shared__ __align__(16) int s_mcws[(B / 64) * MCW_LDS];   // wave MC scratch, one slice per wave
   static_assert((B / 64) * MCW_LDS >= MCB_LDS, "large-component MC needs the block's whole scratch");
   if (threadIdx.x == 0) s_big = 0;
   const int N = P.N;
@@ -150,7 +150,7 @@ __global__ void __launch_bounds__(B) k_persistent(Params P, Ptrs D, PersArgs A) 
           const int n = A.seg_n[root];
           if (n > MCL_PAIRS) continue;
           int *sg = A.seg + (size_t)root * SEGCAP;
-          if (!mc_component_lane(D, N, 0, 0, root, sg, n, beta, A.seed, step))
+          if (!mc_component_lane(D, P.max_bp_per_nt, N, 0, root, sg, n, beta, A.seed, step))
             mc_component_serial(mc_arrays(D), P.N, 0, 0, root, sg, n, beta, A.seed, step);
         }
         const int wave = gtid / 64, nwaves = gthreads / 64;
@@ -592,7 +592,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
   __shared__ int s_exc[EXC_LDS];   // component roots with excess (MC steps)
   __shared__ int s_nexc, s_big, s_nw, s_next, s_huge;
   __shared__ int s_wl[MCW_LIST];   // wavefront-MC components of this step: size << 21 | root
-  __shared__ int s_mcws[(B / 64) * MCW_LDS];   // wave MC scratch, one slice per wave
+  __shared__ __align__(16) int s_mcws[(B / 64) * MCW_LDS];   // wave MC scratch, one slice per wave
   static_assert((B / 64) * MCW_LDS >= MCB_LDS, "large-component MC needs the block's whole scratch");
   const int N = P.N;
   const int tid = threadIdx.x;
@@ -879,7 +879,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
               const int n = segn[root];
               if (n <= MCL_PAIRS) {
                 int *sg = J.seg + gr * SEGCAP;
-                if (!mc_component_lane(DM, N, rm, J.rk, root, sg, n, beta, J.seed, step))
+                if (!mc_component_lane(DM, P.max_bp_per_nt, N, J.rk, root, sg, n, beta, J.seed, step))
                   mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, root, sg, n, beta, J.seed, step);
               }
             }
