@@ -48,12 +48,6 @@ def bytes_per_bead_step(p_wca, p_ele, p_bp):
     return 144.0 + 36.0 + 8.0 * p_wca + 8.0 * p_ele + 44.0 * p_bp
 
 
-def force_kernel_bytes(p_wca, p_ele):
-    """Algorithmic bytes of the per-phase pair/integrator kernel per bead:
-    state read + write and the WCA / DH pair indices."""
-    return 144.0 + 8.0 * p_wca + 8.0 * p_ele
-
-
 def load_traffic(workload, mode):
     """Measured HBM bytes per bead-step of the dominant kernel (FETCH_SIZE +
     WRITE_SIZE, calibrated; profiles/traffic.json names the summary each
@@ -428,15 +422,8 @@ def main():
     assert np.all(np.isfinite(x)), "non-finite coordinates"
     mode_used0 = {1: "phases", 2: "persistent", 3: "batched"}.get(info2["mode"], "")
     if mode_used0 == "phases" and dom_n == 0:
-        # replayed graphs carry no per-kernel events: time the pair /
-        # integrator kernel on host-launched steps of the same state
-        pe = Engine(sysd, precision=prec, parity=False, mode="phases", seed=2024, no_graph=True,
-                    exchange_every=int(sysd.get("exchange_every", 0)))
-        pe.set_state(x, v, a)
-        pe.neighbor_list(0)
-        pe.step(min(steps, 50))
-        dom_ms, dom_n = pe.last_ms(3), int(pe.last_ms(4))
-        pe.close()
+        # a step's four launches share its work: the whole step is timed
+        dom_ms, dom_n = 1e3 * wall / steps, steps
     eng.close()
     print(f"[bench] timed {steps} steps {wall:.3f}s", flush=True)
     bead_steps = nmp * nrep * steps
@@ -446,13 +433,12 @@ def main():
     p_bp = info2["nbp"] / nmp
     B = bytes_per_bead_step(p_wca, p_ele, p_bp)
     mode_used = {1: "phases", 2: "persistent", 3: "batched"}.get(info2["mode"], str(info2["mode"]))
-    # one k_force_lanes launch per step in the per-phase form; the batched
-    # and persistent kernels run whole segments per launch
+    # the four launches of a step in the per-phase form; the batched and
+    # persistent kernels run whole segments per launch
     steps_per_launch = 1 if mode_used == "phases" else steps / max(dom_n, 1)
-    if mode_used == "phases":
-        kname, kbytes = "k_force_lanes", force_kernel_bytes(p_wca, p_ele)
-    else:
-        kname, kbytes = {"persistent": "k_persistent", "batched": "k_batched"}[mode_used], B
+    kname = {"phases": "k_step_bp + k_step_seg + k_step_mc + k_step_move", "persistent": "k_persistent",
+             "batched": "k_batched"}[mode_used]
+    kbytes = B
     ns_day = (steps / wall) * 0.05 * TAU_FS * 86400 * 1e-6
     out = {
         "metric": METRIC,

@@ -101,8 +101,8 @@ typedef struct sis_options {
                                 (0 = as many as fit on the device) */
     int32_t flags;           /* bit0 SIS_OPT_HOST_EXCHANGE: batched runs exchange on the
                                 host between segments (no device exchange, no graph);
-                                bit1 SIS_OPT_NO_GRAPH: the per-phase form launches every
-                                step from the host instead of replaying a captured graph */
+                                bit1 SIS_OPT_NO_GRAPH: the per-phase form issues every
+                                launch from the host instead of replaying a captured graph */
 } sis_options;
 #define SIS_OPT_HOST_EXCHANGE 1
 #define SIS_OPT_NO_GRAPH 2
@@ -483,8 +483,9 @@ int sis_gpu_get_info(sis_gpu_ctx *ctx, int64_t *out, int32_t n);
 /* Device time (ms, HIP events on the context stream) of the last call of
  * a kind: 0 = step, 1 = rebuild, 2 = force; 3 = mean duration of one
  * launch of the step's dominant kernel during the last sis_gpu_step call
- * (the fused force + integrator kernel, or the persistent / batched step
- * kernel), 4 = number of such launches. */
+ * (the persistent / batched step kernel; the force + integrator kernel of
+ * steps launched one by one, as with external terms), 4 = number of such
+ * launches (0: steps in device-driven batches). */
 double sis_gpu_last_kernel_ms(sis_gpu_ctx *ctx, int32_t which);
 
 /* ---- Job pool: the serving form -------------------------------------

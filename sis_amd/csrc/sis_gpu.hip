@@ -14,6 +14,7 @@
 #include "../../include/sis_gpu.h"
 #include "sis_device.h"
 #include "sis_kernels.h"
+#include "sis_step.h"
 #include "sis_persistent.h"
 #include "sis_exchange.h"
 #include "sis_external.h"
@@ -89,7 +90,8 @@ struct PhaseGraphKey {
   Params P;
   Ptrs D;
   const void *pos;
-  int nblk, block;
+  uint64_t seed;
+  int sep_huge;
 };
 
 struct sis_gpu_ctx {
@@ -221,8 +223,14 @@ struct sis_gpu_ctx {
   int block = 256;
   int dev = 0;   // the HIP device current when the context was created
   // replayed per-phase steps (phases_graph_steps)
-  DevBuf<int64_t> g_step_d;
+  DevBuf<StepWords> g_step_d;
+  void *step_pin = nullptr;     // pinned copies of it, two batches' worth
+  hipEvent_t step_ev[2] = {nullptr, nullptr};
   DevBuf<int> g_int_d;
+  DevBuf<double4> step_fpair_d, step_noise_d;
+  DevBuf<double> step_top2_d;
+  bool circular = false;        // some chain is circular
+  bool step_sep_huge = false;   // a component above the bucket capacity was met
   // device exchange of the batched form (sis_exchange.h)
   DevBuf<int> dx_rep2lab_d, dx_lab2rep_d, dx_pair_tb_d, dx_idx_d, dx_has_d, dx_vsdiv_d, dx_nexch_d, dx_acc_d;
   DevBuf<double> dx_labT_d, dx_labCoef_d, dx_labLam_d, dx_labCr_d, dx_oppT_d, dx_oppCoef_d, dx_oppLam_d,
@@ -319,7 +327,13 @@ struct sis_gpu_ctx {
     for (auto &e : pg_exec)
       if (e) (void)hipGraphExecDestroy(e);
     g_step_d.free_();
+    if (step_pin) (void)hipHostFree(step_pin);
+    for (auto e : step_ev)
+      if (e) (void)hipEventDestroy(e);
     g_int_d.free_();
+    step_fpair_d.free_();
+    step_noise_d.free_();
+    step_top2_d.free_();
     for (auto e : tev) (void)hipEventDestroy(e);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -690,17 +704,13 @@ void analysis_rebuild(sis_gpu_ctx *c) {
 }
 
 // Base-pair evaluation + limit MC (force_bp_limit_triplet / force_bp_triplet).
-// mc: limit-MC flags per replica, uploaded here; null when the flags are
-// already on the device (replayed graph steps, whose step number is
-// step_dev's)
-void bp_phase(sis_gpu_ctx *c, const std::vector<int> *mc, const double *ecT_dev, const int *mask_dev,
-              const int64_t *step_dev = nullptr, bool resets_done = false) {
+// mc: limit-MC flags per replica, uploaded here.
+void bp_phase(sis_gpu_ctx *c, const std::vector<int> &mc, const double *ecT_dev, const int *mask_dev) {
   const int N = c->N, R = c->R, B = 256;
-  if (mc) set_mc(c, *mc);
+  set_mc(c, mc);
   Ptrs D = c->ptrs();
-  bool any_mc = !mc;
-  if (mc)
-    for (int r = 0; r < R; r++) any_mc |= (*mc)[r] != 0;
+  bool any_mc = false;
+  for (int r = 0; r < R; r++) any_mc |= mc[r] != 0;
   any_mc = any_mc && c->P.nstep_bp_mc > 0;
   // performance-form MC: counts, union-find and buckets reset in one pass,
   // the union done by the evaluation itself, the components with excess
@@ -710,53 +720,46 @@ void bp_phase(sis_gpu_ctx *c, const std::vector<int> *mc, const double *ecT_dev,
   if (perf_mc) {
     if (c->seg_d.n < RN * SEGCAP) c->seg_d.alloc(RN * SEGCAP);
     if (c->exc_list_d.n < RN + 1) c->exc_list_d.alloc(RN + 1);
-    if (!resets_done)
-      hipLaunchKernelGGL(k_mc_reset, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->exc_cnt_d.p,
+    hipLaunchKernelGGL(k_mc_reset, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->exc_cnt_d.p,
                          c->exc_fill_d.p, c->exc_list_d.p, mask_dev);
-  } else if (!resets_done) {
+  } else {
     hipLaunchKernelGGL(k_reset_cnt, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, mask_dev);
   }
-  // captured steps launch over the candidate capacity and read the count
-  // on the device, so that their graph stays valid across rebuilds
-  const bool dev_count = step_dev != nullptr;
-  const int nbp_arg = dev_count ? -1 : (int)c->nbp_total;
-  const int64_t nbp_grid = dev_count ? c->D.maxbp : c->nbp_total;
-  if (nbp_grid > 0) {
+  const int nbp = (int)c->nbp_total;
+  if (nbp > 0) {
     if (c->precision == 1)
-      hipLaunchKernelGGL(k_bp_eval<float>, dim3((nbp_grid + B - 1) / B), dim3(B), 0, c->stream, c->P, D,
-                         nbp_arg, c->mc_d.p, ecT_dev, mask_dev, perf_mc ? 1 : 0);
+      hipLaunchKernelGGL(k_bp_eval<float>, dim3((nbp + B - 1) / B), dim3(B), 0, c->stream, c->P, D, nbp, c->mc_d.p,
+                         ecT_dev, mask_dev, perf_mc ? 1 : 0);
     else
-      hipLaunchKernelGGL(k_bp_eval<double>, dim3((nbp_grid + B - 1) / B), dim3(B), 0, c->stream, c->P, D,
-                         nbp_arg, c->mc_d.p, ecT_dev, mask_dev, perf_mc ? 1 : 0);
+      hipLaunchKernelGGL(k_bp_eval<double>, dim3((nbp + B - 1) / B), dim3(B), 0, c->stream, c->P, D, nbp, c->mc_d.p,
+                         ecT_dev, mask_dev, perf_mc ? 1 : 0);
   }
   if (!any_mc) return;
   if (c->parity) {
     hipLaunchKernelGGL(k_mc_serial, dim3(R), dim3(64), 0, c->stream, c->P, D, c->mc_d.p, ecT_dev,
                        c->ntlist_d.p, c->bpseq_d.p, mask_dev);
   } else {
-    if (nbp_grid == 0) return;
-    hipLaunchKernelGGL(k_seg_fill, dim3((nbp_grid + B - 1) / B), dim3(B), 0, c->stream, c->P, D,
-                       nbp_arg, c->exc_cnt_d.p, c->seg_d.p, c->exc_fill_d.p, c->mc_d.p, mask_dev,
-                       c->exc_list_d.p);
+    if (nbp == 0) return;
+    hipLaunchKernelGGL(k_seg_fill, dim3((nbp + B - 1) / B), dim3(B), 0, c->stream, c->P, D, nbp, c->exc_cnt_d.p,
+                       c->seg_d.p, c->exc_fill_d.p, c->mc_d.p, mask_dev, c->exc_list_d.p);
     // one block per listed component as far as the device holds them at
-    // once (C4 lists about 3,400 a step): a block that takes two in turn
-    // can start the longest deletion chain late
+    // once: a block that takes two in turn can start the longest deletion
+    // chain late
     const int nlist = (int)std::min<int64_t>((int64_t)std::max<int64_t>(RN, 1), 8192);
     hipLaunchKernelGGL(k_mc_list, dim3(nlist), dim3(64), 0, c->stream, c->P, D, c->exc_cnt_d.p, c->seg_d.p,
-                       c->exc_list_d.p, ecT_dev, c->seed, c->istep, c->huge_d.p, step_dev);
+                       c->exc_list_d.p, ecT_dev, c->seed, c->istep, c->huge_d.p);
     hipLaunchKernelGGL(k_mc_huge, dim3(R), dim3(64), 0, c->stream, c->P, D, c->exc_cnt_d.p, c->seg_d.p,
-                       c->exc_fill_d.p, c->huge_d.p, ecT_dev, c->seed, c->istep, step_dev);
+                       c->exc_fill_d.p, c->huge_d.p, ecT_dev, c->seed, c->istep);
   }
 }
 
 // launch shape of the pair/integrator kernel: FORCE_B threads per
 // workgroup, FORCE_LPB lanes per bead; force_blocks = workgroups per replica
-constexpr int FORCE_B = 256, FORCE_LPB = 8;
+constexpr int FORCE_B = STEP_B, FORCE_LPB = PAIR_LPB;
 inline int force_blocks(int N) { return (N + FORCE_B / FORCE_LPB - 1) / (FORCE_B / FORCE_LPB); }
 
 // mark: time the pair/integrator kernel with the context's event pairs
-void force_kernel(sis_gpu_ctx *c, int integrate, const int *mask_dev, const int64_t *step_dev = nullptr,
-                  bool mark = false) {
+void force_kernel(sis_gpu_ctx *c, int integrate, const int *mask_dev, bool mark = false) {
   const int N = c->N, R = c->R;
   constexpr int B = FORCE_B, LPB = FORCE_LPB;
   dim3 g(force_blocks(N), R);
@@ -773,10 +776,10 @@ void force_kernel(sis_gpu_ctx *c, int integrate, const int *mask_dev, const int6
   if (mark) c->tmark();
   if (c->precision == 1)
     hipLaunchKernelGGL((k_force_lanes<float, LPB, B>), g, dim3(B), 0, c->stream, c->P, c->ptrs(), integrate,
-                       c->parity, c->seed, c->istep, mask_dev, step_dev, inl);
+                       c->parity, c->seed, c->istep, mask_dev, inl);
   else
     hipLaunchKernelGGL((k_force_lanes<double, LPB, B>), g, dim3(B), 0, c->stream, c->P, c->ptrs(), integrate,
-                       c->parity, c->seed, c->istep, mask_dev, step_dev, inl);
+                       c->parity, c->seed, c->istep, mask_dev, inl);
   if (mark) c->tmark();
 }
 
@@ -820,7 +823,7 @@ void energy_phase(sis_gpu_ctx *c, const std::vector<int> &mask, const std::vecto
   if (!(flags & 2)) {
     std::vector<int> mc(R, 0);
     for (int r = 0; r < R; r++) mc[r] = (flags & 1) && mask[r];
-    bp_phase(c, &mc, c->ecT_d.p, c->mask_d.p);
+    bp_phase(c, mc, c->ecT_d.p, c->mask_d.p);
   }
   dim3 g = grid_beads(N, R, B);
   if ((int64_t)c->ene_part_d.n < (int64_t)R * g.x * 8) c->ene_part_d.alloc((size_t)R * g.x * 8);
@@ -1074,7 +1077,7 @@ void step_phases(sis_gpu_ctx *c) {
   }
   std::vector<int> all(R, 1);
   set_mask(c, all);
-  bp_phase(c, &mc, nullptr, nullptr);
+  bp_phase(c, mc, nullptr, nullptr);
   if (c->P.nstep_bp_mc > 1) {
     // bp_status_MC = bp_status of the replicas that did MC
     // (src/job_md.F90:399-401); candidates are grouped by replica
@@ -1091,161 +1094,231 @@ void step_phases(sis_gpu_ctx *c) {
   }
   if (c->parity)
     hipLaunchKernelGGL(k_noise_parity, dim3(1), dim3(1), 0, c->stream, c->P, c->ptrs(), 3 * N, 0, nullptr);
-  force_kernel(c, 1, nullptr, nullptr, true);
+  force_kernel(c, 1, nullptr, true);
   std::swap(c->pos_d, c->pos2_d);   // updated positions become current
-  hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(), c->nblk_force, GStep{});
+  hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(),
+                     c->blk_top2_d.p, c->nblk_force);
 }
 
-// Whether the per-phase form can replay its steps from a captured graph:
+// Whether the per-phase form can run its steps in device-driven batches:
 // the performance form without external terms or a fixed rebuild cadence.
-bool graph_steps_ok(sis_gpu_ctx *c) {
-  return !c->parity && !c->ext_on && c->opt.rebuild_every == 0 && !(c->opt.flags & SIS_OPT_NO_GRAPH);
-}
+bool graph_steps_ok(sis_gpu_ctx *c) { return !c->parity && !c->ext_on && c->opt.rebuild_every == 0; }
 
-// The per-phase form's steps (step_phases) replayed from a HIP graph of
-// GRAPH_STEPS steps, with no host round trip per step: the step number and
-// the limit-MC flags come from k_gstep_begin, and k_skin halts the steps
-// that follow when a replica needs a rebuild (or the requested count is
-// reached).  The host then rebuilds, captures again (rebuilds resize the
-// launches) and replays on.  Same kernels, same arithmetic and random
-// streams as step_phases.
-constexpr int GRAPH_STEPS = 16;   // even: the positions end in the buffer they started in
-
-// Runs batches of GRAPH_STEPS steps (launch() issues one batch: a captured
-// graph's replay or the same launches issued directly) until a replica
-// halts them (a rebuild is due) or the requested step is reached.
+// The per-phase form's steps in batches of GRAPH_STEPS with no host round
+// trip per step (sis_step.h): every launch reads the step from the device,
+// and the first launch of a step halts it and those after it when a replica
+// needs a rebuild or the requested count is reached.  A batch is replayed
+// from a HIP graph or issued directly.  The host then rebuilds and goes on.
+// Same terms and random streams as step_phases.
+//
+// Runs batches until the steps halt or `stop` is reached; c->istep and the
+// current position buffer follow.  launch(n) issues a batch of n steps from
+// the current buffer (GRAPH_STEPS unless `exact`, where the last batch is cut
+// to what is left).  The next batch is issued before the last one's halt
+// word is read, so the device does not wait for the host in between: what
+// follows a halt does nothing.  Returns true when the last step waits for a
+// component above the bucket capacity (k_step_huge).
 template <typename F>
-void run_phase_batches(sis_gpu_ctx *c, F &&launch) {
-  int halt = 0;
-  int64_t now = c->istep;
-  while (!halt) {
-    launch();
-    HIPCHK(hipMemcpyAsync(&halt, c->g_int_d.p, sizeof halt, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipMemcpyAsync(&now, c->g_step_d.p, sizeof now, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (!halt && now - c->istep != (int64_t)GRAPH_STEPS) throw ApiError{SIS_ERR_STATE, "graph steps did not advance"};
-    if (!halt) c->istep = now;
+bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
+  if (!c->step_pin) {
+    HIPCHK(hipHostMalloc(&c->step_pin, 2 * sizeof(StepWords), hipHostMallocDefault));
+    for (auto &e : c->step_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
-  // an odd number of steps in the last replay leaves the positions in the
-  // other buffer
-  if ((now - c->istep) % 2) std::swap(c->pos_d, c->pos2_d);
-  c->istep = now;
+  StepWords *pin = static_cast<StepWords *>(c->step_pin);
+  const int64_t base = c->istep;
+  double4 *const pos0 = c->pos_d.p;
+  int64_t issued = 0, nb = 0, nread = 0;
+  bool halt = false, huge = false;
+  int64_t done = 0;
+  while (!halt && !huge) {
+    // one batch until it has run through: where rebuilds are frequent the
+    // second would be issued for nothing
+    while (nb - nread < (nread > 0 ? 2 : 1) && base + issued < stop) {
+      const int n = exact ? (int)std::min<int64_t>(GRAPH_STEPS, stop - base - issued) : GRAPH_STEPS;
+      launch(n);
+      issued += n;
+      HIPCHK(hipMemcpyAsync(pin + nb % 2, c->g_step_d.p, sizeof(StepWords), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipEventRecord(c->step_ev[nb % 2], c->stream));
+      nb++;
+    }
+    if (nread == nb) break;
+    HIPCHK(hipEventSynchronize(c->step_ev[nread % 2]));
+    const StepWords &w = pin[nread % 2];
+    halt = w.halt != 0;
+    huge = w.huge_any != 0 && !c->step_sep_huge;   // (with its launch in every step it is done within it)
+    done = w.done;
+    nread++;
+  }
+  HIPCHK(hipStreamSynchronize(c->stream));
+  if (huge && !halt) {   // noted by a later step's first launch, if there was one
+    const StepWords &w = pin[(nb - 1) % 2];
+    halt = w.halt != 0;
+    done = w.done;
+  }
+  c->istep = halt ? done : huge ? base + issued - 1 : base + issued;
+  // the positions are in the buffer that so many steps leave them in
+  if (c->pos_d.p != pos0) std::swap(c->pos_d, c->pos2_d);
+  if ((c->istep - base) % 2) std::swap(c->pos_d, c->pos2_d);
+  return huge;
 }
+
+inline int pad8(int64_t n) { return (int)((n + 7) / 8 * 8); }
 
 void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
-  const int R = c->R;
-  if (c->g_step_d.n < 3) c->g_step_d.alloc(3);
-  if (c->g_int_d.n < (size_t)(1 + 3 * R)) {
-    c->g_int_d.alloc(1 + 3 * R);
-    HIPCHK(hipMemset(c->g_int_d.p, 0, (1 + 3 * (size_t)R) * sizeof(int)));
-  }
-  GStep G{};
-  G.istep = c->g_step_d.p;
-  G.istep_cur = c->g_step_d.p + 1;
-  G.stop = c->g_step_d.p + 2;
-  G.halt = c->g_int_d.p;
-  G.active = c->g_int_d.p + 1;
-  G.force_mc = c->g_int_d.p + 1 + R;
-  G.mc = c->mc_d.p;
-  std::vector<int> fmc(R, 0), flag(R, 0);
+  const int N = c->N, R = c->R, B = STEP_B;
+  const size_t RN = (size_t)R * N;
+  const bool mc_on = c->P.nstep_bp_mc > 0;
+  if (c->g_step_d.n < 1) c->g_step_d.alloc(1);
+  if (c->g_int_d.n < (size_t)R) c->g_int_d.alloc(R);
+  if (c->step_fpair_d.n < RN) { c->step_fpair_d.alloc(RN); c->step_noise_d.alloc(RN); }
+  const bool bd = c->P.bd != 0;   // forces and update in one launch (k_step_force)
+  const int nblk = bd ? force_blocks(N) : (N + B - 1) / B;
+  if (c->step_top2_d.n < (size_t)R * nblk * 2) c->step_top2_d.alloc((size_t)R * nblk * 2);
+  if (mc_on && c->seg_d.n < RN * SEGCAP) c->seg_d.alloc(RN * SEGCAP);
+  if (mc_on && c->exc_list_d.n < RN + 1) c->exc_list_d.alloc(RN + 1);
+  StepArgs A{};
+  A.w = c->g_step_d.p;
+  A.force_mc = c->g_int_d.p;
+  A.huge = c->huge_d.p;
+  A.seg_n = c->exc_cnt_d.p;
+  A.has_exc = c->exc_fill_d.p;
+  A.exc_list = c->exc_list_d.p;
+  A.fpair = c->step_fpair_d.p;
+  A.noise = c->step_noise_d.p;
+  A.top2 = c->step_top2_d.p;
+  A.seed = c->seed;
+  A.nblk = nblk;
+  A.nbead = bd ? 0 : pad8((int64_t)R * ((N + BEAD_TILE - 1) / BEAD_TILE));
+  A.npair = (N + PAIR_TILE - 1) / PAIR_TILE;
+  A.circ = c->circular ? 1 : 0;
+  // pair tiles of the three launches that carry them
+  const int ntile = bd ? 0 : R * A.npair;
+  const int t1 = mc_on ? (int)(ntile * STEP_SHARE_BP) : ntile, t2 = mc_on ? (int)(ntile * (STEP_SHARE_BP + STEP_SHARE_SEG)) : ntile;
+  std::vector<int> flag(R, 0);
   const int64_t stop = c->istep + nsteps;
+  auto kernels = [&](auto zero, int part, int j) {
+    using T = decltype(zero);
+    A.j = j;
+    const Ptrs D = c->ptrs();
+    if (part == 0) {
+      A.p0 = 0; A.p1 = t1;
+      hipLaunchKernelGGL(k_step_bp<T>, dim3(A.ncand + A.nbead + t1), dim3(B), 0, c->stream, c->P, D, A);
+      if (mc_on) {
+        A.p0 = t1; A.p1 = t2;
+        A.nlist = A.ncand;
+        hipLaunchKernelGGL(k_step_seg<T>, dim3(A.nlist + t2 - t1), dim3(B), 0, c->stream, c->P, D, A);
+        A.p0 = t2; A.p1 = ntile;
+        // a wavefront for each component there may be, as far as the
+        // device holds them at once
+        A.nlist = pad8(std::min<int64_t>(2048, (int64_t)(RN + 63) / 64));
+        hipLaunchKernelGGL(k_step_mc<T>, dim3(A.nlist + ntile - t2), dim3(B), 0, c->stream, c->P, D, A);
+      }
+    }
+    if (A.sep_huge && mc_on) hipLaunchKernelGGL(k_step_huge, dim3(R), dim3(64), 0, c->stream, c->P, D, A);
+    if (c->P.nstep_bp_mc > 1)
+      hipLaunchKernelGGL(k_step_keep, dim3(A.ncand), dim3(B), 0, c->stream, c->P, D, A);
+    if (bd) {
+      hipLaunchKernelGGL(k_step_force<T>, dim3(nblk, R), dim3(B), 0, c->stream, c->P, D, A);
+      if (j == A.nj - 1) hipLaunchKernelGGL(k_step_commit, dim3(1), dim3(1), 0, c->stream, A);
+    } else {
+      hipLaunchKernelGGL(k_step_move, dim3(nblk, R), dim3(B), 0, c->stream, c->P, D, A);
+    }
+    std::swap(c->pos_d, c->pos2_d);
+  };
+  auto launch_step = [&](int part, int j) {
+    if (c->precision == 1) kernels(0.0f, part, j);
+    else kernels(0.0, part, j);
+  };
+  auto launch_batch = [&](int n) {
+    A.nj = n;
+    for (int j = 0; j < n; j++) launch_step(0, j);
+  };
   while (c->istep < stop) {
     // a rebuild due from the last skin test, or lists not built yet
     // (src/job_md.F90:376-395); the rebuilt replicas do the limit MC first
     if (!c->lists_valid) {
       std::fill(flag.begin(), flag.end(), 1);
     } else {
-      HIPCHK(hipMemcpy(flag.data(), c->rebuild_flag_d.p, R * sizeof(int), hipMemcpyDeviceToHost));
+      HIPCHK(hipMemcpyAsync(flag.data(), c->rebuild_flag_d.p, R * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipStreamSynchronize(c->stream));
     }
     bool any = false;
     for (int r = 0; r < R; r++) any = any || flag[r];
+    std::vector<int> fmc(R, 0);
     if (any) {
       rebuild(c, flag);
       c->rebuilds++;
-      for (int r = 0; r < R; r++) fmc[r] = (c->rebuilt[r] && c->P.nstep_bp_mc > 0) ? 1 : fmc[r];
+      for (int r = 0; r < R; r++) fmc[r] = c->rebuilt[r] && mc_on ? 1 : 0;
     }
-    const int64_t st[3] = {c->istep, c->istep, stop};
-    const int zero = 0;
-    HIPCHK(hipMemcpyAsync(c->g_step_d.p, st, sizeof st, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->g_int_d.p, &zero, sizeof zero, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(G.force_mc, fmc.data(), R * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    const StepWords w0{c->istep, stop, 0, any ? c->istep + 1 : -1, 0, 0};
+    HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w0, sizeof w0, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(hipMemcpyAsync(c->g_int_d.p, fmc.data(), R * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    // no skin test before the first step: the rebuild above was its answer
+    HIPCHK(hipMemsetAsync(c->step_top2_d.p, 0, (size_t)R * nblk * 2 * sizeof(double), c->stream));
+    hipLaunchKernelGGL(k_mc_reset, grid_beads(N, R, 256), dim3(256), 0, c->stream, c->P, c->ptrs(), c->exc_cnt_d.p,
+                       c->exc_fill_d.p, c->exc_list_d.p, nullptr);
     HIPCHK(hipStreamSynchronize(c->stream));
-    std::fill(fmc.begin(), fmc.end(), 0);
-    // buffers the captured kernels use are allocated before the capture
-    const int nblk = force_blocks(c->N);
-    c->nblk_force = nblk;
-    if ((int64_t)c->blk_top2_d.n < (int64_t)R * nblk * 2) c->blk_top2_d.alloc((size_t)R * nblk * 2);
-    if (c->P.nstep_bp_mc > 0 && c->seg_d.n < (size_t)R * c->N * SEGCAP) c->seg_d.alloc((size_t)R * c->N * SEGCAP);
-    if (c->P.nstep_bp_mc > 0 && c->exc_list_d.n < (size_t)R * c->N + 1) c->exc_list_d.alloc((size_t)R * c->N + 1);
-    // GRAPH_STEPS steps from the current position buffer, captured once
-    // and replayed until something the launches take by value changes
-    // (parameters, buffer addresses and capacities, the current buffer)
+    A.seg = c->seg_d.p;
+    A.ncand = pad8(std::max<int64_t>(1, (c->D.maxbp + B - 1) / B));   // the capacity; the count is read on the device
+    A.sep_huge = c->step_sep_huge ? 1 : 0;
+    // captured once and replayed until something the launches take by
+    // value changes (parameters, buffer addresses and capacities, the
+    // current buffer)
     PhaseGraphKey key;
     std::memset(&key, 0, sizeof key);
     key.P = c->P;
     key.D = c->ptrs();
     key.pos = c->pos_d.p;
-    key.nblk = c->nblk_force;
-    key.block = c->block;
-    const bool perf_mc = c->P.nstep_bp_mc > 0;
-    // one batch of steps: begin + resets, base pairs (+ MC), pair forces +
-    // update, skin test; the host's buffer swaps return to the start
-    auto launch_steps = [&]() {
-      for (int j = 0; j < GRAPH_STEPS; j++) {
-        hipLaunchKernelGGL(k_gstep_reset, grid_beads(c->N, R, 256), dim3(256), 0, c->stream, c->P, c->ptrs(), G,
-                           c->exc_cnt_d.p, c->exc_fill_d.p, perf_mc ? c->exc_list_d.p : nullptr, perf_mc ? 1 : 0);
-        bp_phase(c, nullptr, nullptr, G.active, G.istep_cur, true);
-        if (c->P.nstep_bp_mc > 1 && c->D.maxbp > 0)
-          hipLaunchKernelGGL(k_mc_keep, dim3((c->D.maxbp + 255) / 256), dim3(256), 0, c->stream, c->P, c->ptrs(),
-                             -1, G.mc, G.active);
-        force_kernel(c, 1, G.active, G.istep_cur);
-        std::swap(c->pos_d, c->pos2_d);
-        // a large system's thousands of block top-2 values over 1,024
-        // threads (C4: 1.3% a step); a few hundred over 256
-        if (c->nblk_force > 1024)
-          hipLaunchKernelGGL(k_skin<1024>, dim3(R), dim3(1024), 0, c->stream, c->P, c->ptrs(), c->nblk_force, G);
-        else
-          hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(), c->nblk_force, G);
-      }
-    };
+    key.seed = c->seed;
+    key.sep_huge = A.sep_huge;
+    bool wait_huge = false;
     // issued directly: the host's launch cost overlaps the device's work,
     // which pays for large systems (a graph launch costs more per node
     // than a kernel launch here)
-    if (c->pg_eager) {
-      run_phase_batches(c, launch_steps);
-      continue;
+    if (c->pg_eager || (c->opt.flags & SIS_OPT_NO_GRAPH)) {
+      wait_huge = run_phase_batches(c, stop, true, launch_batch);
+    } else {
+      int slot = -1;
+      for (int q = 0; q < 2; q++)
+        if (c->pg_exec[q] && std::memcmp(&key, &c->pg_key[q], sizeof key) == 0) slot = q;
+      if (slot < 0) {
+        // the slot of the other buffer's graph is kept when it is still valid
+        slot = 0;
+        if (c->pg_exec[0]) {
+          PhaseGraphKey k0 = c->pg_key[0];
+          k0.pos = key.pos;
+          k0.D.pos = key.D.pos;
+          k0.D.pos_out = key.D.pos_out;
+          if (std::memcmp(&k0, &key, sizeof key) == 0) slot = 1;
+        }
+        if (c->pg_exec[slot]) {
+          HIPCHK(hipGraphExecDestroy(c->pg_exec[slot]));
+          c->pg_exec[slot] = nullptr;
+        }
+        hipGraph_t graph = nullptr;
+        HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
+        launch_batch(GRAPH_STEPS);
+        HIPCHK(hipStreamEndCapture(c->stream, &graph));
+        HIPCHK(hipGraphInstantiate(&c->pg_exec[slot], graph, nullptr, nullptr, 0));
+        HIPCHK(hipGraphDestroy(graph));
+        c->pg_key[slot] = key;
+      }
+      const hipGraphExec_t ex = c->pg_exec[slot];
+      wait_huge = run_phase_batches(c, stop, false, [&](int) { HIPCHK(hipGraphLaunch(ex, c->stream)); });
     }
-    int slot = -1;
-    for (int q = 0; q < 2; q++)
-      if (c->pg_exec[q] && std::memcmp(&key, &c->pg_key[q], sizeof key) == 0) slot = q;
-    if (slot >= 0) {
-      hipGraphExec_t ex = c->pg_exec[slot];
-      run_phase_batches(c, [&]() { HIPCHK(hipGraphLaunch(ex, c->stream)); });
-      continue;
+    if (wait_huge) {
+      // the rest of that step; from now on such components have their
+      // launch in every step
+      c->step_sep_huge = true;
+      A.sep_huge = 1;
+      const StepWords w1{c->istep, stop, 0, w0.force_step, 0, 0};
+      HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w1, sizeof w1, hipMemcpyHostToDevice, c->stream));
+      A.nj = 1;
+      launch_step(1, 0);
+      HIPCHK(hipStreamSynchronize(c->stream));
+      c->istep++;
     }
-    // the slot of the other buffer's graph is kept when it is still valid
-    slot = 0;
-    if (c->pg_exec[0]) {
-      PhaseGraphKey k0 = c->pg_key[0];
-      k0.pos = key.pos;
-      k0.D.pos = key.D.pos;
-      k0.D.pos_out = key.D.pos_out;
-      if (std::memcmp(&k0, &key, sizeof key) == 0) slot = 1;
-    }
-    if (c->pg_exec[slot]) {
-      HIPCHK(hipGraphExecDestroy(c->pg_exec[slot]));
-      c->pg_exec[slot] = nullptr;
-    }
-    hipGraph_t graph = nullptr;
-    hipGraphExec_t exec = nullptr;
-    HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    launch_steps();
-    HIPCHK(hipStreamEndCapture(c->stream, &graph));
-    HIPCHK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
-    HIPCHK(hipGraphDestroy(graph));
-    c->pg_exec[slot] = exec;
-    c->pg_key[slot] = key;
-    run_phase_batches(c, [&]() { HIPCHK(hipGraphLaunch(exec, c->stream)); });
+    hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(), c->step_top2_d.p, nblk);
   }
 }
 
@@ -1374,6 +1447,7 @@ int sis_gpu_create(const sis_topo *topo, const sis_params *prm, const sis_option
         if (sq < 0 || sq > 4) throw ApiError{SIS_ERR_ARG, "sequence code out of range"};
         bool q = prm->dummy_has_charge ? true : sq != SQ_D;  // src/init_ele.F90:58-68
         if (!charged[imp]) q = false;
+        if (topo->moltype[ch] == 2) c->circular = true;
         c->topo[imp] = Topo{imp - i + 1, n, i, (topo->moltype[ch] == 2 ? 1 : 0) | (sq << 4) | ((q ? 1 : 0) << 8)};
       }
     }
@@ -1673,7 +1747,7 @@ int sis_gpu_force(sis_gpu_ctx *c, int32_t irep, int32_t bp_mc, double *forces) {
     // (which builds the MD job's lists itself)
     batched_force(c, irep - 1, bp_mc);
   } else {
-    bp_phase(c, &mc, nullptr, c->mask_d.p);
+    bp_phase(c, mc, nullptr, c->mask_d.p);
     force_kernel(c, 0, c->mask_d.p);
   }
   HIPCHK(hipEventRecord(c->ev1, c->stream));

@@ -421,6 +421,18 @@ __device__ __forceinline__ int uf_find(int *p, int x) {
   }
 }
 
+// one conflict component for the nucleotides a and b of a formed pair
+// (larger root linked under the smaller)
+__device__ __forceinline__ void uf_join(int *p, int a, int b) {
+  while (true) {
+    a = uf_find(p, a);
+    b = uf_find(p, b);
+    if (a == b) return;
+    if (a > b) { int t = a; a = b; b = t; }
+    if (atomicCAS(&p[b], b, a) == b) return;
+  }
+}
+
 // ---------------------------------------------------------------------
 // nbp_total < 0: the count of the current lists, read from the device (the
 // end of the candidates' scan; graph replays launch over the capacity)
@@ -473,20 +485,53 @@ __global__ void k_bp_eval(Params P, Ptrs D, int nbp_total, const int *mc, const 
     }
     atomicAdd(&D.nt_cnt[(size_t)r * N + mp[0] - 1], 1);
     atomicAdd(&D.nt_cnt[(size_t)r * N + mp[1] - 1], 1);
-    // performance-form MC: join the pair's nucleotides into one conflict
-    // component (union-find, larger root linked under the smaller)
-    if (do_union && mc[r]) {
-      int *pc = D.comp + (size_t)r * N;
-      int ua = mp[0] - 1, ub = mp[1] - 1;
-      while (true) {
-        ua = uf_find(pc, ua);
-        ub = uf_find(pc, ub);
-        if (ua == ub) break;
-        if (ua > ub) { int t = ua; ua = ub; ub = t; }
-        if (atomicCAS(&pc[ub], ub, ua) == ub) break;
-      }
-    }
+    // performance-form MC: one conflict component for the pair's nucleotides
+    if (do_union && mc[r]) uf_join(D.comp + (size_t)r * N, mp[0] - 1, mp[1] - 1);
   }
+}
+
+// one base-pair candidate (src/force_bp_limit_triplet.F90:85-256);
+// returns 1 if formed
+template <typename T>
+__device__ __forceinline__ int bp_eval_one(const Params &P, const Ptrs &D, int gb, int mc,
+                                           const double4 *xr = nullptr, const int *mpl = nullptr,
+                                           int *ntc = nullptr) {
+  const int *mp = mpl ? mpl : D.bp_mp + (size_t)gb * 8;   // mpl: the same record staged in LDS
+  const int r = mp[7];
+  const int N = P.N;
+  D.bp_status[gb] = 0;
+  D.ene_bp[gb] = 0.0;
+  if (!mc && P.nstep_bp_mc > 0 && !D.bp_status_mc[gb]) return 0;
+  double tK = D.tK[r];
+  double dG = 1.0;   // models 1/3: U0 exp(-u) (src/force_bp.F90:203)
+  if (P.bp_model == 5) {
+    dG = D.bp_coef[2 * (size_t)gb] - tK * D.bp_coef[2 * (size_t)gb + 1];
+    if (dG >= 0.0) return 0;
+  }
+  const double *box = D.box + 3 * r;
+  const double4 *x = xr ? xr : D.pos + (size_t)r * N;
+  double4 p1 = x[mp[0] - 1], p2 = x[mp[1] - 1];
+  V3<double> v12 = pvec(P, box, p1, p2), v13 = pvec(P, box, p1, x[mp[2] - 1]),
+             v15 = pvec(P, box, p1, x[mp[4] - 1]), v42 = pvec(P, box, x[mp[3] - 1], p2),
+             v62 = pvec(P, box, x[mp[5] - 1], p2);
+  const BpPara &bp = D.bpp[mp[6]];
+  T u;
+  V3<T> fb[6];
+  if (!bp_geom<T>(bp, v12, v13, v15, v42, v62, u, fb)) return 0;
+  double e = bp.U0 * dG * exp(-(double)u);
+  if (!(e <= P.bp_cutoff_energy)) return 0;   // also rejects a NaN energy
+  D.bp_status[gb] = 1;
+  D.ene_bp[gb] = e;
+  double *fo = D.for_bp + (size_t)gb * 18;
+  for (int q = 0; q < 6; q++) {
+    fo[3 * q] = e * (double)fb[q].x;
+    fo[3 * q + 1] = e * (double)fb[q].y;
+    fo[3 * q + 2] = e * (double)fb[q].z;
+  }
+  int *cnt = ntc ? ntc : D.nt_cnt + (size_t)r * N;   // ntc: this replica's counts in LDS
+  atomicAdd(&cnt[mp[0] - 1], 1);
+  atomicAdd(&cnt[mp[1] - 1], 1);
+  return 1;
 }
 
 // ---------------------------------------------------------------------
@@ -552,111 +597,7 @@ __global__ void k_mc_serial(Params P, Ptrs D, const int *mc, const double *ecT, 
 // only changes counts inside the component of the chosen nucleotide, and
 // the uniform choice among all excess nucleotides restricted to one
 // component is uniform within it.  Each component is therefore resolved
-// independently by one thread with its own counter-RNG stream.
-__global__ void k_uf_init(Params P, Ptrs D, int *cnt_exc, int *fill, const int *mask) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-  if (i >= P.N || (mask && !mask[r])) return;
-  size_t g = (size_t)r * P.N + i;
-  D.comp[g] = i;
-  cnt_exc[g] = 0;
-  fill[g] = 0;
-}
-__global__ void k_uf_union(Params P, Ptrs D, int nbp_total, const int *mc, const int *mask) {
-  int gb = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gb >= nbp_total || !D.bp_status[gb]) return;
-  const int *mp = D.bp_mp + (size_t)gb * 8;
-  int r = mp[7];
-  if ((mask && !mask[r]) || !mc[r]) return;
-  int *p = D.comp + (size_t)r * P.N;
-  int a = mp[0] - 1, b = mp[1] - 1;
-  while (true) {
-    a = uf_find(p, a);
-    b = uf_find(p, b);
-    if (a == b) return;
-    if (a > b) { int t = a; a = b; b = t; }
-    if (atomicCAS(&p[b], b, a) == b) return;  // link larger root under smaller
-  }
-}
-__global__ void k_uf_count(Params P, Ptrs D, int *cnt_exc, const int *mc, const int *mask) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-  if (i >= P.N || (mask && !mask[r]) || !mc[r]) return;
-  size_t g = (size_t)r * P.N + i;
-  if (D.nt_cnt[g] > 0) {
-    int root = uf_find(D.comp + (size_t)r * P.N, i);
-    atomicAdd(&cnt_exc[(size_t)r * P.N + root], 1);
-  }
-}
-__global__ void k_uf_fill(Params P, Ptrs D, const int *exc_off, int *fill, int *exc_list,
-                          const int *mc, const int *mask) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-  if (i >= P.N || (mask && !mask[r]) || !mc[r]) return;
-  size_t g = (size_t)r * P.N + i;
-  if (D.nt_cnt[g] > 0) {
-    int root = uf_find(D.comp + (size_t)r * P.N, i);
-    size_t gr = (size_t)r * P.N + root;
-    int slot = atomicAdd(&fill[gr], 1);
-    exc_list[exc_off[gr] + slot] = i;
-  }
-}
-__global__ void k_mc_comp(Params P, Ptrs D, const int *exc_off, const int *cnt_exc,
-                          int *exc_list, const int *mc, const double *ecT, uint64_t seed,
-                          int64_t step, const int *mask) {
-  int root = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-  if (root >= P.N || (mask && !mask[r]) || !mc[r]) return;
-  const int N = P.N;
-  size_t gr = (size_t)r * N + root;
-  int ne = cnt_exc[gr];
-  if (ne == 0) return;
-  int *E = exc_list + exc_off[gr];
-  for (int x = 1; x < ne; x++) {
-    int v = E[x], y = x - 1;
-    while (y >= 0 && E[y] > v) { E[y + 1] = E[y]; y--; }
-    E[y + 1] = v;
-  }
-  double tK = ecT ? ecT[r] : D.tK[r];
-  double beta = mc_beta(P, tK, ecT == nullptr);
-  int *cnt = D.nt_cnt + (size_t)r * N;
-  uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)(seed >> 32) ^ (0x5bd1e995u * (uint32_t)(r + 1));
-  uint32_t draw = 0;
-  auto uni = [&]() {
-    U4 o = philox(U4{(uint32_t)step, (uint32_t)(step >> 32) ^ 0x4d43u, (uint32_t)root, draw++}, k0, k1);
-    return u01(o.x, o.y);
-  };
-  const int CAP = 64;
-  int seqv[CAP];
-  size_t st = N;
-  for (;;) {
-    int nact = 0;
-    for (int k = 0; k < ne; k++) nact += cnt[E[k]] > 0;
-    if (nact == 0) break;
-    int pick = (int)ceil(uni() * nact), ntd = -1;
-    for (int k = 0, c = 0; k < ne; k++)
-      if (cnt[E[k]] > 0 && ++c == pick) { ntd = E[k]; break; }
-    if (ntd < 0) break;
-    int ni = min(D.n_inc[(size_t)r * N + ntd], D.maxinc), ns = 0;
-    const int *inc = D.inc + (size_t)r * D.maxinc * N + ntd;
-    for (int k = 0; k < ni && ns < CAP; k++) {
-      int e = inc[k * st], gb = e >> 3, role = e & 7;
-      if (role <= 1 && D.bp_status[gb]) seqv[ns++] = gb;
-    }
-    for (int k = 0; k < ns; k++) {
-      int sw = (int)ceil(uni() * ns) - 1;
-      int sv = seqv[k]; seqv[k] = seqv[sw]; seqv[sw] = sv;
-    }
-    if (ns == 0) { D.flags[1] = 2; break; }
-    int del = seqv[0];
-    for (int k = 1; k < ns; k++) {
-      int jb = seqv[k];
-      double ratio = exp((D.ene_bp[jb] - D.ene_bp[del]) * beta);
-      if (uni() < ratio) del = jb;
-    }
-    D.bp_status[del] = 0;
-    const int *mp = D.bp_mp + (size_t)del * 8;
-    cnt[mp[0] - 1] -= 1;
-    cnt[mp[1] - 1] -= 1;
-  }
-}
-
+// independently with its own counter-RNG stream.
 // Performance-form components: union-find roots, pairs bucketed per root
 // (capacity SEGCAP per component), one wavefront per component with excess.
 constexpr int SEGCAP = 256;
@@ -681,26 +622,29 @@ __global__ void k_mc_reset(Params P, Ptrs D, int *seg_n, int *has_exc, int *exc_
   seg_n[g] = 0;
   has_exc[g] = 0;
 }
-__global__ void k_seg_fill(Params P, Ptrs D, int nbp_total, int *seg_n, int *seg, int *has_exc,
-                           const int *mc, const int *mask, int *exc_list) {
-  int gb = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gb >= bp_count(P, D, nbp_total) || !D.bp_status[gb]) return;
+// formed pair gb into the bucket of its component; the component listed if
+// it has excess (exc_list: [0] count, then replica * N + root)
+__device__ __forceinline__ void seg_fill_one(const Params &P, const Ptrs &D, int gb, int *seg_n, int *seg, int *has_exc,
+                                             int *exc_list) {
   const int *mp = D.bp_mp + (size_t)gb * 8;
-  int r = mp[7];
-  if ((mask && !mask[r]) || !mc[r]) return;
-  const int N = P.N;
+  const int r = mp[7], N = P.N;
   int a = mp[0] - 1, b = mp[1] - 1;
-  // the counts (final since k_bp_eval) are loaded before the dependent
+  // the counts (final since the evaluation) are loaded before the dependent
   // chain of the root walk and the bucket atomic, not after it
   const bool exc = D.nt_cnt[(size_t)r * N + a] > 0 || D.nt_cnt[(size_t)r * N + b] > 0;
   int root = uf_find(D.comp + (size_t)r * N, a);
   size_t gr = (size_t)r * N + root;
   int slot = atomicAdd(&seg_n[gr], 1);
   if (slot < SEGCAP) seg[gr * SEGCAP + slot] = gb;
-  if (exc) {
-    // listed once (exc_list: [0] count, then replica * N + root)
-    if (atomicExch(&has_exc[gr], 1) == 0 && exc_list) exc_list[1 + atomicAdd(&exc_list[0], 1)] = (int)gr;
-  }
+  if (exc && atomicExch(&has_exc[gr], 1) == 0) exc_list[1 + atomicAdd(&exc_list[0], 1)] = (int)gr;   // listed once
+}
+__global__ void k_seg_fill(Params P, Ptrs D, int nbp_total, int *seg_n, int *seg, int *has_exc,
+                           const int *mc, const int *mask, int *exc_list) {
+  int gb = blockIdx.x * blockDim.x + threadIdx.x;
+  if (gb >= nbp_total || !D.bp_status[gb]) return;
+  const int r = D.bp_mp[(size_t)gb * 8 + 7];
+  if ((mask && !mask[r]) || !mc[r]) return;
+  seg_fill_one(P, D, gb, seg_n, seg, has_exc, exc_list);
 }
 // serial fallback for a component larger than one wave holds: the same
 // algorithm on global memory by one lane
@@ -960,14 +904,11 @@ __device__ __noinline__ bool mc_component_huge(const McArrays D, const int N, in
   return true;
 }
 
-// Per-phase form: components above SEGCAP pairs, one wavefront per
-// replica after k_mc_wave (which marks the replicas that have them).
-__global__ void __launch_bounds__(64) k_mc_huge(Params P, Ptrs D, const int *seg_n, int *seg, const int *has_exc,
-                                                int *huge, const double *ecT, uint64_t seed, int64_t step0,
-                                                const int64_t *step_dev) {
-  const int r = blockIdx.x, L = threadIdx.x, N = P.N;
-  if (!huge[r]) return;
-  const int64_t step = step_dev ? *step_dev : step0;   // graph replays read the step from the device
+// Per-phase form: the components of replica r above SEGCAP pairs, by one
+// wavefront (64 threads) after the others are resolved
+__device__ __forceinline__ void mc_huge_replica(const Params &P, const Ptrs &D, int r, const int *seg_n, int *seg,
+                                                const int *has_exc, const double *ecT, uint64_t seed, int64_t step) {
+  const int L = threadIdx.x, N = P.N;
   __shared__ int sseq[64];
   const double tK = ecT ? ecT[r] : D.tK[r];
   const double beta = mc_beta(P, tK, ecT == nullptr);
@@ -987,53 +928,46 @@ __global__ void __launch_bounds__(64) k_mc_huge(Params P, Ptrs D, const int *seg
         if (L == 0) D.flags[5] = 1;
     }
   }
-  if (L == 0) huge[r] = 0;
 }
-// one conflict component (root of replica r) resolved by a 64-thread
-// block: one lane, one wavefront, or the serial fallback; components above
-// the bucket capacity are flagged for k_mc_huge
-__device__ __forceinline__ void mc_one_component(const Params &P, const Ptrs &D, int r, int root, int *seg_n,
+// ... for the replicas that k_mc_list marked
+__global__ void __launch_bounds__(64) k_mc_huge(Params P, Ptrs D, const int *seg_n, int *seg, const int *has_exc,
+                                                int *huge, const double *ecT, uint64_t seed, int64_t step) {
+  const int r = blockIdx.x;
+  if (!huge[r]) return;
+  mc_huge_replica(P, D, r, seg_n, seg, has_exc, ecT, seed, step);
+  if (threadIdx.x == 0) huge[r] = 0;
+}
+// one conflict component (root of replica r) resolved by a wavefront with
+// MCB_LDS ints of LDS: one lane, the whole wave, or the serial fallback; a
+// component above the bucket capacity is flagged in huge[r] (returns true)
+__device__ __forceinline__ bool mc_one_component(const Params &P, const Ptrs &D, int r, int root, int *seg_n,
                                                  int *seg, const double *ecT, uint64_t seed, int64_t step,
                                                  int *huge, int *ws) {
+  const int L = lane_id();
   size_t gr = (size_t)r * P.N + root;
   int n = seg_n[gr];
   double tK = ecT ? ecT[r] : D.tK[r];
   double beta = mc_beta(P, tK, ecT == nullptr);
-  if (n > SEGCAP) {   // above the bucket capacity: k_mc_huge takes it
-    if (threadIdx.x == 0) huge[r] = 1;
-    return;
+  if (n > SEGCAP) {
+    if (L == 0) huge[r] = 1;
+    return true;
   }
   int *sg = seg + gr * SEGCAP;
-  if (n <= MCL_PAIRS) {   // small component: one lane, same result
-    if (threadIdx.x == 0 && !mc_component_lane(D, P.max_bp_per_nt, P.N, r, root, sg, n, beta, seed, step))
+  if (n <= MCL_PAIRS) {   // two pairs: one lane, same result
+    if (L == 0 && !mc_component_lane(D, P.max_bp_per_nt, P.N, r, root, sg, n, beta, seed, step))
       mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
-    return;
+    return false;
   }
   const bool ok = n <= 64 * MCW_ITEMS ? mc_component_wave_any(P, D, r, r, root, sg, n, beta, seed, step, ws)
                                       : mc_component_wave<MCB_ITEMS, MCB_NODES>(P, D, r, r, root, sg, n, beta, seed, step, ws);
-  if (!ok && threadIdx.x == 0) mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
-}
-
-__global__ void __launch_bounds__(64) k_mc_wave(Params P, Ptrs D, int *seg_n, int *seg,
-                                                const int *has_exc, const int *mc,
-                                                const double *ecT, uint64_t seed, int64_t step0,
-                                                const int *mask, int *huge, const int64_t *step_dev) {
-  int root = blockIdx.x, r = blockIdx.y;
-  if ((mask && !mask[r]) || !mc[r]) return;
-  const int64_t step = step_dev ? *step_dev : step0;   // graph replays read the step from the device
-  size_t gr = (size_t)r * P.N + root;
-  if (!has_exc[gr]) return;
-  __shared__ __align__(16) int ws[MCB_LDS];
-  mc_one_component(P, D, r, root, seg_n, seg, ecT, seed, step, huge, ws);
+  if (!ok && L == 0) mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
+  return false;
 }
 
 // The components listed by k_seg_fill (exc_list: [0] count, then
-// replica * N + root), a grid-stride loop of 64-thread blocks: the same
-// per-component work as k_mc_wave without a block per nucleotide.
+// replica * N + root), a grid-stride loop of 64-thread blocks.
 __global__ void __launch_bounds__(64) k_mc_list(Params P, Ptrs D, int *seg_n, int *seg, const int *exc_list,
-                                                const double *ecT, uint64_t seed, int64_t step0, int *huge,
-                                                const int64_t *step_dev) {
-  const int64_t step = step_dev ? *step_dev : step0;
+                                                const double *ecT, uint64_t seed, int64_t step, int *huge) {
   const int n = exc_list[0];
   __shared__ __align__(16) int ws[MCB_LDS];
   for (int k = blockIdx.x; k < n; k += gridDim.x) {
@@ -1082,102 +1016,6 @@ __global__ void k_noise_parity(Params P, Ptrs D, int count, int dest, const int 
 }
 
 // ---------------------------------------------------------------------
-// Owner-computes force on bead a of replica r: bonded terms recomputed
-// per owner, WCA / DH over the full neighbour lists, 6-bead BP forces
-// gathered through the incidence list (no atomics on forces).
-template <typename T>
-__device__ __forceinline__ V3<double> bead_force(const Params &P, const Ptrs &D, int r, int a) {
-  const int N = P.N;
-  const double *box = D.box + 3 * r;
-  const double4 *x = D.pos + (size_t)r * N;
-  double4 pa = x[a];
-  Topo ta = D.topo[a];
-  int loc = ta.loc, n = ta.len, st = ta.start;
-  bool circ = topo_circ(ta);
-  V3<double> F{0.0, 0.0, 0.0};
-  auto at = [&](int s, int k) -> int {  // bead of term starting at local s, position k
-    int l = s + k;
-    if (l > n) l -= n;
-    return st + l - 1;
-  };
-  auto valid = [&](int &s, int m) -> bool {  // term of m beads starting at local s
-    if (circ) {
-      if (n < m) return false;
-      if (s < 1) s += n;
-      return true;
-    }
-    return s >= 1 && s + m - 1 <= n;
-  };
-  // bonds (src/list_local.F90:24-58)
-  for (int p = 0; p < 2; p++) {
-    int s = loc - p;
-    if (!valid(s, 2)) continue;
-    V3<double> v = pvec(P, box, x[at(s, 0)], x[at(s, 1)]);
-    V3<double> f[2];
-    bond_force<double>(P, v, f);
-    F = F + f[p];
-  }
-  for (int p = 0; p < 3; p++) {
-    int s = loc - p;
-    if (!valid(s, 3)) continue;
-    double4 p0 = x[at(s, 0)], p1 = x[at(s, 1)], p2 = x[at(s, 2)];
-    V3<double> v12 = pvec(P, box, p0, p1), v32 = pvec(P, box, p2, p1);
-    V3<double> f[3];
-    angle_force<double>(P, v12, v32, f);
-    F = F + f[p];
-  }
-  if (P.dih_type) {
-    for (int p = 0; p < 4; p++) {
-      int s = loc - p;
-      if (!valid(s, 4)) continue;
-      double4 p0 = x[at(s, 0)], p1 = x[at(s, 1)], p2 = x[at(s, 2)], p3 = x[at(s, 3)];
-      V3<double> vij = pvec(P, box, p0, p1), vkj = pvec(P, box, p2, p1), vkl = pvec(P, box, p2, p3);
-      V3<double> f[4];
-      dih_force<double>(P, vij, vkj, vkl, f);
-      F = F + f[p];
-    }
-  }
-  size_t g = (size_t)r * N + a;
-  // WCA
-  {
-    int nw = min(D.n_wca[g], D.maxw);
-    const int *nb = D.nb_wca + (size_t)r * D.maxw * N + a;
-    for (int k = 0; k < nw; k++) {
-      int b = nb[(size_t)k * N];
-      V3<T> v = cvt<T>(pvec(P, box, pa, x[b]));
-      F = F + cvt<double>(wca_force<T>(P, v));
-    }
-  }
-  // Debye-Hueckel
-  if (P.ele_on) {
-    int ne = min(D.n_ele[g], D.maxnb);
-    const int *nb = D.nb_ele + (size_t)r * D.maxnb * N + a;
-    T coef = (T)D.ele_coef[r], rc2 = (T)(D.ele_cut[r] * D.ele_cut[r]), rl = (T)(1.0 / D.lambdaD[r]);
-    V3<T> acc{0, 0, 0};
-    V3<double> accd{0.0, 0.0, 0.0};
-    for (int k = 0; k < ne; k++) {
-      int b = nb[(size_t)k * N];
-      V3<T> v = cvt<T>(pvec(P, box, pa, x[b]));
-      V3<T> f = dh_force<T>(coef, rc2, rl, v);
-      accd = accd + cvt<double>(f);
-    }
-    (void)acc;
-    F = F + accd;
-  }
-  // base pairs
-  {
-    int ni = min(D.n_inc[g], D.maxinc);
-    const int *inc = D.inc + (size_t)r * D.maxinc * N + a;
-    for (int k = 0; k < ni; k++) {
-      int e = inc[(size_t)k * N], gb = e >> 3, role = e & 7;
-      if (!D.bp_status[gb]) continue;
-      const double *fo = D.for_bp + (size_t)gb * 18 + 3 * role;
-      F.x += fo[0]; F.y += fo[1]; F.z += fo[2];
-    }
-  }
-  return F;
-}
-
 // GJF-2GJ update of one bead (src/job_md.F90:415-444), or the
 // Ermak-McCammon Brownian step (lines 446-456) when P.bd; g = r*N + a.
 // Returns |move|^2.
@@ -1210,63 +1048,6 @@ __device__ __forceinline__ double move_bead(const Params &P, const Ptrs &D, size
   // other beads still read D.pos in this pass: write the next buffer
   D.pos_out[g] = double4{p.x + dx, p.y + dy, p.z + dz, p.w};
   return dot_nc(mv.x, mv.y, mv.z, mv.x, mv.y, mv.z);
-}
-
-// Force (and optionally the GJF-2GJ update, src/job_md.F90:415-444) per
-// bead; block-level top-2 of the accumulated displacement for the skin
-// test (src/job_md.F90:376-386).
-template <typename T, int B>
-__global__ void __launch_bounds__(B) k_force_int(Params P, Ptrs D, int integrate, int parity,
-                                                uint64_t seed, int64_t step, const int *mask) {
-  __shared__ double s1[B], s2[B];
-  int a = blockIdx.x * B + threadIdx.x, r = blockIdx.y;
-  const int N = P.N;
-  double d2 = 0.0;
-  bool act = a < N && !(mask && !mask[r]);
-  if (act) {
-    size_t g = (size_t)r * N + a;
-    V3<double> F = bead_force<T>(P, D, r, a);
-    D.nt_cnt[g] = -P.max_bp_per_nt;
-    if (!integrate) {
-      D.frc[g] = double4{F.x, F.y, F.z, 0.0};
-    } else {
-      double n0, n1, n2;
-      if (parity) {
-        const double *nz = D.noise + g * 3;
-        n0 = nz[0]; n1 = nz[1]; n2 = nz[2];
-      } else {
-        U4 o = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6973u},
-                      (uint32_t)seed, (uint32_t)(seed >> 32) ^ (0x9e3779b9u * (uint32_t)(r + 1)));
-        U4 o2 = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6974u},
-                       (uint32_t)seed, (uint32_t)(seed >> 32) ^ (0x9e3779b9u * (uint32_t)(r + 1)));
-        double u1 = u01(o.x, o.y), u2 = u01(o.z, o.w), u3 = u01(o2.x, o2.y), u4 = u01(o2.z, o2.w);
-        double rr = sqrt(-2.0 * log(u1)), r2 = sqrt(-2.0 * log(u3));
-        n0 = rr * cos(6.283185307179586 * u2);
-        n1 = rr * sin(6.283185307179586 * u2);
-        n2 = r2 * cos(6.283185307179586 * u4);
-      }
-      d2 = move_bead(P, D, g, a, F, n0, n1, n2);
-    }
-  }
-  if (!integrate) return;
-  // block top-2 of d2
-  s1[threadIdx.x] = d2;
-  s2[threadIdx.x] = 0.0;
-  __syncthreads();
-  for (int off = B / 2; off > 0; off >>= 1) {
-    if (threadIdx.x < off) {
-      double a1 = s1[threadIdx.x], a2 = s2[threadIdx.x], b1 = s1[threadIdx.x + off], b2 = s2[threadIdx.x + off];
-      double m1 = a1 > b1 ? a1 : b1;
-      double m2 = a1 > b1 ? (a2 > b1 ? a2 : b1) : (a1 > b2 ? a1 : b2);
-      s1[threadIdx.x] = m1;
-      s2[threadIdx.x] = m2;
-    }
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    D.blk_top2[((size_t)r * gridDim.x + blockIdx.x) * 2] = s1[0];
-    D.blk_top2[((size_t)r * gridDim.x + blockIdx.x) * 2 + 1] = s2[0];
-  }
 }
 
 // Lane-split owner-computes: LPB lanes share bead a; lane l takes items
@@ -1377,16 +1158,47 @@ __device__ __forceinline__ V3<double> pair_bp(const Params &P, const Ptrs &D, in
   return F;
 }
 
+// pair_bp of a bead by one lane: incidences in batches of four, their
+// loads issued before the sums
+__device__ __forceinline__ V3<double> pair_bp4(const Params &P, const Ptrs &D, int r, int a, V3<double> F) {
+  const int N = P.N;
+  const int ni = min(D.n_inc[(size_t)r * N + a], D.maxinc);
+  const int *inc = D.inc + (size_t)r * D.maxinc * N + a;
+  for (int k0 = 0; k0 < ni; k0 += 4) {
+    int e[4];
+    bool on[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) e[u] = k0 + u < ni ? inc[(size_t)(k0 + u) * N] : -1;
+#pragma unroll
+    for (int u = 0; u < 4; u++) on[u] = e[u] >= 0 && D.bp_status[e[u] >> 3];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+      if (on[u]) {
+        const double *fo = D.for_bp + (size_t)(e[u] >> 3) * 18 + 3 * (e[u] & 7);
+        F.x += fo[0]; F.y += fo[1]; F.z += fo[2];
+      }
+  }
+  return F;
+}
+
 template <typename T>
 __device__ __forceinline__ V3<double> pair_part(const Params &P, const Ptrs &D, int r, int a, int l,
                                                 int LPB, const double4 *xr = nullptr) {
   return pair_bp(P, D, r, a, l, LPB, pair_nb<T>(P, D, r, a, l, LPB, xr, V3<double>{0.0, 0.0, 0.0}));
 }
 
-template <typename T>
-__device__ __forceinline__ V3<double> bead_force_part(const Params &P, const Ptrs &D, int r, int a,
-                                                      int l, int LPB) {
-  return bonded_part(P, D, r, a, l, LPB) + pair_part<T>(P, D, r, a, l, LPB);
+// The three normal draws of bead a on `step` (counter RNG; rk keys the
+// replica's stream)
+__device__ __forceinline__ void noise_normals(uint64_t seed, int rk, int64_t step, int a, double &n0, double &n1,
+                                              double &n2) {
+  uint32_t k1 = (uint32_t)(seed >> 32) ^ (0x9e3779b9u * (uint32_t)(rk + 1));
+  U4 o = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6973u}, (uint32_t)seed, k1);
+  U4 o2 = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6974u}, (uint32_t)seed, k1);
+  double u1 = u01(o.x, o.y), u2 = u01(o.z, o.w), u3 = u01(o2.x, o2.y), u4 = u01(o2.z, o2.w);
+  double rr = sqrt(-2.0 * log(u1)), r2 = sqrt(-2.0 * log(u3));
+  n0 = rr * cos(6.283185307179586 * u2);
+  n1 = rr * sin(6.283185307179586 * u2);
+  n2 = r2 * cos(6.283185307179586 * u4);
 }
 
 // One bead's update with its noise draws (the injected MT words in the
@@ -1401,14 +1213,7 @@ __device__ __forceinline__ double gjf_update(const Params &P, const Ptrs &D, int
     const double *nz = D.noise + g * 3;
     n0 = nz[0]; n1 = nz[1]; n2 = nz[2];
   } else {
-    uint32_t k1 = (uint32_t)(seed >> 32) ^ (0x9e3779b9u * (uint32_t)(rk + 1));
-    U4 o = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6973u}, (uint32_t)seed, k1);
-    U4 o2 = philox(U4{(uint32_t)step, (uint32_t)(step >> 32), (uint32_t)a, 0x6e6f6974u}, (uint32_t)seed, k1);
-    double u1 = u01(o.x, o.y), u2 = u01(o.z, o.w), u3 = u01(o2.x, o2.y), u4 = u01(o2.z, o2.w);
-    double rr = sqrt(-2.0 * log(u1)), r2 = sqrt(-2.0 * log(u3));
-    n0 = rr * cos(6.283185307179586 * u2);
-    n1 = rr * sin(6.283185307179586 * u2);
-    n2 = r2 * cos(6.283185307179586 * u4);
+    noise_normals(seed, rk, step, a, n0, n1, n2);
   }
   return move_bead(P, D, g, a, F, n0, n1, n2);
 }
@@ -1444,53 +1249,6 @@ __device__ __forceinline__ void top2_merge(double &m1, double &m2, double b1, do
   m2 = n2;
 }
 
-// Steps replayed from a captured graph (the per-phase form without a host
-// round trip per step): the step each launch works on, when it stops, and
-// the rebuild it stopped for.
-struct GStep {
-  int64_t *istep;        // [1] last completed step
-  int64_t *istep_cur;    // [1] step of the current launch sequence
-  const int64_t *stop;   // [1] stop once this step is completed
-  int *halt;             // [1] 1: the next steps do nothing (a rebuild or the stop is due)
-  int *active;           // [R] mask of the step's kernels (0 after a halt)
-  int *force_mc;         // [R] limit MC on the next step (after a rebuild)
-  int *mc;               // [R] limit MC on the current step
-};
-
-// the skin decision of replica r from its nblk block maxima, reduced by the
-// calling workgroup (B threads, s1/s2 of B doubles); with a graph step
-// also the halt and the step's commit.  Called by every thread.
-template <int B>
-__device__ __forceinline__ void skin_decide(const Params &P, const Ptrs &D, int r, int nblk, const GStep &G,
-                                            double *s1, double *s2) {
-  const int t = threadIdx.x;
-  double m1 = 0.0, m2 = 0.0;
-  for (int b = t; b < nblk; b += B)
-    top2_merge(m1, m2, D.blk_top2[((size_t)r * nblk + b) * 2], D.blk_top2[((size_t)r * nblk + b) * 2 + 1]);
-  s1[t] = m1;
-  s2[t] = m2;
-  __syncthreads();
-  for (int off = B / 2; off > 0; off >>= 1) {
-    if (t < off) {
-      double a1 = s1[t], a2 = s2[t];
-      top2_merge(a1, a2, s1[t + off], s2[t + off]);
-      s1[t] = a1;
-      s2[t] = a2;
-    }
-    __syncthreads();
-  }
-  if (t != 0) return;
-  const int f = (sqrt(s1[0]) + sqrt(s2[0]) > P.nl_margin) ? 1 : 0;
-  D.rebuild_flag[r] = f;
-  if (G.halt) {
-    if (f) atomicOr(G.halt, 1);
-    if (r == 0) {
-      *G.istep = *G.istep_cur;
-      if (*G.istep_cur >= *G.stop) atomicOr(G.halt, 1);
-    }
-  }
-}
-
 // Workgroups are dispatched to the eight XCDs in turn (linear ID mod 8),
 // each XCD with its own L2.  xcd_tile maps a linear workgroup ID to a tile
 // so that XCD x takes the x-th contiguous slice of the n tiles: the
@@ -1501,12 +1259,13 @@ __device__ __forceinline__ int xcd_tile(int id, int n) {
   return x * q + min(x, rem) + (id >> 3);
 }
 
+// Force of every bead and its update in one pass: LPB lanes a bead over the
+// pair lists, the base-pair incidences and the bonded terms.  g_own: the
+// bead this thread updated (unchanged if none).
 template <typename T, int LPB, int B>
-__global__ void __launch_bounds__(B) k_force_lanes(Params P, Ptrs D, int integrate, int parity,
-                                                  uint64_t seed, int64_t step0, const int *mask,
-                                                  const int64_t *step_dev, int bonded_inline) {
+__device__ __forceinline__ void force_lanes(const Params &P, const Ptrs &D, int integrate, int parity, uint64_t seed,
+                                            int64_t step, const int *mask, int bonded_inline, double *top2, int &g_own) {
   __shared__ double s1[B / LPB], s2[B / LPB];
-  const int64_t step = step_dev ? *step_dev : step0;   // graph replays read the step from the device
   const int grp = threadIdx.x / LPB, l = threadIdx.x % LPB;
   // tile (bx, r) of this workgroup: grid x = tiles of a replica, y = replicas
   const int tile = xcd_tile(blockIdx.y * gridDim.x + blockIdx.x, gridDim.x * gridDim.y);
@@ -1530,6 +1289,7 @@ __global__ void __launch_bounds__(B) k_force_lanes(Params P, Ptrs D, int integra
     const double4 fb = bonded_inline ? double4{Fb.x, Fb.y, Fb.z, 0.0} : D.fbond[g];
     F.x += fb.x; F.y += fb.y; F.z += fb.z;
     D.nt_cnt[g] = -P.max_bp_per_nt;
+    g_own = (int)g;
     if (!integrate) D.frc[g] = double4{F.x, F.y, F.z, 0.0};
     else d2 = gjf_update(P, D, r, r, a, F, parity, seed, step);
   }
@@ -1545,73 +1305,41 @@ __global__ void __launch_bounds__(B) k_force_lanes(Params P, Ptrs D, int integra
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    D.blk_top2[((size_t)r * gridDim.x + bx) * 2] = s1[0];
-    D.blk_top2[((size_t)r * gridDim.x + bx) * 2 + 1] = s2[0];
+    top2[((size_t)r * gridDim.x + bx) * 2] = s1[0];
+    top2[((size_t)r * gridDim.x + bx) * 2 + 1] = s2[0];
   }
 }
+template <typename T, int LPB, int B>
+__global__ void __launch_bounds__(B) k_force_lanes(Params P, Ptrs D, int integrate, int parity, uint64_t seed,
+                                                  int64_t step, const int *mask, int bonded_inline) {
+  int g;
+  force_lanes<T, LPB, B>(P, D, integrate, parity, seed, step, mask, bonded_inline, D.blk_top2, g);
+}
+
 
 // skin test per replica (src/job_md.F90:376-395): sqrt(d2max) +
-// sqrt(d2max_2nd) > nl_margin over the per-block top-2 displacements,
-// reduced by a workgroup (the top two are the same values in any order).
-// With a graph step: a replica needing a rebuild halts the steps that
-// follow, and the step is committed.
+// sqrt(d2max_2nd) > nl_margin over the top-2 displacements of nblk blocks
+// (top2), reduced by a workgroup (the top two are the same values in any
+// order).
 template <int B>
-__global__ void __launch_bounds__(B) k_skin(Params P, Ptrs D, int nblk, GStep G) {
+__global__ void __launch_bounds__(B) k_skin(Params P, Ptrs D, const double *top2, int nblk) {
   __shared__ double s1[B], s2[B];
-  const int r = blockIdx.x;
-  if (G.halt && !G.active[r]) return;
-  skin_decide<B>(P, D, r, nblk, G, s1, s2);
-}
-
-// start of a replayed step: nothing if halted; else the step number and
-// the limit-MC flags (every nstep_MC steps and after a rebuild,
-// src/job_md.F90:364-394)
-__global__ void k_gstep_begin(Params P, GStep G) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= P.R) return;
-  const bool halted = *G.halt != 0;
-  G.active[r] = halted ? 0 : 1;
-  if (halted) return;
-  const int64_t s = *G.istep + 1;
-  if (r == 0) *G.istep_cur = s;
-  G.mc[r] = P.nstep_bp_mc > 0 && ((s % P.nstep_bp_mc) == 0 || G.force_mc[r]) ? 1 : 0;
-  G.force_mc[r] = 0;
-}
-
-// start of a replayed step and its resets in one pass: the step number,
-// limit-MC flags and mask (as k_gstep_begin), then for an active step the
-// formed-pair counts and, for the performance-form MC, union-find parents,
-// buckets and the list of components with excess (as k_mc_reset)
-__global__ void k_gstep_reset(Params P, Ptrs D, GStep G, int *seg_n, int *has_exc, int *exc_list, int mc_reset) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x, r = blockIdx.y;
-  const bool halted = *G.halt != 0;
-  if (i == 0) {
-    G.active[r] = halted ? 0 : 1;
-    if (!halted) {
-      const int64_t s = *G.istep + 1;
-      if (r == 0) *G.istep_cur = s;
-      G.mc[r] = P.nstep_bp_mc > 0 && ((s % P.nstep_bp_mc) == 0 || G.force_mc[r]) ? 1 : 0;
-      G.force_mc[r] = 0;
+  const int r = blockIdx.x, t = threadIdx.x;
+  double m1 = 0.0, m2 = 0.0;
+  for (int b = t; b < nblk; b += B) top2_merge(m1, m2, top2[((size_t)r * nblk + b) * 2], top2[((size_t)r * nblk + b) * 2 + 1]);
+  s1[t] = m1;
+  s2[t] = m2;
+  __syncthreads();
+  for (int off = B / 2; off > 0; off >>= 1) {
+    if (t < off) {
+      double a1 = s1[t], a2 = s2[t];
+      top2_merge(a1, a2, s1[t + off], s2[t + off]);
+      s1[t] = a1;
+      s2[t] = a2;
     }
-    if (r == 0 && exc_list) exc_list[0] = 0;
+    __syncthreads();
   }
-  if (halted || i >= P.N) return;
-  const size_t g = (size_t)r * P.N + i;
-  D.nt_cnt[g] = -P.max_bp_per_nt;
-  if (mc_reset) {
-    D.comp[g] = i;
-    seg_n[g] = 0;
-    has_exc[g] = 0;
-  }
-}
-
-// bp_status_MC = bp_status for the replicas that did the MC this step
-// (src/job_md.F90:399-401)
-__global__ void k_mc_keep(Params P, Ptrs D, int nbp_total, const int *mc, const int *mask) {
-  const int gb = blockIdx.x * blockDim.x + threadIdx.x;
-  if (gb >= bp_count(P, D, nbp_total)) return;
-  const int r = D.bp_mp[(size_t)gb * 8 + 7];
-  if (mask[r] && mc[r]) D.bp_status_mc[gb] = D.bp_status[gb];
+  if (t == 0) D.rebuild_flag[r] = (sqrt(s1[0]) + sqrt(s2[0]) > P.nl_margin) ? 1 : 0;
 }
 
 __global__ void k_clear_move(Params P, Ptrs D, const int *mask) {

@@ -41,50 +41,6 @@ __device__ __forceinline__ void grid_barrier(unsigned long long *bar, unsigned l
   __syncthreads();
 }
 
-// one candidate of phase A (src/force_bp_limit_triplet.F90:85-256);
-// returns 1 if formed
-template <typename T>
-__device__ __forceinline__ int bp_eval_one(const Params &P, const Ptrs &D, int gb, int mc,
-                                           const double4 *xr = nullptr, const int *mpl = nullptr,
-                                           int *ntc = nullptr) {
-  const int *mp = mpl ? mpl : D.bp_mp + (size_t)gb * 8;   // mpl: the same record staged in LDS
-  const int r = mp[7];
-  const int N = P.N;
-  D.bp_status[gb] = 0;
-  D.ene_bp[gb] = 0.0;
-  if (!mc && P.nstep_bp_mc > 0 && !D.bp_status_mc[gb]) return 0;
-  double tK = D.tK[r];
-  double dG = 1.0;   // models 1/3: U0 exp(-u) (src/force_bp.F90:203)
-  if (P.bp_model == 5) {
-    dG = D.bp_coef[2 * (size_t)gb] - tK * D.bp_coef[2 * (size_t)gb + 1];
-    if (dG >= 0.0) return 0;
-  }
-  const double *box = D.box + 3 * r;
-  const double4 *x = xr ? xr : D.pos + (size_t)r * N;
-  double4 p1 = x[mp[0] - 1], p2 = x[mp[1] - 1];
-  V3<double> v12 = pvec(P, box, p1, p2), v13 = pvec(P, box, p1, x[mp[2] - 1]),
-             v15 = pvec(P, box, p1, x[mp[4] - 1]), v42 = pvec(P, box, x[mp[3] - 1], p2),
-             v62 = pvec(P, box, x[mp[5] - 1], p2);
-  const BpPara &bp = D.bpp[mp[6]];
-  T u;
-  V3<T> fb[6];
-  if (!bp_geom<T>(bp, v12, v13, v15, v42, v62, u, fb)) return 0;
-  double e = bp.U0 * dG * exp(-(double)u);
-  if (!(e <= P.bp_cutoff_energy)) return 0;   // also rejects a NaN energy
-  D.bp_status[gb] = 1;
-  D.ene_bp[gb] = e;
-  double *fo = D.for_bp + (size_t)gb * 18;
-  for (int q = 0; q < 6; q++) {
-    fo[3 * q] = e * (double)fb[q].x;
-    fo[3 * q + 1] = e * (double)fb[q].y;
-    fo[3 * q + 2] = e * (double)fb[q].z;
-  }
-  int *cnt = ntc ? ntc : D.nt_cnt + (size_t)r * N;   // ntc: this replica's counts in LDS
-  atomicAdd(&cnt[mp[0] - 1], 1);
-  atomicAdd(&cnt[mp[1] - 1], 1);
-  return 1;
-}
-
 template <typename T, int LPB, int B>
 __global__ void __launch_bounds__(B) k_persistent(Params P, Ptrs D, PersArgs A) {
   __shared__ double s1[B / LPB], s2[B / LPB];
@@ -109,14 +65,7 @@ __global__ void __launch_bounds__(B) k_persistent(Params P, Ptrs D, PersArgs A) 
     for (int gb = gtid; gb < A.nbp_total; gb += gthreads) {
       if (bp_eval_one<T>(P, D, gb, mc) && mc) {
         const int *mp = D.bp_mp + (size_t)gb * 8;
-        int a = mp[0] - 1, b = mp[1] - 1;
-        while (true) {
-          a = uf_find(D.comp, a);
-          b = uf_find(D.comp, b);
-          if (a == b) break;
-          if (a > b) { int t = a; a = b; b = t; }
-          if (atomicCAS(&D.comp[b], b, a) == b) break;
-        }
+        uf_join(D.comp, mp[0] - 1, mp[1] - 1);
       }
     }
     // bonded forces read only positions: computed here, added in phase D
@@ -772,14 +721,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
       const int *mpl = s_mpok ? s_mp + 8 * k : nullptr;
       if (bp_eval_one<T>(P, D, gb, mc, xr, mpl, st ? ntc : nullptr) && mc) {
         const int *mp = mpl ? mpl : D.bp_mp + (size_t)gb * 8;
-        int a = mp[0] - 1, b = mp[1] - 1;
-        while (true) {
-          a = uf_find(comp, a);
-          b = uf_find(comp, b);
-          if (a == b) break;
-          if (a > b) { int t = a; a = b; b = t; }
-          if (atomicCAS(&comp[b], b, a) == b) break;
-        }
+        uf_join(comp, mp[0] - 1, mp[1] - 1);
       }
     }
     if (!ovl)

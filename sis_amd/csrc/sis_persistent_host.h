@@ -603,7 +603,7 @@ void autotune(sis_gpu_ctx *c, const double *skins, int nskin, int64_t nsteps, do
   int mode = c->mode ? c->mode : choose_mode(c);
   const bool batched = mode == 3 && batched_ok(c);
   const bool pers = mode == 2 && c->R == 1 && !c->ext_on;
-  const bool phases = !batched && !pers && mode == 1 && graph_steps_ok(c);
+  const bool phases = !batched && !pers && mode == 1 && graph_steps_ok(c) && !(c->opt.flags & SIS_OPT_NO_GRAPH);
   if (!batched && !pers && !phases)
     throw ApiError{SIS_ERR_UNSUPPORTED, "the autotuner covers the batched, persistent and per-phase graph forms"};
   const int R = c->R, N = c->N;
