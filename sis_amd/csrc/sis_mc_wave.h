@@ -176,67 +176,21 @@ __device__ __forceinline__ int mc_pick(unsigned wh, double wu, int nact, int o) 
 // The Monte Carlo loop of mc_component_wave over its pair slots (IT chunks
 // of 64: endpoints ua, ub as nucleotide slots, energies en) and nucleotides
 // (ND chunks of 64: excess counts cnt).  live: the pairs left at the end.
-// Uniform arguments; all 64 lanes call it.
+// Uniform arguments; all 64 lanes call it.  Returns false on an
+// inconsistent state.
 //
-// One deletion is a chain of dependent scalar and lane operations, and its
-// latency is the kernel's time, so as little as possible stays on the
-// chain.  Most nucleotides of a large component have two pairs, and for
-// those every nucleotide's lane works out beforehand which of its two it
-// would delete with the draws to come: the two pairs (F, G: slot << 9 |
-// other nucleotide) and the Metropolis argument D = dE beta change only when
-// the nucleotide itself loses its third pair.  The chain is then: count of
-// active nucleotides, pick (mc_pick: a 32-bit multiply for an FP64 product,
-// ceiling and conversion), the lane of the picked bit, its answer, the
-// partner's count.  With wave_rank for the two sorts of the set-up (each
-// took a loop over all pairs) a step of 256 replicas of 128 nt went from
-// 85 to 75 us.
+// One deletion is a serial chain of scalar and lane operations on one
+// wavefront, which issues an instruction every four to eight cycles, so its
+// time is the number of instructions on it: live pairs are scalar masks,
+// nothing is worked out ahead (answers kept per nucleotide for the draws to
+// come took more instructions than they saved), the pick is mc_pick's
+// 32-bit multiply for an FP64 product, ceiling and conversion, and a
+// sequence of up to 8 pairs is packed in 64 bits.
 template <int IT, int ND>
-__device__ __forceinline__ bool mc_sweep(int max_bp, int rk, int root, int n, double beta, uint64_t seed, int64_t step,
-                                         int *ws, const int (&ua)[IT], const int (&ub)[IT], const double (&en)[IT],
-                                         const int (&cnt)[ND], unsigned long long (&live)[IT]) {
-  static_assert(ND <= 8, "excess counts are packed in bytes");
+__device__ __forceinline__ bool mc_sweep(int rk, int root, double beta, uint64_t seed, int64_t step, int *sseq,
+                                         const int (&ua)[IT], const int (&ub)[IT], const double (&en)[IT],
+                                         int (&cnt)[ND], unsigned long long (&live)[IT]) {
   const int L = lane_id();
-  const int c2 = 2 - max_bp;   // excess count of a nucleotide with two pairs
-  int *sseq = ws, *sfirst = ws + 64 + 128 * IT, *slast = sfirst + 64 * ND;
-  double *sen = reinterpret_cast<double *>(ws + 64);
-  // ---- first and last pair of every nucleotide
-#pragma unroll
-  for (int q = 0; q < ND; q++) {
-    sfirst[L + 64 * q] = 0x7fffffff;
-    slast[L + 64 * q] = -1;
-  }
-  wave_lds_fence();
-#pragma unroll
-  for (int k = 0; k < IT; k++) {
-    const int t = L + 64 * k;
-    live[k] = __ballot(t < n);
-    if (t < n) {
-      sen[t] = en[k];
-      atomicMin(&sfirst[ua[k]], t << 9 | ub[k]);
-      atomicMax(&slast[ua[k]], t << 9 | ub[k]);
-      atomicMin(&sfirst[ub[k]], t << 9 | ua[k]);
-      atomicMax(&slast[ub[k]], t << 9 | ua[k]);
-    }
-  }
-  wave_lds_fence();
-  int F[ND], G[ND];
-  double D[ND];
-  unsigned long long am[ND];   // active nucleotides (excess > 0)
-  unsigned c0 = 0, c1 = 0;     // their excess (at most 255), a byte for each chunk
-#pragma unroll
-  for (int q = 0; q < ND; q++) {
-    const unsigned e = cnt[q] > 0 ? (unsigned)cnt[q] << (8 * (q & 3)) : 0u;
-    if (q < 4) c0 |= e; else c1 |= e;
-    F[q] = G[q] = -1;
-    D[q] = 0.0;
-    am[q] = __ballot(cnt[q] > 0);
-    if (cnt[q] > 0 && cnt[q] == c2) {
-      F[q] = sfirst[L + 64 * q];
-      G[q] = slast[L + 64 * q];
-      D[q] = (sen[G[q] >> 9] - sen[F[q] >> 9]) * beta;
-    }
-  }
-  wave_lds_fence();
   // energy of pair slot `slot` (wave-uniform)
   auto ene_of = [&](int slot) {
     double x = en[0];
@@ -244,68 +198,26 @@ __device__ __forceinline__ bool mc_sweep(int max_bp, int rk, int root, int n, do
     for (int k = 1; k < IT; k++) x = (slot >> 6) == k ? en[k] : x;
     return bcast(x, slot & 63);
   };
-  // the other nucleotide of pair slot `slot` of nucleotide x
-  auto partner_of = [&](int slot, int x) {
-    int a = ua[0], b = ub[0];
-#pragma unroll
-    for (int k = 1; k < IT; k++) {
-      a = (slot >> 6) == k ? ua[k] : a;
-      b = (slot >> 6) == k ? ub[k] : b;
-    }
-    return bcast(a, slot & 63) + bcast(b, slot & 63) - x;
-  };
-  // nucleotide x loses a pair: no longer active, or down to its last two
-  // pairs, where its answer is worked out
-  auto lose_one = [&](int x) {
-    const int sh = 8 * ((x >> 6) & 3);
-    const bool hi = ND > 4 && x >= 256;
-    const int was = (bcast((int)(hi ? c1 : c0), x & 63) >> sh) & 255;
-    if (was == 0) return;
-    const unsigned one = L == (x & 63) ? 1u << sh : 0u;
-    if (hi) c1 -= one; else c0 -= one;
-    const int c = was - 1;
-    if (c == 0) {
-#pragma unroll
-      for (int q = 0; q < ND; q++)
-        if ((x >> 6) == q) am[q] &= ~(1ull << (x & 63));
-    } else if (c == c2) {
-      int la = -1, lb = -1;
-#pragma unroll
-      for (int k = 0; k < IT; k++) {
-        const unsigned long long m = (__ballot(ua[k] == x) | __ballot(ub[k] == x)) & live[k];
-        if (m) {
-          if (la < 0) la = 64 * k + __builtin_ctzll(m);
-          lb = 64 * k + 63 - __builtin_clzll(m);
-        }
-      }
-      if (la < 0) return;   // counts and pairs disagree: the pick finds it
-      const int f = la << 9 | partner_of(la, x), g = lb << 9 | partner_of(lb, x);
-      const double d = (ene_of(lb) - ene_of(la)) * beta;
-#pragma unroll
-      for (int q = 0; q < ND; q++) {
-        const bool me = L + 64 * q == x;
-        F[q] = me ? f : F[q];
-        G[q] = me ? g : G[q];
-        D[q] = me ? d : D[q];
-      }
-    }
-  };
-  // ---- draws: a window of 64 counters, lane i holding draw w0 + i, its
-  // logarithm (Metropolis test: log u < dE beta) and its upper 32 bits;
-  // g2: draws above one half (the swap target of a two-pair sequence)
   uint32_t draw = 0, w0 = (uint32_t)-64;
   double wu = 0.0, wl = 0.0;
   unsigned wh = 0;
   unsigned long long g2 = 0;
   for (;;) {
+    // active nucleotides (excess > 0) in ascending id order
+    unsigned long long am[ND];
     int pc[ND], nact = 0;
 #pragma unroll
     for (int q = 0; q < ND; q++) {
+      am[q] = __ballot(cnt[q] > 0);
       pc[q] = __popcll(am[q]);
       nact += pc[q];
     }
     if (nact == 0) return true;
-    if ((int)(draw - w0) > 64 - 16) {   // the window holds any sequence of up to eight pairs
+    // draws: a window of 64 counters, lane i holding draw w0 + i, its
+    // logarithm (Metropolis test: log u < dE beta) and its upper 32 bits;
+    // g2: draws above one half (the swap target of a two-pair sequence).
+    // It holds any sequence of up to eight pairs.
+    if ((int)(draw - w0) > 64 - 16) {
       w0 = draw;
       wu = philox_u(seed, rk, step, root, w0 + (uint32_t)L);
       wl = log(wu);
@@ -313,18 +225,6 @@ __device__ __forceinline__ bool mc_sweep(int max_bp, int rk, int root, int n, do
       g2 = __ballot(wu > 0.5);
     }
     const int o = (int)(draw - w0);
-    // what every nucleotide with two pairs would delete: the swap sweep
-    // leaves its pairs reversed exactly when both swap draws fall on the
-    // same side of one half; then one Metropolis test
-    const unsigned t2 = (unsigned)(g2 >> (o + 1)) & 3u;
-    const bool flip = t2 == 0u || t2 == 3u;
-    // in list order the first goes when w >= D; reversed, when D < -w: the
-    // same comparison with the double below -w (w < 0)
-    const long long wb = __double_as_longlong(bcast(wl, o + 3));
-    const double w = __longlong_as_double(flip ? (wb ^ (1ll << 63)) - 1 : wb);
-    int R[ND];
-#pragma unroll
-    for (int q = 0; q < ND; q++) R[q] = D[q] <= w ? F[q] : G[q];
     int want = mc_pick(wh, wu, nact, o);
     unsigned long long amq = am[0];
     int base = 0;
@@ -335,102 +235,114 @@ __device__ __forceinline__ bool mc_sweep(int max_bp, int rk, int root, int n, do
       amq = next ? am[q] : amq;
       base = next ? 64 * q : base;
     }
-    int Rq = R[0];
+    const int ntd = base + __builtin_ctzll(__ballot(below(amq) == want) & amq);
+    // its pairs in list order
+    unsigned long long sm[IT];
+    int ns = 0;
 #pragma unroll
-    for (int q = 1; q < ND; q++) Rq = base == 64 * q ? R[q] : Rq;
-    const int ln = __builtin_ctzll(__ballot(below(amq) == want) & amq);
-    const int ntd = base + ln;
-    int got = bcast(Rq, ln);
-    int ns = 2;
-    if (got < 0) {
-      // three pairs or more: ntd's pairs in list order
-      unsigned long long sm[IT];
-      ns = 0;
-#pragma unroll
-      for (int k = 0; k < IT; k++) {
-        sm[k] = (__ballot(ua[k] == ntd) | __ballot(ub[k] == ntd)) & live[k];
-        ns += __popcll(sm[k]);
-      }
-      if (ns == 0) return false;
-      if (ns > 64) ns = 64;
-      // draws used: 1 (pick) + ns (shuffle) + ns - 1 (Metropolis) = 2 ns
-      int del;
-      if (ns <= 8) {
-        // short sequence: kept in scalar registers, entry m in bits
-        // 8m..8m+7 (slots < 256)
-        uint64_t sp = 0;
-        int m = 0;
-#pragma unroll
-        for (int k = 0; k < IT; k++)
-          for (unsigned long long mk = sm[k]; mk; mk &= mk - 1) {
-            sp |= (uint64_t)(64 * k + __builtin_ctzll(mk)) << (8 * m);
-            m++;
-          }
-        const int swv = 8 * ((int)ceil(wu * ns) - 1);
-        // reference shuffle: for i = 1..n swap(i, ceil(rnd*n))
-        for (int i = 0; i < 8 * ns; i += 8) {
-          const int sw = bcast(swv, o + 1 + (i >> 3));
-          const uint64_t x = ((sp >> i) ^ (sp >> sw)) & 0xffull;   // swap entries i and sw
-          sp ^= (x << i) | (x << sw);
-        }
-        // Metropolis sweep on the energies of the sequence's pairs
-        del = (int)(sp & 0xffull);
-        double edel = ene_of(del);
-        for (int i = 1; i < ns; i++) {
-          const int si = (int)((sp >> (8 * i)) & 0xffull);
-          const double ej = ene_of(si);
-          if (bcast(wl, o + ns + i) < (ej - edel) * beta) { del = si; edel = ej; }
-        }
-      } else {
-        // long sequence: entry m in lane m (through LDS)
-#pragma unroll
-        for (int k = 0, m0 = 0; k < IT; k++) {
-          const int m = m0 + below(sm[k]);
-          if (((sm[k] >> L) & 1ull) && m < 64) sseq[m] = 64 * k + L;
-          m0 += __popcll(sm[k]);
-        }
-        wave_lds_fence();
-        int seqv = L < ns ? sseq[L] : 0;
-        // lane i: the i-th swap target, and the logarithm of the draw that
-        // decides on entry i
-        const double us = philox_u(seed, rk, step, root, draw + 1u + (uint32_t)L);
-        const double ul = log(philox_u(seed, rk, step, root, draw + (uint32_t)(ns + L)));
-        const int swl = (int)ceil(us * ns) - 1;
-        for (int i = 0; i < ns; i++) {
-          const int sw = bcast(swl, i);
-          const int ti = bcast(seqv, i), ts = bcast(seqv, sw);
-          seqv = setlane(seqv, ts, i);
-          seqv = setlane(seqv, ti, sw);
-        }
-        del = bcast(seqv, 0);
-        double edel = ene_of(del);
-        for (int i = 1; i < ns; i++) {
-          const int si = bcast(seqv, i);
-          const double ej = ene_of(si);
-          if (bcast(ul, i) < (ej - edel) * beta) { del = si; edel = ej; }
-        }
-        wave_lds_fence();
-      }
-      got = del << 9 | partner_of(del, ntd);
+    for (int k = 0; k < IT; k++) {
+      sm[k] = (__ballot(ua[k] == ntd) | __ballot(ub[k] == ntd)) & live[k];
+      ns += __popcll(sm[k]);
     }
-    draw += 2u * (uint32_t)ns;
-    const int del = got >> 9, other = got & 511;
+    if (ns == 0) return false;
+    if (ns > 64) ns = 64;
+    int del;
+    if (ns == 2) {
+      // two pairs: the swap sweep leaves them reversed exactly when both
+      // swap draws fall on the same side of one half
+      int la = -1, lb = -1;
 #pragma unroll
-    for (int k = 0; k < IT; k++)
-      if ((del >> 6) == k) live[k] &= ~(1ull << (del & 63));
-    lose_one(ntd);
-    lose_one(other);
+      for (int k = IT - 1; k >= 0; k--)
+        if (sm[k]) la = 64 * k + __builtin_ctzll(sm[k]);
+#pragma unroll
+      for (int k = 0; k < IT; k++)
+        if (sm[k]) lb = 64 * k + 63 - __builtin_clzll(sm[k]);
+      const unsigned t = (unsigned)(g2 >> (o + 1)) & 3u;
+      const bool flip = t == 0u || t == 3u;
+      const int s0 = flip ? lb : la, s1 = flip ? la : lb;
+      const double e0 = ene_of(s0), w = bcast(wl, o + 3);
+      double ev = en[0];
+#pragma unroll
+      for (int k = 1; k < IT; k++) ev = (s1 >> 6) == k ? en[k] : ev;
+      const bool acc = (__ballot(w < (ev - e0) * beta) >> (s1 & 63)) & 1ull;
+      del = acc ? s1 : s0;
+    } else if (ns <= 8) {
+      // short sequence: kept in scalar registers, entry m in bits
+      // 8m..8m+7 (slots < 256)
+      uint64_t sp = 0;
+      int m = 0;
+#pragma unroll
+      for (int k = 0; k < IT; k++)
+        for (unsigned long long mk = sm[k]; mk; mk &= mk - 1) {
+          sp |= (uint64_t)(64 * k + __builtin_ctzll(mk)) << m;
+          m += 8;
+        }
+      const int swv = 8 * ((int)ceil(wu * ns) - 1);
+      // reference shuffle: for i = 1..n swap(i, ceil(rnd*n))
+      for (int i = 0; i < 8 * ns; i += 8) {
+        const int sw = bcast(swv, o + 1 + (i >> 3));
+        const uint64_t x = ((sp >> i) ^ (sp >> sw)) & 0xffull;   // swap entries i and sw
+        sp ^= (x << i) | (x << sw);
+      }
+      // Metropolis sweep on the energies of the sequence's pairs
+      del = (int)(sp & 0xffull);
+      double edel = ene_of(del);
+      for (int i = 1; i < ns; i++) {
+        const int si = (int)((sp >> (8 * i)) & 0xffull);
+        const double ej = ene_of(si);
+        if (bcast(wl, o + ns + i) < (ej - edel) * beta) { del = si; edel = ej; }
+      }
+    } else {
+      // long sequence: entry m in lane m (through LDS)
+#pragma unroll
+      for (int k = 0, m0 = 0; k < IT; k++) {
+        const int m = m0 + below(sm[k]);
+        if (((sm[k] >> L) & 1ull) && m < 64) sseq[m] = 64 * k + L;
+        m0 += __popcll(sm[k]);
+      }
+      wave_lds_fence();
+      int seqv = L < ns ? sseq[L] : 0;
+      // lane i: the i-th swap target, and the logarithm of the draw that
+      // decides on entry i
+      const double us = philox_u(seed, rk, step, root, draw + 1u + (uint32_t)L);
+      const double ul = log(philox_u(seed, rk, step, root, draw + (uint32_t)(ns + L)));
+      const int swl = (int)ceil(us * ns) - 1;
+      for (int i = 0; i < ns; i++) {
+        const int sw = bcast(swl, i);
+        const int ti = bcast(seqv, i), ts = bcast(seqv, sw);
+        seqv = setlane(seqv, ts, i);
+        seqv = setlane(seqv, ti, sw);
+      }
+      del = bcast(seqv, 0);
+      double edel = ene_of(del);
+      for (int i = 1; i < ns; i++) {
+        const int si = bcast(seqv, i);
+        const double ej = ene_of(si);
+        if (bcast(ul, i) < (ej - edel) * beta) { del = si; edel = ej; }
+      }
+      wave_lds_fence();
+    }
+    // draws used: 1 (pick) + ns (shuffle) + ns - 1 (Metropolis) = 2 ns
+    draw += 2u * (uint32_t)ns;
+    int a = ua[0], b = ub[0];
+#pragma unroll
+    for (int k = 1; k < IT; k++) {
+      a = (del >> 6) == k ? ua[k] : a;
+      b = (del >> 6) == k ? ub[k] : b;
+    }
+    const int da = bcast(a, del & 63), db = bcast(b, del & 63);
+#pragma unroll
+    for (int k = 0; k < IT; k++) live[k] &= (del >> 6) == k ? ~(1ull << (del & 63)) : ~0ull;
+#pragma unroll
+    for (int q = 0; q < ND; q++) cnt[q] -= (L + 64 * q == da) + (L + 64 * q == db);
   }
 }
 
 // The same loop for components of at most 64 pairs and 128 nucleotides, one
 // pair and two nucleotides a lane: the live pairs are one 64-bit mask, and
-// a sequence of up to 8 pairs a 4-bit permutation of their ranks.  These
-// components are short and dense (three pairs a nucleotide and more), where
-// a deletion's time is the number of instructions on it, so nothing is
-// worked out ahead: 1,250 cycles a deletion (34 deletions of a 40-pair
-// component in 42,000) against 2,000 for the loop above and 1,700 with the
-// FP64 pick.  Its loops stay rolled: unrolled ones gained 5% on such a
+// a sequence of up to 8 pairs a 4-bit permutation of their ranks.  1,250
+// cycles a deletion (34 deletions of a 40-pair component in 42,000), 1,700
+// with the FP64 pick and 2,000 with answers worked out ahead.  Its loops stay rolled: unrolled ones gained 5% on such a
 // component and lost 30% on one of five pairs, to instruction fetch.
 // Returns false if a nucleotide has more than 8 formed
 // pairs or the state is inconsistent (the caller then runs the general loop
@@ -601,15 +513,22 @@ __device__ __forceinline__ bool mc_component_wave(const Params &P, const Ptrs &D
     ub[k] = ok[k] ? u2[2 * k + 1] : -1;
   }
   unsigned long long live[IT];
-  // two nucleotide chunks do for nearly all components of up to 128 pairs
+#pragma unroll
+  for (int k = 0; k < IT; k++) live[k] = __ballot(ok[k]);
+  // half the nucleotide chunks do for nearly all components
   bool done = false;
-  if constexpr (IT == 1) done = mc_sweep64(rk, root, n, beta, seed, step, ua[0], ub[0], en[0], cnt[0], cnt[1], live[0]);
+  if constexpr (IT == 1) {
+    done = mc_sweep64(rk, root, n, beta, seed, step, ua[0], ub[0], en[0], cnt[0], cnt[1], live[0]);
+    live[0] = done ? live[0] : __ballot(ok[0]);
+  }
   if (done) {
-  } else if (ND == 4 && nn <= 128) {
-    const int c[2] = {cnt[0], cnt[1]};
-    done = mc_sweep<IT, 2>(P.max_bp_per_nt, rk, root, n, beta, seed, step, ws, ua, ub, en, c, live);
+  } else if (IT > 1 && nn <= 32 * ND) {
+    int c[ND / 2];
+#pragma unroll
+    for (int q = 0; q < ND / 2; q++) c[q] = cnt[q];
+    done = mc_sweep<IT, ND / 2>(rk, root, beta, seed, step, ws, ua, ub, en, c, live);
   } else {
-    done = mc_sweep<IT, ND>(P.max_bp_per_nt, rk, root, n, beta, seed, step, ws, ua, ub, en, cnt, live);
+    done = mc_sweep<IT, ND>(rk, root, beta, seed, step, ws, ua, ub, en, cnt, live);
   }
   if (!done) return false;
   // write back the pairs deleted here
