@@ -313,23 +313,27 @@ __device__ __forceinline__ V3<double> dih_force_p(const Params &P, const V3<doub
   return (-a) * fi + (-1.0 + b) * fl;
 }
 
+// Pair forces take no branch: beyond the cutoff, and for a pair that is not
+// there (on = false), the factor of v12 is zero.  A wavefront works several
+// pairs at a time through these dependent chains (divide, square root,
+// exponential), and a branch around each would run them one by one.
+//
 // WCA (src/force_wca.F90:51-58): force on bead 1 of v12 = x1 - x2.
 template <typename T>
-__device__ __forceinline__ V3<T> wca_force(const Params &P, const V3<T> &v12) {
+__device__ __forceinline__ V3<T> wca_force(const Params &P, const V3<T> &v12, bool on) {
   T d2 = dot(v12, v12);
-  if (d2 >= (T)P.wca_sig2) return V3<T>{0, 0, 0};
   // FP32: hardware reciprocal (1 ulp) instead of the correctly rounded divide
   T s;
   if constexpr (sizeof(T) == 4) s = (T)P.wca_sig2 * __builtin_amdgcn_rcpf(d2);
   else s = (T)P.wca_sig2 / d2;
   T s2 = s * s, s4 = s2 * s2, s7 = s4 * s2 * s;
-  return ((T)P.wca_coef * (s7 - s4)) * v12;
+  const T f = (T)P.wca_coef * (s7 - s4);
+  return (!on || d2 >= (T)P.wca_sig2 ? (T)0 : f) * v12;
 }
 // Debye-Hueckel (src/force_ele_DH.F90:57-68): force on bead 1 of v12.
 template <typename T>
-__device__ __forceinline__ V3<T> dh_force(T coef, T rc2, T rlam, const V3<T> &v12) {
+__device__ __forceinline__ V3<T> dh_force(T coef, T rc2, T rlam, const V3<T> &v12, bool on) {
   T d2 = dot(v12, v12);
-  if (d2 > rc2) return V3<T>{0, 0, 0};
   // FP32: hardware reciprocal square root (1 ulp) gives 1/d and d = d2/d
   T d1, r1;
   if constexpr (sizeof(T) == 4) {
@@ -340,7 +344,7 @@ __device__ __forceinline__ V3<T> dh_force(T coef, T rc2, T rlam, const V3<T> &v1
     r1 = (T)1 / d1;
   }
   T dv = coef * r1 * r1 * (r1 + rlam) * m_exp(-d1 * rlam);
-  return dv * v12;
+  return (!on || d2 > rc2 ? (T)0 : dv) * v12;
 }
 
 // One BP angle term for the angle between a (= v12) and b, with

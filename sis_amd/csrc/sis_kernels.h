@@ -1095,6 +1095,7 @@ __device__ __forceinline__ V3<double> bonded_part(const Params &P, const Ptrs &D
 // Pair forces on bead a, lane l of LPB: WCA and Debye-Hueckel neighbours
 // (pair_nb), then the formed base pairs it takes part in (pair_bp), both
 // accumulated onto F in that order.  pair_part is the two in sequence.
+constexpr int PAIR_U = 4;   // neighbours a lane works on at a time
 template <typename T>
 __device__ __forceinline__ V3<double> pair_nb(const Params &P, const Ptrs &D, int r, int a, int l, int LPB,
                                               const double4 *xr, V3<double> F) {
@@ -1106,38 +1107,42 @@ __device__ __forceinline__ V3<double> pair_nb(const Params &P, const Ptrs &D, in
   const int nw = min(D.n_wca[g], D.maxw);
   const int ne = P.ele_on ? min(D.n_ele[g], D.maxnb) : 0;
   const T coef = (T)D.ele_coef[r], rc2 = (T)(D.ele_cut[r] * D.ele_cut[r]), rl = (T)(1.0 / D.lambdaD[r]);
-  // neighbours in batches of PU: their index and position loads are all
-  // issued before the arithmetic; the summation order is unchanged
-  constexpr int PU = 4;
+  // neighbours in batches of PAIR_U: their index and position loads are all
+  // issued before the arithmetic, and the arithmetic of a batch is
+  // independent up to the sums; the summation order is unchanged
   const int *nbw = D.nb_wca + (size_t)r * D.maxw * N + a;
-  for (int k0 = l; k0 < nw; k0 += PU * LPB) {
-    int id[PU];
-    double4 pb[PU];
+  for (int k0 = l; k0 < nw; k0 += PAIR_U * LPB) {
+    int id[PAIR_U];
+    double4 pb[PAIR_U];
+    V3<T> f[PAIR_U];
 #pragma unroll
-    for (int u = 0; u < PU; u++) {
+    for (int u = 0; u < PAIR_U; u++) {
       const int k = k0 + u * LPB;
       id[u] = k < nw ? nbw[(size_t)k * N] : -1;
     }
 #pragma unroll
-    for (int u = 0; u < PU; u++) pb[u] = x[id[u] >= 0 ? id[u] : a];
+    for (int u = 0; u < PAIR_U; u++) pb[u] = x[id[u] >= 0 ? id[u] : a];
 #pragma unroll
-    for (int u = 0; u < PU; u++)
-      if (id[u] >= 0) F = F + cvt<double>(wca_force<T>(P, cvt<T>(pvec(P, box, pa, pb[u]))));
+    for (int u = 0; u < PAIR_U; u++) f[u] = wca_force<T>(P, cvt<T>(pvec(P, box, pa, pb[u])), id[u] >= 0);
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
   }
   const int *nbe = D.nb_ele + (size_t)r * D.maxnb * N + a;
-  for (int k0 = l; k0 < ne; k0 += PU * LPB) {
-    int id[PU];
-    double4 pb[PU];
+  for (int k0 = l; k0 < ne; k0 += PAIR_U * LPB) {
+    int id[PAIR_U];
+    double4 pb[PAIR_U];
+    V3<T> f[PAIR_U];
 #pragma unroll
-    for (int u = 0; u < PU; u++) {
+    for (int u = 0; u < PAIR_U; u++) {
       const int k = k0 + u * LPB;
       id[u] = k < ne ? nbe[(size_t)k * N] : -1;
     }
 #pragma unroll
-    for (int u = 0; u < PU; u++) pb[u] = x[id[u] >= 0 ? id[u] : a];
+    for (int u = 0; u < PAIR_U; u++) pb[u] = x[id[u] >= 0 ? id[u] : a];
 #pragma unroll
-    for (int u = 0; u < PU; u++)
-      if (id[u] >= 0) F = F + cvt<double>(dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, pb[u]))));
+    for (int u = 0; u < PAIR_U; u++) f[u] = dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, pb[u])), id[u] >= 0);
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
   }
   return F;
 }

@@ -525,9 +525,27 @@ __device__ __forceinline__ V3<double> pair_nb_lds(const Params &P, const Ptrs &D
   const int nw = cnt >> 16, ne = P.ele_on ? (cnt & 0xffff) : 0;
   const T coef = (T)D.ele_coef[r], rc2 = (T)(D.ele_cut[r] * D.ele_cut[r]), rl = (T)(1.0 / D.lambdaD[r]);
   V3<double> F{0.0, 0.0, 0.0};
-  for (int k = l; k < nw; k += LPB) F = F + cvt<double>(wca_force<T>(P, cvt<T>(pvec(P, box, pa, x[s_nb[off + k]]))));
+  for (int k0 = l; k0 < nw; k0 += PAIR_U * LPB) {
+    V3<T> f[PAIR_U];
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) {
+      const int k = k0 + u * LPB;
+      f[u] = wca_force<T>(P, cvt<T>(pvec(P, box, pa, x[k < nw ? s_nb[off + k] : a])), k < nw);
+    }
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+  }
   const int *e = s_nb + off + nw;
-  for (int k = l; k < ne; k += LPB) F = F + cvt<double>(dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, x[e[k]]))));
+  for (int k0 = l; k0 < ne; k0 += PAIR_U * LPB) {
+    V3<T> f[PAIR_U];
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) {
+      const int k = k0 + u * LPB;
+      f[u] = dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, x[k < ne ? e[k] : a])), k < ne);
+    }
+#pragma unroll
+    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+  }
   return F;
 }
 
