@@ -197,7 +197,7 @@ struct sis_gpu_ctx {
       n_bp_d, inc_d, n_inc_d, nt_cnt_d, comp_d, flags_d;
   DevBuf<double> bp_coef_d, ene_bp_d, for_bp_d;
   DevBuf<uint8_t> bp_status_d, bp_status_mc_d, bp_status_keep_d;
-  DevBuf<int> cell_of_d, cell_cnt_d, cell_start_d, cell_beads_d, cell_fill_d;
+  DevBuf<int> cell_of_d, cell_cnt_d, cell_start_d, cell_beads_d, cell_unsorted_d, cell_fill_d;
   DevBuf<double> blk_top2_d;
   DevBuf<int> rebuild_flag_d, mask_d, mc_d, scan_bsum_d, scan_total_d;
   DevBuf<int> exc_cnt_d, exc_off_d, exc_fill_d, exc_list_d, ntlist_d, bpseq_d, seg_d;
@@ -283,7 +283,7 @@ struct sis_gpu_ctx {
     DevBuf<int> *ib[] = {&bp3_hash_d, &nb_ele_d, &n_ele_d, &nb_wca_d, &n_wca_d, &bp_tmp_d,
                          &n_bp_tmp_d, &bp_off_d, &bp_mp_d, &n_bp_d, &inc_d, &n_inc_d, &nt_cnt_d,
                          &comp_d, &flags_d, &cell_of_d, &cell_cnt_d, &cell_start_d,
-                         &cell_beads_d, &cell_fill_d, &rebuild_flag_d, &mask_d, &mc_d,
+                         &cell_beads_d, &cell_unsorted_d, &cell_fill_d, &rebuild_flag_d, &mask_d, &mc_d,
                          &scan_bsum_d, &scan_total_d, &exc_cnt_d, &exc_off_d, &exc_fill_d,
                          &exc_list_d, &ntlist_d, &bpseq_d, &seg_d, &huge_d, &pers_sync_d, &chain_id_d,
                          &bp_val_d, &bp_val2_d, &bp_mp2_d};
@@ -459,7 +459,7 @@ void scan_exclusive(sis_gpu_ctx *c, const int *in, int *out, int64_t n, int *tot
   int64_t nb = (n + B - 1) / B;
   if ((int64_t)c->scan_bsum_d.n < nb + 1) c->scan_bsum_d.alloc(nb + 1);
   hipLaunchKernelGGL(k_scan_blocks<B>, dim3(nb), dim3(B), 0, c->stream, in, out, c->scan_bsum_d.p, n);
-  hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(1), 0, c->stream, c->scan_bsum_d.p, (int)nb,
+  hipLaunchKernelGGL(k_scan_bsum<256>, dim3(1), dim3(256), 0, c->stream, c->scan_bsum_d.p, (int)nb,
                      c->scan_total_d.p, out + n);
   hipLaunchKernelGGL(k_scan_add<B>, dim3(nb), dim3(B), 0, c->stream, out, c->scan_bsum_d.p, n);
   (void)total_dev;
@@ -514,6 +514,7 @@ void setup_cells(sis_gpu_ctx *c) {
   c->cell_start_d.alloc(RC + 1);
   c->cell_fill_d.alloc(RC);
   c->cell_beads_d.alloc((size_t)c->R * c->N);
+  c->cell_unsorted_d.alloc((size_t)c->R * c->N);
 }
 
 // Per-replica conditions: set_ele and set_md_coef (src/job_md.F90:700-767).
@@ -592,7 +593,6 @@ void rebuild(sis_gpu_ctx *c, const std::vector<int> &mask_in) {
   const std::vector<int64_t> old_off = c->bp_rep_off;
   set_mask(c, mask);
   for (int attempt = 0; attempt < 8; attempt++) {
-    HIPCHK(hipMemsetAsync(c->flags_d.p, 0, 8 * sizeof(int), c->stream));
     Ptrs D = c->ptrs();
     hipLaunchKernelGGL(k_wrap, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->mask_d.p);
     if (c->use_cells) {
@@ -601,40 +601,49 @@ void rebuild(sis_gpu_ctx *c, const std::vector<int> &mask_in) {
       HIPCHK(hipMemsetAsync(c->cell_fill_d.p, 0, RC * sizeof(int), c->stream));
       hipLaunchKernelGGL(k_cell_count, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->mask_d.p);
       scan_exclusive(c, c->cell_cnt_d.p, c->cell_start_d.p, (int64_t)RC, nullptr);
-      hipLaunchKernelGGL(k_cell_fill, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->mask_d.p,
+      Ptrs Df = D;
+      Df.cell_beads = c->cell_unsorted_d.p;
+      hipLaunchKernelGGL(k_cell_fill, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, Df, c->mask_d.p,
                          c->cell_fill_d.p);
-      hipLaunchKernelGGL(k_cell_sort, dim3((RC + B - 1) / B), dim3(B), 0, c->stream, c->P, D, c->mask_d.p);
-      hipLaunchKernelGGL(k_search_cell, grid_beads(N, R, 128), dim3(128), 0, c->stream, c->P, D, c->mask_d.p);
-    } else {
-      hipLaunchKernelGGL(k_search_brute<128>, grid_beads(N, R, 128), dim3(128), 0, c->stream, c->P, D,
-                         c->mask_d.p);
+      hipLaunchKernelGGL(k_cell_sort, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, c->mask_d.p,
+                         c->cell_unsorted_d.p);
     }
+    const dim3 gs((unsigned)(((size_t)R * N + SEARCH_WAVES - 1) / SEARCH_WAVES)), bs(64 * SEARCH_WAVES);
+    if (c->use_cells) hipLaunchKernelGGL(k_search_cell, gs, bs, 0, c->stream, c->P, D, c->mask_d.p);
+    else hipLaunchKernelGGL(k_search_brute, gs, bs, 0, c->stream, c->P, D, c->mask_d.p);
     // BP candidate list in reference order over all replicas
     scan_exclusive(c, c->n_bp_tmp_d.p, c->bp_off_d.p, (int64_t)R * N, nullptr);
-    HIPCHK(hipMemsetAsync(c->n_inc_d.p, 0, (size_t)R * N * sizeof(int), c->stream));
     hipLaunchKernelGGL(k_bp_fill, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, nullptr);
     int hflags[8];
     int total = 0;
+    // candidates into the reference's list order, then their incidences.
+    // They come ordered by (replica, i, j), which is that order already for
+    // one chain and for the analysis lists: no sort, and no round trip for
+    // its length (the incidences launch over the capacity)
+    const bool ordered = c->P.nchains == 1 || c->P.list_rule != 0;
     HIPCHK(hipMemcpyAsync(&total, c->bp_off_d.p + (size_t)R * N, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(hipStreamSynchronize(c->stream));
-    if (total > 0 && total <= c->D.maxbp) {
-      // candidates into the reference's list order, then their incidences
-      size_t tb = 0;
-      HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, c->bp_key_d.p, c->bp_key2_d.p, c->bp_val_d.p,
-                                                c->bp_val2_d.p, total, 0, 64, c->stream));
-      if (c->sort_tmp_d.n < tb) c->sort_tmp_d.alloc(tb);
-      HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp_d.p, tb, c->bp_key_d.p, c->bp_key2_d.p, c->bp_val_d.p,
-                                                c->bp_val2_d.p, total, 0, 64, c->stream));
-      hipLaunchKernelGGL(k_bp_permute, dim3((total + B - 1) / B), dim3(B), 0, c->stream, D, total, c->bp_val2_d.p,
-                         c->bp_mp2_d.p, c->bp_coef2_d.p);
-      // back into the same buffers: captured step graphs keep their pointers
-      HIPCHK(hipMemcpyAsync(c->bp_mp_d.p, c->bp_mp2_d.p, (size_t)total * 8 * sizeof(int), hipMemcpyDeviceToDevice,
-                            c->stream));
-      HIPCHK(hipMemcpyAsync(c->bp_coef_d.p, c->bp_coef2_d.p, (size_t)total * 2 * sizeof(double),
-                            hipMemcpyDeviceToDevice, c->stream));
-      hipLaunchKernelGGL(k_bp_inc, dim3((total + B - 1) / B), dim3(B), 0, c->stream, c->P, D, total);
+    if (ordered) {
+      hipLaunchKernelGGL(k_bp_inc, dim3((c->D.maxbp + B - 1) / B), dim3(B), 0, c->stream, c->P, D, -1);
+    } else {
+      HIPCHK(hipStreamSynchronize(c->stream));
+      if (total > 0 && total <= c->D.maxbp) {
+        size_t tb = 0;
+        HIPCHK(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, c->bp_key_d.p, c->bp_key2_d.p, c->bp_val_d.p,
+                                                  c->bp_val2_d.p, total, 0, 64, c->stream));
+        if (c->sort_tmp_d.n < tb) c->sort_tmp_d.alloc(tb);
+        HIPCHK(hipcub::DeviceRadixSort::SortPairs(c->sort_tmp_d.p, tb, c->bp_key_d.p, c->bp_key2_d.p, c->bp_val_d.p,
+                                                  c->bp_val2_d.p, total, 0, 64, c->stream));
+        hipLaunchKernelGGL(k_bp_permute, dim3((total + B - 1) / B), dim3(B), 0, c->stream, D, total, c->bp_val2_d.p,
+                           c->bp_mp2_d.p, c->bp_coef2_d.p);
+        // back into the same buffers: captured step graphs keep their pointers
+        HIPCHK(hipMemcpyAsync(c->bp_mp_d.p, c->bp_mp2_d.p, (size_t)total * 8 * sizeof(int), hipMemcpyDeviceToDevice,
+                              c->stream));
+        HIPCHK(hipMemcpyAsync(c->bp_coef_d.p, c->bp_coef2_d.p, (size_t)total * 2 * sizeof(double),
+                              hipMemcpyDeviceToDevice, c->stream));
+        hipLaunchKernelGGL(k_bp_inc, dim3((total + B - 1) / B), dim3(B), 0, c->stream, c->P, D, total);
+      }
     }
-    hipLaunchKernelGGL(k_inc_sort, grid_beads(N, R, B), dim3(B), 0, c->stream, c->P, D, nullptr);
+    hipLaunchKernelGGL(k_inc_sort, grid_beads(N, R, 64), dim3(64), 0, c->stream, c->P, D, nullptr);
     HIPCHK(hipMemcpyAsync(hflags, c->flags_d.p, sizeof hflags, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
     bool grow = false;
@@ -827,7 +836,7 @@ void energy_phase(sis_gpu_ctx *c, const std::vector<int> &mask, const std::vecto
   }
   dim3 g = grid_beads(N, R, B);
   if ((int64_t)c->ene_part_d.n < (int64_t)R * g.x * 8) c->ene_part_d.alloc((size_t)R * g.x * 8);
-  hipLaunchKernelGGL(k_energy<B>, g, dim3(B), 0, c->stream, c->P, c->ptrs(), c->ecT_d.p, c->eCoef_d.p,
+  hipLaunchKernelGGL(k_energy<B>, g, dim3(B * ENE_LPB), 0, c->stream, c->P, c->ptrs(), c->ecT_d.p, c->eCoef_d.p,
                      c->eLam_d.p, c->ene_part_d.p, c->mask_d.p, flags & 1, -1, 0.0, 0.0);
   const double *ext = nullptr;
   if (c->ext_on) {
@@ -854,8 +863,7 @@ void energy_phase(sis_gpu_ctx *c, const std::vector<int> &mask, const std::vecto
   hipLaunchKernelGGL(k_energy_reduce, dim3(R), dim3(1), 0, c->stream, c->ene_part_d.p, (int)g.x, c->ene_out_d.p,
                      ext, -1);
   HIPCHK(hipMemcpyAsync(out, c->ene_out_d.p, (size_t)R * 16 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(hipStreamSynchronize(c->stream));
-  check_flags(c);
+  check_flags(c);   // waits for both copies
   if (c->ext_on && c->X.stage) {
     int err = 0;
     HIPCHK(hipMemcpy(&err, c->x_err_d.p, sizeof err, hipMemcpyDeviceToHost));
@@ -1826,7 +1834,7 @@ int sis_gpu_energy_noalloc(sis_gpu_ctx *c, int32_t irep, double tempK, int32_t f
                            c->nbp_total, mc, ecT, mask, 0);
     }
   }
-  hipLaunchKernelGGL(k_energy<B>, dim3(nblk, 1), dim3(B), 0, c->stream, c->P, D, ecT, nullptr, nullptr, partial,
+  hipLaunchKernelGGL(k_energy<B>, dim3(nblk, 1), dim3(B * ENE_LPB), 0, c->stream, c->P, D, ecT, nullptr, nullptr, partial,
                      mask, 0, r0, coef, lam);
   const double *ext = nullptr;
   if (c->ext_on) {   // external terms into their own buffer (made by sis_gpu_set_external)
