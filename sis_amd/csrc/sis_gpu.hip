@@ -59,7 +59,7 @@ struct DevBuf {
       HIPCHK(hipFree(p));
     }
     p = nullptr;
-    n = count;
+    n = 0;   // a failed allocation leaves an empty buffer
     if (count) {
       // the engine works on a non-blocking stream: finish the zero fill
       // before any kernel can touch the new buffer
@@ -68,6 +68,7 @@ struct DevBuf {
       HIPCHK(hipMemset(p, 0, count * sizeof(T)));
       HIPCHK(hipDeviceSynchronize());
     }
+    n = count;
   }
   void free_() {
     if (p) (void)hipFree(p);
@@ -229,6 +230,7 @@ struct sis_gpu_ctx {
   DevBuf<int> g_int_d;
   DevBuf<double4> step_fpair_d, step_noise_d;
   DevBuf<double> step_top2_d;
+  DevBuf<double> state3_d;      // (3, nmp, nrep) on its way between host and device
   bool circular = false;        // some chain is circular
   bool step_sep_huge = false;   // a component above the bucket capacity was met
   // device exchange of the batched form (sis_exchange.h)
@@ -334,6 +336,7 @@ struct sis_gpu_ctx {
     step_fpair_d.free_();
     step_noise_d.free_();
     step_top2_d.free_();
+    state3_d.free_();
     for (auto e : tev) (void)hipEventDestroy(e);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -1567,7 +1570,7 @@ int sis_gpu_create(const sis_topo *topo, const sis_params *prm, const sis_option
     c->bpp_d.alloc(7);
     HIPCHK(hipMemcpy(c->bpp_d.p, c->bpp_h, sizeof c->bpp_h, hipMemcpyHostToDevice));
     c->ecT_d.alloc(R); c->eCoef_d.alloc(R); c->eLam_d.alloc(R);
-    c->pos_d.alloc(RN); c->pos2_d.alloc(RN); c->fbond_d.alloc(RN); c->vel_d.alloc(RN); c->acc_d.alloc(RN); c->move_d.alloc(RN); c->frc_d.alloc(RN);
+    c->pos_d.alloc(RN); c->pos2_d.alloc(RN); c->fbond_d.alloc(RN); c->vel_d.alloc(RN); c->acc_d.alloc(RN); c->move_d.alloc(RN); c->frc_d.alloc(RN); c->state3_d.alloc(3 * RN);
     c->n_ele_d.alloc(RN); c->n_wca_d.alloc(RN); c->n_bp_tmp_d.alloc(RN); c->bp_off_d.alloc(RN + 1);
     c->n_bp_d.alloc(R); c->n_inc_d.alloc(RN); c->nt_cnt_d.alloc(RN); c->comp_d.alloc(RN);
     c->flags_d.alloc(8);
@@ -1617,11 +1620,11 @@ int sis_gpu_destroy(sis_gpu_ctx *c) {
 int sis_gpu_set_state(sis_gpu_ctx *c, const double *xyz, const double *velos, const double *accels) {
   API_BEGIN
   if (!c) return fail(SIS_ERR_ARG, "null context");
-  size_t RN = (size_t)c->R * c->N;
-  std::vector<double4> h(RN);
+  const size_t RN = (size_t)c->R * c->N;
   auto up = [&](const double *src, DevBuf<double4> &dst) {
-    for (size_t g = 0; g < RN; g++) h[g] = double4{src[3 * g], src[3 * g + 1], src[3 * g + 2], 0.0};
-    HIPCHK(hipMemcpy(dst.p, h.data(), RN * sizeof(double4), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyAsync(c->state3_d.p, src, 3 * RN * sizeof(double), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(k_state_in, dim3((unsigned)((RN + 255) / 256)), dim3(256), 0, c->stream, c->state3_d.p, dst.p, RN);
+    HIPCHK(hipStreamSynchronize(c->stream));
   };
   if (xyz) { up(xyz, c->pos_d); c->lists_valid = false; }
   if (velos) up(velos, c->vel_d);
@@ -1662,12 +1665,11 @@ int sis_gpu_get_rng_tape_pos(sis_gpu_ctx *c, int32_t irep, int64_t *pos) {
 int sis_gpu_get_state(sis_gpu_ctx *c, double *xyz, double *velos, double *accels) {
   API_BEGIN
   if (!c) return fail(SIS_ERR_ARG, "null context");
-  HIPCHK(hipStreamSynchronize(c->stream));
-  size_t RN = (size_t)c->R * c->N;
-  std::vector<double4> h(RN);
+  const size_t RN = (size_t)c->R * c->N;
   auto down = [&](double *dst, DevBuf<double4> &src) {
-    HIPCHK(hipMemcpy(h.data(), src.p, RN * sizeof(double4), hipMemcpyDeviceToHost));
-    for (size_t g = 0; g < RN; g++) { dst[3 * g] = h[g].x; dst[3 * g + 1] = h[g].y; dst[3 * g + 2] = h[g].z; }
+    hipLaunchKernelGGL(k_state_out, dim3((unsigned)((RN + 255) / 256)), dim3(256), 0, c->stream, src.p, c->state3_d.p, RN);
+    HIPCHK(hipMemcpyAsync(dst, c->state3_d.p, 3 * RN * sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
   };
   if (xyz) down(xyz, c->pos_d);
   if (velos) down(velos, c->vel_d);
