@@ -1181,7 +1181,8 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
   const bool mc_on = c->P.nstep_bp_mc > 0;
   if (c->g_step_d.n < 1) c->g_step_d.alloc(1);
   if (c->g_int_d.n < (size_t)R) c->g_int_d.alloc(R);
-  if (c->step_fpair_d.n < RN) { c->step_fpair_d.alloc(RN); c->step_noise_d.alloc(RN); }
+  if (c->step_fpair_d.n < RN) c->step_fpair_d.alloc(RN);
+  if (c->step_noise_d.n < RN) c->step_noise_d.alloc(RN);
   const bool bd = c->P.bd != 0;   // forces and update in one launch (k_step_force)
   const int nblk = bd ? force_blocks(N) : (N + B - 1) / B;
   if (c->step_top2_d.n < (size_t)R * nblk * 2) c->step_top2_d.alloc((size_t)R * nblk * 2);
