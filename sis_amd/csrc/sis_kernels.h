@@ -1084,9 +1084,7 @@ __device__ __forceinline__ bool mc_one_component(const Params &P, const Ptrs &D,
       mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
     return false;
   }
-  const bool ok = n <= 64 * MCW_ITEMS ? mc_component_wave_any(P, D, r, r, root, sg, n, beta, seed, step, ws)
-                                      : mc_component_wave<MCB_ITEMS, MCB_NODES>(P, D, r, r, root, sg, n, beta, seed, step, ws);
-  if (!ok && L == 0) mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
+  if (!mc_component_wave_big(P, D, r, r, root, sg, n, beta, seed, step, ws) && L == 0) mc_component_serial(mc_arrays(D), P.N, r, r, root, sg, n, beta, seed, step);
   return false;
 }
 

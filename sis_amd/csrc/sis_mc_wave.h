@@ -546,6 +546,13 @@ __device__ __forceinline__ bool mc_component_wave_any(const Params &P, const Ptr
   if (n <= 64) return mc_component_wave<1, 2>(P, D, r, rk, root, seg, n, beta, seed, step, ws);
   return mc_component_wave(P, D, r, rk, root, seg, n, beta, seed, step, ws);
 }
+// The same up to the bucket capacity.  ws holds MCB_LDS ints.
+__device__ __forceinline__ bool mc_component_wave_big(const Params &P, const Ptrs &D, int r, int rk, int root,
+                                                      const int *seg, int n, double beta, uint64_t seed,
+                                                      int64_t step, int *ws) {
+  if (n <= 64 * MCW_ITEMS) return mc_component_wave_any(P, D, r, rk, root, seg, n, beta, seed, step, ws);
+  return mc_component_wave<MCB_ITEMS, MCB_NODES>(P, D, r, rk, root, seg, n, beta, seed, step, ws);
+}
 
 // ---------------------------------------------------------------------
 // A component of two pairs (the usual smallest one) by one lane: with one

@@ -552,15 +552,20 @@ __device__ __forceinline__ V3<double> pair_nb_lds(const Params &P, const Ptrs &D
 // Whole job_md steps of system r (src/job_md.F90:374-460) for J.todo steps.
 template <typename T, int B>
 __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, const SysIO &J, const int r) {
-  __shared__ double s1[B], s2[B];
-  __shared__ int s_scan[B];
-  __shared__ double4 s_tile[B];
+  // One region for what is never live at the same time: the wave MC scratch
+  // (a slice per wave, each large enough for a component of the bucket
+  // capacity), and the arrays of the rebuild, the list staging and the
+  // block sums.  Barriers stand between the work list and each of these.
+  __shared__ __align__(32) int s_mcws[(B / 64) * MCB_LDS];
+  static_assert((B / 64) * MCB_LDS * sizeof(int) >= B * (sizeof(double4) + 2 * sizeof(double) + sizeof(int)),
+                "the block arrays share the MC scratch");
+  double4 *s_tile = reinterpret_cast<double4 *>(s_mcws);
+  double *s1 = reinterpret_cast<double *>(s_tile + B), *s2 = s1 + B;
+  int *s_scan = reinterpret_cast<int *>(s2 + B);
   __shared__ int s_flag, s_exit;
   __shared__ int s_exc[EXC_LDS];   // component roots with excess (MC steps)
-  __shared__ int s_nexc, s_big, s_nw, s_next, s_huge;
+  __shared__ int s_nexc, s_nw, s_next, s_huge;
   __shared__ int s_wl[MCW_LIST];   // wavefront-MC components of this step: size << 21 | root
-  __shared__ __align__(16) int s_mcws[(B / 64) * MCW_LDS];   // wave MC scratch, one slice per wave
-  static_assert((B / 64) * MCW_LDS >= MCB_LDS, "large-component MC needs the block's whole scratch");
   const int N = P.N;
   const int tid = threadIdx.x;
   const size_t base = (size_t)r * N;
@@ -750,7 +755,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
         F = group_sum_rt(F, lpb);
         if (a < N && l == 0) DS.fbond[sb + a] = double4{F.x, F.y, F.z, 0.0};
       }
-    if (tid == 0) { s_nexc = 0; s_big = 0; s_nw = 0; s_next = 0; s_huge = 0; }
+    if (tid == 0) { s_nexc = 0; s_nw = 0; s_next = 0; s_huge = 0; }
     __syncthreads();
     int nw = 0, nexc = 0;
     bool listed = true;
@@ -774,7 +779,8 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
       __syncthreads();
       // ---- C: components with excess classified by size (components are
       // disjoint and keyed by their root, so the order does not matter):
-      // the wavefront ones listed with their size, the large ones flagged;
+      // the wavefront ones listed with their size, those above the bucket
+      // capacity flagged;
       // the small ones (one lane each) are work-list items below
       const int wave = tid / 64;
       nexc = s_nexc;
@@ -784,7 +790,6 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
         if (!hexc[root]) continue;
         const int n = segn[root];
         if (n > SEGCAP) { s_huge = 1; continue; }
-        if (n > 64 * MCW_ITEMS) { s_big = 1; continue; }
         if (n > MCL_PAIRS) {
           const int q = atomicAdd(&s_nw, 1);
           if (q < MCW_LIST) s_wl[q] = (n << 21) | root;   // root < 2^21 (N <= 2048 here)
@@ -811,6 +816,11 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
     // partial forces fit in LDS, the bonded and WCA/Debye-Hueckel forces of
     // groups of beads (they do not depend on the MC).  The longest wave is
     // then close to the largest component, with the rest in its shadow.
+    // Components of 129 to 256 pairs are among them: on one wave after the
+    // list, while the others waited, they took 128 of 208 us a step in the
+    // slowest replica of 99 x 211 nucleotides (300 steps with exchanges 50.5
+    // -> 41.9 ms).  The scratch of each wave that this takes, 6.4 KB, costs
+    // no LDS: it is the block arrays' region.
     {
       const int wave = tid / 64, L = tid & 63;
       const int nmc = (mc && nw <= MCW_LIST) ? nw : 0;
@@ -826,7 +836,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
           const int key = s_wl[k];
           const int root = key & 0x1fffff, n = key >> 21;
           int *sg = J.seg + (base + root) * SEGCAP;
-          if (!mc_component_wave_any(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCW_LDS))
+          if (!mc_component_wave_big(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCB_LDS))
             if (L == 0) mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, root, sg, n, beta, J.seed, step);
           continue;
         }
@@ -868,35 +878,10 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
           const size_t gr = base + root;
           if (!hexc[root]) continue;
           const int n = segn[root];
-          if (n <= MCL_PAIRS || n > 64 * MCW_ITEMS) continue;
+          if (n <= MCL_PAIRS || n > SEGCAP) continue;
           int *sg = J.seg + gr * SEGCAP;
-          if (!mc_component_wave_any(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCW_LDS))
+          if (!mc_component_wave_big(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCB_LDS))
             if ((tid & 63) == 0) mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, root, sg, n, beta, J.seed, step);
-        }
-        __syncthreads();
-      }
-      // components above one wave's scratch: wave 0 with the whole block's
-      if (s_big) {
-        if (wave == 0) {
-          const int cnt = listed ? nexc : N;
-          for (int i0 = 0; i0 < cnt; i0 += 64) {
-            const int it = i0 + (tid & 63);
-            int root = 0;
-            bool big = false;
-            if (it < cnt) {
-              root = listed ? s_exc[it] : it;
-              const int n = segn[root];
-              big = hexc[root] && n > 64 * MCW_ITEMS && n <= SEGCAP;
-            }
-            for (unsigned long long m = __ballot(big); m; m &= m - 1) {
-              const int rt = bcast(root, __ffsll((long long)m) - 1);
-              const size_t gr = base + rt;
-              const int n = segn[rt];
-              int *sg = J.seg + gr * SEGCAP;
-              if (!mc_component_wave<MCB_ITEMS, MCB_NODES>(P, DM, rm, J.rk, rt, sg, n, beta, J.seed, step, s_mcws))
-                if ((tid & 63) == 0) mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, rt, sg, n, beta, J.seed, step);
-            }
-          }
         }
         __syncthreads();
       }
