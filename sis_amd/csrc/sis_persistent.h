@@ -814,8 +814,12 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
     // the wavefront-MC components (largest first), then the small
     // components, one lane each, 64 listed roots an item, then, when the
     // partial forces fit in LDS, the bonded and WCA/Debye-Hueckel forces of
-    // groups of beads (they do not depend on the MC).  The longest wave is
-    // then close to the largest component, with the rest in its shadow.
+    // groups of beads, then, with the state in LDS, the noise draws (neither
+    // depends on the MC).  The longest wave is then close to the largest
+    // component, with the rest in its shadow.  The noise takes a bead a lane
+    // here; in the update it ran on one lane in lpb with the others waiting
+    // (500 steps of 14 x 47 nt with exchanges 14.8 -> 14.0 ms, 1,000 of 256
+    // x 128 77.2 -> 76.5).
     // Components of 129 to 256 pairs are among them: on one wave after the
     // list, while the others waited, they took 128 of 208 us a step in the
     // slowest replica of 99 x 211 nucleotides (300 steps with exchanges 50.5
@@ -823,18 +827,23 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
     // no LDS: it is the block arrays' region.
     {
       const int wave = tid / 64, L = tid & 63;
-      const int nmc = (mc && nw <= MCW_LIST) ? nw : 0;
       const int nroot = listed ? nexc : N;
+      // more wavefront components than the list holds: one item a root
+      const bool over = nw > MCW_LIST;
+      const int nmc = !mc ? 0 : over ? nroot : nw;
       const int nlane = mc ? (nroot + 63) / 64 : 0;
       const int bpw = 64 / lpb, nchunk = ovl ? (N + bpw - 1) / bpw : 0;
+      const int nnoise = st ? (N + 63) / 64 : 0;
       for (;;) {
         int k = 0;
         if (L == 0) k = atomicAdd(&s_next, 1);
         k = bcast(k, 0);
-        if (k >= nmc + nlane + nchunk) break;
+        if (k >= nmc + nlane + nchunk + nnoise) break;
         if (k < nmc) {
-          const int key = s_wl[k];
-          const int root = key & 0x1fffff, n = key >> 21;
+          const int key = over ? 0 : s_wl[k];
+          const int root = !over ? key & 0x1fffff : listed ? s_exc[k] : k;
+          const int n = !over ? key >> 21 : hexc[root] ? segn[root] : 0;
+          if (n <= MCL_PAIRS || n > SEGCAP) continue;
           int *sg = J.seg + (base + root) * SEGCAP;
           if (!mc_component_wave_big(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCB_LDS))
             if (L == 0) mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, root, sg, n, beta, J.seed, step);
@@ -856,6 +865,15 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
           }
           continue;
         }
+        if (k >= nmc + nlane + nchunk) {
+          const int a = (k - nmc - nlane - nchunk) * 64 + L;
+          if (a < N) {
+            double n0, n1, n2;
+            noise_normals(J.seed, J.rk, step, a, n0, n1, n2);
+            DS.pos_out[a] = double4{n0, n1, n2, 0.0};
+          }
+          continue;
+        }
         const int a = (k - nmc - nlane) * bpw + L / lpb, lw = L % lpb;
         V3<double> F{0.0, 0.0, 0.0};
         if (a < N) {
@@ -870,21 +888,7 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
     }
     __syncthreads();
     if (mc) {
-      const int wave = tid / 64, nwaves = B / 64;
-      if (nw > MCW_LIST) {
-        // more than the list holds: static round robin over the roots
-        for (int it = wave; it < (listed ? nexc : N); it += nwaves) {
-          const int root = listed ? s_exc[it] : it;
-          const size_t gr = base + root;
-          if (!hexc[root]) continue;
-          const int n = segn[root];
-          if (n <= MCL_PAIRS || n > SEGCAP) continue;
-          int *sg = J.seg + gr * SEGCAP;
-          if (!mc_component_wave_big(P, DM, rm, J.rk, root, sg, n, beta, J.seed, step, s_mcws + wave * MCB_LDS))
-            if ((tid & 63) == 0) mc_component_serial(mc_arrays(DM), P.N, rm, J.rk, root, sg, n, beta, J.seed, step);
-        }
-        __syncthreads();
-      }
+      const int wave = tid / 64;
       // components above the bucket capacity: wave 0, global scratch (the
       // replica's bucket region, free once the passes above are done)
       if (s_huge) {
@@ -975,7 +979,13 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
         if (J.force_only) {
           D.frc[g] = double4{F.x, F.y, F.z, 0.0};
         } else {
-          const double d2 = gjf_update(P, DS, rs, J.rk, a, F, 0, J.seed, step);
+          double d2;
+          if (st) {   // the draws the work list left where the new position goes
+            const double4 z = DS.pos_out[a];
+            d2 = move_bead(P, DS, a, a, F, z.x, z.y, z.z);
+          } else {
+            d2 = gjf_update(P, DS, rs, J.rk, a, F, 0, J.seed, step);
+          }
           if (d2 > m1) { m2 = m1; m1 = d2; }
           else if (d2 > m2) m2 = d2;
         }

@@ -140,3 +140,35 @@ def test_limit_mc_decisions(case, prec):
     assert sizes
     assert not np.any(b["status"][~formed])
     np.testing.assert_array_equal(b["status"][formed] != 0, left)
+
+
+def test_batched_form_with_many_components():
+    """More wavefront components in a replica than the batched kernel's sorted
+    list holds (64): the formed pairs that one step's limit MC leaves are
+    those of the per-phase form, whole-number decisions on the same draws."""
+    rng = np.random.default_rng(11)
+    n, ncl, nrep = 12, 85, 2     # clusters of G and C along one chain, out of each other's reach
+    x = np.concatenate([_cloud(rng, [n], 11.0, (60.0 * (k % 10), 60.0 * (k // 10), 0.0)) for k in range(ncl)])
+    s = _mk("clusters", [random_seq(rng, n * ncl, 1.0)], x, default_params(tempK=310.0, nl_margin=5.0), nrep=nrep,
+            temps=np.array([300.0, 330.0]))
+    print("[case] limit MC, batched form, many components", flush=True)
+    res = []
+    for mode in ("phases", "batched"):
+        e = Engine(s, mode=mode, seed=21)
+        e.neighbor_list(0)
+        if mode == "phases":
+            e.force(1, 1)
+            b = e.bp(1)
+            f = np.signbit(b["ene"])
+            pairs = [tuple(int(v) for v in q[:2] - 1) for q in b["bp"][f]]
+            _, sizes = _limit_mc(pairs, b["ene"][f], 1.6, 21, 0, 0, 1)
+            print(f"[case] components with excess: {sorted(sizes)}", flush=True)
+            assert sum(v > 2 for v in sizes) > 64
+        e.step(1)
+        assert e.info()["mode"] == {"phases": 1, "batched": 3}[mode]
+        res.append([e.bp(r) for r in range(1, nrep + 1)])
+        e.close()
+    for a, b in zip(*res):
+        np.testing.assert_array_equal(a["bp"], b["bp"])
+        assert np.any(a["status"])
+        np.testing.assert_array_equal(a["status"] != 0, b["status"] != 0)
