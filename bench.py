@@ -49,7 +49,7 @@ def bytes_per_bead_step(p_wca, p_ele, p_bp):
 
 
 def load_traffic(workload, mode):
-    """Measured HBM bytes per bead-step of the dominant kernel (FETCH_SIZE +
+    """Measured HBM bytes per bead-step of the roofline's kernels (FETCH_SIZE +
     WRITE_SIZE, calibrated; profiles/traffic.json names the summary each
     figure comes from), or None."""
     f = ROOT / "profiles" / "traffic.json"
