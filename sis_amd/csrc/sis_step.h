@@ -23,7 +23,7 @@
 // skin test, the resets and the large-component pass inside these launches
 // a step takes four launches where it took seven.  Before and after, one
 // MI355X, microseconds a step: 64 nt FP64 50 -> 33, 397 nt FP32 75 -> 62,
-// 9,400 beads FP64 79 -> 61, 94,000 beads FP32 139 -> 119.
+// 9,400 beads FP64 79 -> 61, 94,000 beads FP32 139 -> 111.
 #pragma once
 #include "sis_kernels.h"
 
