@@ -313,10 +313,27 @@ __device__ __forceinline__ V3<double> dih_force_p(const Params &P, const V3<doub
   return (-a) * fi + (-1.0 + b) * fl;
 }
 
+// Sum without contraction: the products that a and b come from are rounded
+// before they are added, whatever code stands around the sum.
+__device__ __forceinline__ V3<double> add_nc(const V3<double> &a, const V3<double> &b) {
+#pragma clang fp contract(off)
+  return V3<double>{a.x + b.x, a.y + b.y, a.z + b.z};
+}
+// a where `on`, else zero (not 0 * a: that is NaN for an infinite a)
+template <typename T>
+__device__ __forceinline__ V3<T> keep(bool on, const V3<T> &a) {
+  return V3<T>{on ? a.x : (T)0, on ? a.y : (T)0, on ? a.z : (T)0};
+}
+
 // Pair forces take no branch: beyond the cutoff, and for a pair that is not
-// there (on = false), the factor of v12 is zero.  A wavefront works several
-// pairs at a time through these dependent chains (divide, square root,
-// exponential), and a branch around each would run them one by one.
+// there (on = false), the force is selected to be zero.  A wavefront works
+// several pairs at a time through these dependent chains (divide, square
+// root, exponential), and a branch around each would run them one by one.
+//
+// A pair's force is rounded before it is added (add_nc).  Without a branch
+// between them the compiler contracts the last product and the sum, and
+// Brownian runs at a step where a bond is stiff (see k_step_force) carry
+// that last bit into other coordinates and other numbers of list rebuilds.
 //
 // WCA (src/force_wca.F90:51-58): force on bead 1 of v12 = x1 - x2.
 template <typename T>
@@ -328,7 +345,7 @@ __device__ __forceinline__ V3<T> wca_force(const Params &P, const V3<T> &v12, bo
   else s = (T)P.wca_sig2 / d2;
   T s2 = s * s, s4 = s2 * s2, s7 = s4 * s2 * s;
   const T f = (T)P.wca_coef * (s7 - s4);
-  return (!on || d2 >= (T)P.wca_sig2 ? (T)0 : f) * v12;
+  return keep(!(!on || d2 >= (T)P.wca_sig2), f * v12);
 }
 // Debye-Hueckel (src/force_ele_DH.F90:57-68): force on bead 1 of v12.
 template <typename T>
@@ -344,7 +361,7 @@ __device__ __forceinline__ V3<T> dh_force(T coef, T rc2, T rlam, const V3<T> &v1
     r1 = (T)1 / d1;
   }
   T dv = coef * r1 * r1 * (r1 + rlam) * m_exp(-d1 * rlam);
-  return (!on || d2 > rc2 ? (T)0 : dv) * v12;
+  return keep(!(!on || d2 > rc2), dv * v12);
 }
 
 // One BP angle term for the angle between a (= v12) and b, with

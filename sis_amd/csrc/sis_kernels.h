@@ -1143,6 +1143,14 @@ __global__ void k_noise_parity(Params P, Ptrs D, int count, int dest, const int 
 // GJF-2GJ update of one bead (src/job_md.F90:415-444), or the
 // Ermak-McCammon Brownian step (lines 446-456) when P.bd; g = r*N + a.
 // Returns |move|^2.
+//
+// The Brownian move says which of its two products is rounded on its own:
+// left to the compiler it depends on the code around it, and a run at a step
+// where a bond is stiff (see k_step_force) turns that last bit into another
+// trajectory.  It is the force's product, but for z in the kernels that keep
+// the state through many steps (Z_NOISE: persistent, batched, jobs) the
+// noise's: the forms that runs of either kind have had all along.
+template <bool Z_NOISE = false>
 __device__ __forceinline__ double move_bead(const Params &P, const Ptrs &D, size_t g, int a,
                                             const V3<double> &F, double n0, double n1, double n2) {
   const double cr = D.md_cr[g], ca = D.md_a[a];
@@ -1151,9 +1159,9 @@ __device__ __forceinline__ double move_bead(const Params &P, const Ptrs &D, size
   double dx, dy, dz;
   if (P.bd) {
     // dx = (h/gamma) F + sqrt(2 kT h/gamma) xi; velocities are not used
-    dx = ca * F.x + cr * n0;
-    dy = ca * F.y + cr * n1;
-    dz = ca * F.z + cr * n2;
+    dx = __builtin_fma(cr, n0, ca * F.x);
+    dy = __builtin_fma(cr, n1, ca * F.y);
+    dz = Z_NOISE ? __builtin_fma(ca, F.z, cr * n2) : __builtin_fma(cr, n2, ca * F.z);
   } else {
     const double cf = D.md_cf[a], cx = D.md_cx[a];
     double4 v = D.vel[g];
@@ -1249,7 +1257,7 @@ __device__ __forceinline__ V3<double> pair_nb(const Params &P, const Ptrs &D, in
 #pragma unroll
     for (int u = 0; u < PAIR_U; u++) f[u] = wca_force<T>(P, cvt<T>(pvec(P, box, pa, pb[u])), id[u] >= 0);
 #pragma unroll
-    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+    for (int u = 0; u < PAIR_U; u++) F = add_nc(F, cvt<double>(f[u]));
   }
   const int *nbe = D.nb_ele + (size_t)r * D.maxnb * N + a;
   for (int k0 = l; k0 < ne; k0 += PAIR_U * LPB) {
@@ -1266,7 +1274,7 @@ __device__ __forceinline__ V3<double> pair_nb(const Params &P, const Ptrs &D, in
 #pragma unroll
     for (int u = 0; u < PAIR_U; u++) f[u] = dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, pb[u])), id[u] >= 0);
 #pragma unroll
-    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+    for (int u = 0; u < PAIR_U; u++) F = add_nc(F, cvt<double>(f[u]));
   }
   return F;
 }
@@ -1333,6 +1341,7 @@ __device__ __forceinline__ void noise_normals(uint64_t seed, int rk, int64_t ste
 // One bead's update with its noise draws (the injected MT words in the
 // parity form, else the counter RNG); r indexes the per-replica arrays,
 // rk keys the random stream.
+template <bool Z_NOISE = false>
 __device__ __forceinline__ double gjf_update(const Params &P, const Ptrs &D, int r, int rk, int a,
                                              const V3<double> &F, int parity, uint64_t seed,
                                              int64_t step) {
@@ -1344,7 +1353,7 @@ __device__ __forceinline__ double gjf_update(const Params &P, const Ptrs &D, int
   } else {
     noise_normals(seed, rk, step, a, n0, n1, n2);
   }
-  return move_bead(P, D, g, a, F, n0, n1, n2);
+  return move_bead<Z_NOISE>(P, D, g, a, F, n0, n1, n2);
 }
 
 template <int LPB>

@@ -187,7 +187,7 @@ __global__ void __launch_bounds__(B) k_persistent(Params P, Ptrs D, PersArgs A) 
           D.comp[a] = a;
           A.seg_n[a] = 0;
           A.has_exc[a] = 0;
-          double d2 = gjf_update(P, D, 0, 0, a, F, 0, A.seed, step);
+          double d2 = gjf_update<true>(P, D, 0, 0, a, F, 0, A.seed, step);
           if (d2 > m1) { m2 = m1; m1 = d2; }
           else if (d2 > m2) m2 = d2;
         }
@@ -533,7 +533,7 @@ __device__ __forceinline__ V3<double> pair_nb_lds(const Params &P, const Ptrs &D
       f[u] = wca_force<T>(P, cvt<T>(pvec(P, box, pa, x[k < nw ? s_nb[off + k] : a])), k < nw);
     }
 #pragma unroll
-    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+    for (int u = 0; u < PAIR_U; u++) F = add_nc(F, cvt<double>(f[u]));
   }
   const int *e = s_nb + off + nw;
   for (int k0 = l; k0 < ne; k0 += PAIR_U * LPB) {
@@ -544,7 +544,7 @@ __device__ __forceinline__ V3<double> pair_nb_lds(const Params &P, const Ptrs &D
       f[u] = dh_force<T>(coef, rc2, rl, cvt<T>(pvec(P, box, pa, x[k < ne ? e[k] : a])), k < ne);
     }
 #pragma unroll
-    for (int u = 0; u < PAIR_U; u++) F = F + cvt<double>(f[u]);
+    for (int u = 0; u < PAIR_U; u++) F = add_nc(F, cvt<double>(f[u]));
   }
   return F;
 }
@@ -982,9 +982,9 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
           double d2;
           if (st) {   // the draws the work list left where the new position goes
             const double4 z = DS.pos_out[a];
-            d2 = move_bead(P, DS, a, a, F, z.x, z.y, z.z);
+            d2 = move_bead<true>(P, DS, a, a, F, z.x, z.y, z.z);
           } else {
-            d2 = gjf_update(P, DS, rs, J.rk, a, F, 0, J.seed, step);
+            d2 = gjf_update<true>(P, DS, rs, J.rk, a, F, 0, J.seed, step);
           }
           if (d2 > m1) { m2 = m1; m1 = d2; }
           else if (d2 > m2) m2 = d2;

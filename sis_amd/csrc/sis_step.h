@@ -331,8 +331,9 @@ __global__ void __launch_bounds__(STEP_B) k_step_move(Params P, Ptrs D, StepArgs
 // launch (force_lanes), in place of the tiles of the other launches and of
 // k_step_move.  Its positions move by h/gamma times the force with no
 // inertia in between, and where a bond is stiff for the step (h k / gamma
-// above 2) such a run amplifies the last bit of every sum, so these runs
-// keep the order of summation that steps launched one by one have.
+// near or above 2) such a run amplifies the last bit of every sum, so these
+// runs keep the order of summation and the rounding that steps launched one
+// by one have (add_nc, move_bead).
 template <typename T>
 __global__ void __launch_bounds__(STEP_B) k_step_force(Params P, Ptrs D, StepArgs A) {
   if (A.w->halt || (!A.sep_huge && A.w->huge_any)) return;
