@@ -1157,16 +1157,11 @@ bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
     const StepWords &w = pin[nread % 2];
     halt = w.halt != 0;
     huge = w.huge_any != 0 && !c->step_sep_huge;   // (with its launch in every step it is done within it)
-    done = w.done;
+    done = huge ? w.huge_step - 1 : w.done;   // that step waits for its update
     nread++;
   }
   HIPCHK(hipStreamSynchronize(c->stream));
-  if (huge && !halt) {   // noted by a later step's first launch, if there was one
-    const StepWords &w = pin[(nb - 1) % 2];
-    halt = w.halt != 0;
-    done = w.done;
-  }
-  c->istep = halt ? done : huge ? base + issued - 1 : base + issued;
+  c->istep = halt || huge ? done : base + issued;
   // the positions are in the buffer that so many steps leave them in
   if (c->pos_d.p != pos0) std::swap(c->pos_d, c->pos2_d);
   if ((c->istep - base) % 2) std::swap(c->pos_d, c->pos2_d);
@@ -1262,7 +1257,7 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
       c->rebuilds++;
       for (int r = 0; r < R; r++) fmc[r] = c->rebuilt[r] && mc_on ? 1 : 0;
     }
-    const StepWords w0{c->istep, stop, 0, any ? c->istep + 1 : -1, 0, 0};
+    const StepWords w0{c->istep, stop, 0, any ? c->istep + 1 : -1, 0, 0, 0};
     HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w0, sizeof w0, hipMemcpyHostToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(c->g_int_d.p, fmc.data(), R * sizeof(int), hipMemcpyHostToDevice, c->stream));
     // no skin test before the first step: the rebuild above was its answer
@@ -1323,7 +1318,7 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
       // launch in every step
       c->step_sep_huge = true;
       A.sep_huge = 1;
-      const StepWords w1{c->istep, stop, 0, w0.force_step, 0, 0};
+      const StepWords w1{c->istep, stop, 0, w0.force_step, 0, 0, 0};
       HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w1, sizeof w1, hipMemcpyHostToDevice, c->stream));
       A.nj = 1;
       launch_step(1, 0);

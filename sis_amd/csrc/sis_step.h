@@ -45,8 +45,9 @@ struct StepWords {
   int64_t stop;         // stop once this step is completed
   int64_t done;         // steps completed when they halted
   int64_t force_step;   // the step whose replicas with force_mc do the limit MC (after a rebuild)
+  int64_t huge_step;    // the step that met a component above the bucket capacity (with huge_any)
   int halt;             // 1: this step and all after it do nothing
-  int huge_any;         // a component above the bucket capacity was met
+  int huge_any;         // such a component was met
 };
 
 // Arguments of one launch of step j (0-based) of a batch of nj.
@@ -90,8 +91,10 @@ __device__ __forceinline__ bool step_halted(const Params &P, const StepArgs &A, 
   int64_t done = at;
   bool h = before;
   if (!h && !A.sep_huge && A.w->huge_any) {
+    // that step waits for its update (step0 may be stale here: a batch whose
+    // last step waits has not committed)
     h = true;
-    done = at - 1;   // the step before waits for its update
+    done = A.w->huge_step - 1;
   }
   h = __syncthreads_or(h || at >= A.w->stop) != 0;   // one answer for the block
   if (!h) {
@@ -275,7 +278,10 @@ __global__ void __launch_bounds__(STEP_B) k_step_mc(Params P, Ptrs D, StepArgs A
   for (int k = blockIdx.x + wave * A.nlist; k < n; k += A.nlist * (STEP_B / 64)) {
     const int gr = A.exc_list[1 + k];
     const int r = gr / P.N, root = gr - r * P.N;
-    if (mc_one_component(P, D, r, root, A.seg_n, A.seg, nullptr, A.seed, step, A.huge, ws[wave])) A.w->huge_any = 1;
+    if (mc_one_component(P, D, r, root, A.seg_n, A.seg, nullptr, A.seed, step, A.huge, ws[wave])) {
+      A.w->huge_step = step;   // every wavefront that meets one writes the same values
+      A.w->huge_any = 1;
+    }
   }
 }
 

@@ -1,0 +1,100 @@
+"""Device-driven batches of steps at the places where the device and the
+host agree on how far a batch got: halts for a rebuild, the stop, and a
+conflict component above the bucket capacity (256 pairs), whose step waits
+for the host.  Compared with the general path, which launches every phase by
+itself (taken with external terms: here an Rg bias of strength zero): the
+same lists, draws and limit-MC choices, sums in another order, so coordinates
+of up to 1,000 A agree within 1e-9 A over these smooth runs."""
+import numpy as np
+import pytest
+
+from sis_amd import configs
+from sis_amd.engine import Engine
+from sis_amd.forcefield import default_params
+
+pytestmark = pytest.mark.gpu
+
+
+def _largest(e):
+    """Pairs of the largest component of the formed pairs (before deletions)."""
+    b = e.bp(1)
+    pairs = b["bp"][np.signbit(b["ene"])][:, :2].astype(int)
+    parent = {}
+
+    def find(x):
+        parent.setdefault(x, x)
+        while parent[x] != x:
+            x = parent[x]
+        return x
+
+    for i, j in pairs:
+        i, j = find(i), find(j)
+        parent[max(i, j)] = min(i, j)
+    return max(np.unique([find(i) for i, _ in pairs], return_counts=True)[1])
+
+
+def _chain(nstep_mc, **over):
+    rng = np.random.default_rng(11)
+    seq = configs.random_seq(rng, 2048, 0.6)
+    return configs._mk("chain2048", [seq], configs.random_coil(rng, 2048),
+                       default_params(tempK=300.0, nl_margin=15.0, nstep_bp_mc=nstep_mc, **over))
+
+
+@pytest.fixture(scope="module")
+def large_state():
+    """A state of a 2,048-nt chain with a component of about 320 pairs."""
+    e = Engine(_chain(1), mode="phases", seed=9)
+    e.init_velocities()
+    e.neighbor_list(0)
+    e.step(100)
+    st = e.get_state()
+    n = _largest(e)
+    e.close()
+    print(f"[case] largest component {n}", flush=True)
+    assert n > 280
+    return st
+
+
+def _run(state, every, at, n, general=False, no_graph=False, **over):
+    """n steps whose at-th is the first with a limit MC."""
+    e = Engine(_chain(every, **over), mode="phases", seed=9, no_graph=no_graph)
+    if general:
+        e.set_external(dict(rg=1, rg_k=0.0, rg_0=10.0))
+    e.set_state(*state)
+    e.neighbor_list(0)
+    e.set_step(every - at)
+    rebuilds = e.step(n)
+    out = (*e.get_state(), e.info()["istep"], rebuilds, e.bp(1)["status"])
+    if general and n == at:
+        assert _largest(e) > 256
+    e.close()
+    return out
+
+
+def _same(a, b, end):
+    assert a[3] == b[3] == end
+    assert a[4] == b[4] == 0
+    np.testing.assert_array_equal(a[2], b[2])      # noise terms: the same draws
+    np.testing.assert_array_equal(a[5], b[5])
+    assert np.abs(a[0] - b[0]).max() < 1e-9
+
+
+@pytest.mark.parametrize("every", [1000, 40])
+def test_first_large_component_at_every_place_of_a_batch(large_state, every):
+    """The first component above the bucket capacity at the edges of a run's
+    first and third batch of 16 steps and at every place of its second, the
+    run ending there or later; every = 40: met again after the hand-over.
+    Replayed from a graph and issued directly."""
+    for at in (1, 2, 15, *range(16, 34), 47, 48, 49) if every > 49 else (1, 16, 31, 32, 33):
+        for n in (at, at + 20) if at in (1, 16, 32, 33) else (at + 20,):
+            want = _run(large_state, every, at, n, general=True)
+            for no_graph in (False, True):
+                print(f"[case] first large component at step {at} of {n}, every {every}, no_graph {no_graph}", flush=True)
+                _same(_run(large_state, every, at, n, no_graph=no_graph), want, every - at + n)
+
+
+@pytest.mark.parametrize("at", [31, 32, 33])
+def test_first_large_component_brownian(large_state, at):
+    print(f"[case] first large component at step {at}, Brownian", flush=True)
+    kw = dict(integrator=2, dt=0.005)
+    _same(_run(large_state, 1000, at, at + 20, **kw), _run(large_state, 1000, at, at + 20, general=True, **kw), 1020)
