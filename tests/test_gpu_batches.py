@@ -98,3 +98,40 @@ def test_first_large_component_brownian(large_state, at):
     print(f"[case] first large component at step {at}, Brownian", flush=True)
     kw = dict(integrator=2, dt=0.005)
     _same(_run(large_state, 1000, at, at + 20, **kw), _run(large_state, 1000, at, at + 20, general=True, **kw), 1020)
+
+
+@pytest.mark.parametrize("case", ["chain, MC every step", "ladder, MC every 3", "box"])
+def test_batches_with_rebuilds_match_single_launches(case):
+    """200 steps with halts for rebuilds inside the batches (0.3 to 1 A
+    skins), the limit MC after them, and exchanges: replayed and issued
+    directly they give the same bits, and the general path the same labels,
+    rebuilds, noise and formed pairs.  Coordinates within 1e-6 A, as other
+    forms agree over hundreds of steps."""
+    nex = 0
+    if case == "chain, MC every step":
+        s = configs.remd_c3(nrep=1, n=128, seed=3, margin=0.3)
+    elif case == "ladder, MC every 3":
+        s, nex = configs.remd_c3(nrep=4, n=128, seed=3, margin=1.0), 25
+        s["params"] = dict(s["params"], nstep_bp_mc=3)
+    else:
+        s = configs.cag_system(40, 47, 1.0, 310.0, margin=1.0)
+    out = []
+    for general, no_graph in ((True, False), (False, False), (False, True)):
+        print(f"[case] batches with rebuilds: {case}, general {general}, no_graph {no_graph}", flush=True)
+        e = Engine(s, mode="phases", precision=1, seed=4242, exchange_every=nex, no_graph=no_graph)
+        if general:
+            e.set_external(dict(rg=1, rg_k=0.0, rg_0=10.0))
+        e.init_velocities()
+        e.neighbor_list(0)
+        reb = e.step(37) + e.step(163)
+        out.append((*e.get_state(), reb, e.labels(), [e.bp(r + 1)["status"] for r in range(s["nrep"])]))
+        e.close()
+    for a in out[1:]:
+        assert a[3] == out[0][3] > 2
+        np.testing.assert_array_equal(a[4], out[0][4])
+        np.testing.assert_array_equal(a[2], out[0][2])
+        for u, v in zip(a[5], out[0][5]):
+            np.testing.assert_array_equal(u, v)
+        assert np.abs(a[0] - out[0][0]).max() < 1e-6
+    for u, v in zip(out[1][:3], out[2][:3]):
+        np.testing.assert_array_equal(u, v)
