@@ -1131,10 +1131,6 @@ bool graph_steps_ok(sis_gpu_ctx *c) { return !c->parity && !c->ext_on && c->opt.
 // component above the bucket capacity (k_step_huge).
 template <typename F>
 bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
-  if (!c->step_pin) {
-    HIPCHK(hipHostMalloc(&c->step_pin, 2 * sizeof(StepWords), hipHostMallocDefault));
-    for (auto &e : c->step_ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  }
   StepWords *pin = static_cast<StepWords *>(c->step_pin);
   const int64_t base = c->istep;
   double4 *const pos0 = c->pos_d.p;
@@ -1170,19 +1166,33 @@ bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
 
 inline int pad8(int64_t n) { return (int)((n + 7) / 8 * 8); }
 
+// blocks per replica of a batch's last launch
+inline int step_blocks(const sis_gpu_ctx *c) { return c->P.bd ? force_blocks(c->N) : (c->N + STEP_B - 1) / STEP_B; }
+
+// What the batches keep in the context.  Made with the first step; the job
+// pool makes them when it admits a job, where they count towards the job's
+// memory and no other job's steps wait for an allocation.
+void step_buffers(sis_gpu_ctx *c) {
+  const size_t RN = (size_t)c->R * c->N, top2 = (size_t)c->R * step_blocks(c) * 2;
+  if (c->g_step_d.n < 1) c->g_step_d.alloc(1);
+  if (c->g_int_d.n < (size_t)c->R) c->g_int_d.alloc(c->R);
+  if (!c->P.bd && c->step_fpair_d.n < RN) c->step_fpair_d.alloc(RN);
+  if (!c->P.bd && c->step_noise_d.n < RN) c->step_noise_d.alloc(RN);
+  if (c->step_top2_d.n < top2) c->step_top2_d.alloc(top2);
+  if (c->P.nstep_bp_mc > 0 && c->seg_d.n < RN * SEGCAP) c->seg_d.alloc(RN * SEGCAP);
+  if (c->P.nstep_bp_mc > 0 && c->exc_list_d.n < RN + 1) c->exc_list_d.alloc(RN + 1);
+  if (!c->step_pin) HIPCHK(hipHostMalloc(&c->step_pin, 2 * sizeof(StepWords), hipHostMallocDefault));
+  for (auto &e : c->step_ev)
+    if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+}
+
 void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
   const int N = c->N, R = c->R, B = STEP_B;
   const size_t RN = (size_t)R * N;
   const bool mc_on = c->P.nstep_bp_mc > 0;
-  if (c->g_step_d.n < 1) c->g_step_d.alloc(1);
-  if (c->g_int_d.n < (size_t)R) c->g_int_d.alloc(R);
-  if (c->step_fpair_d.n < RN) c->step_fpair_d.alloc(RN);
-  if (c->step_noise_d.n < RN) c->step_noise_d.alloc(RN);
   const bool bd = c->P.bd != 0;   // forces and update in one launch (k_step_force)
-  const int nblk = bd ? force_blocks(N) : (N + B - 1) / B;
-  if (c->step_top2_d.n < (size_t)R * nblk * 2) c->step_top2_d.alloc((size_t)R * nblk * 2);
-  if (mc_on && c->seg_d.n < RN * SEGCAP) c->seg_d.alloc(RN * SEGCAP);
-  if (mc_on && c->exc_list_d.n < RN + 1) c->exc_list_d.alloc(RN + 1);
+  const int nblk = step_blocks(c);
+  step_buffers(c);
   StepArgs A{};
   A.w = c->g_step_d.p;
   A.force_mc = c->g_int_d.p;

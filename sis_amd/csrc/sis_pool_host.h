@@ -157,6 +157,7 @@ bool job_admit(sis_pool *p, PoolJob &j) {
     return false;
   }
   if (c->seg_d.n < (size_t)c->N * SEGCAP) c->seg_d.alloc((size_t)c->N * SEGCAP);
+  if (j.nmp > POOL_WG_MAX) step_buffers(c);
   j.slot = p->free_slots.back();
   p->free_slots.pop_back();
   int io[4] = {0, c->nbp_total, 0, 0};

@@ -5,12 +5,16 @@ for the host.  Compared with the general path, which launches every phase by
 itself (taken with external terms: here an Rg bias of strength zero): the
 same lists, draws and limit-MC choices, sums in another order, so coordinates
 of up to 1,000 A agree within 1e-9 A over these smooth runs."""
+import time
+
 import numpy as np
 import pytest
+import torch
 
 from sis_amd import configs
 from sis_amd.engine import Engine
 from sis_amd.forcefield import default_params
+from sis_amd.serving import RUNNING, JobPool
 
 pytestmark = pytest.mark.gpu
 
@@ -135,3 +139,43 @@ def test_batches_with_rebuilds_match_single_launches(case):
         assert np.abs(a[0] - out[0][0]).max() < 1e-6
     for u, v in zip(out[1][:3], out[2][:3]):
         np.testing.assert_array_equal(u, v)
+
+
+def _lattice(nch, n=100):
+    """Zigzag chains on a lattice, 50 A apart."""
+    k = np.arange(n)
+    one = np.stack([5.7 * k, 1.5 * (k % 2), 0.0 * k], 1)
+    at = np.array([[0.0, 50.0 * (c // 40), 50.0 * (c % 40)] for c in range(nch)])
+    rng = np.random.default_rng(5)
+    return configs._mk("lattice", [configs.random_seq(rng, n, 0.5)] * nch, (one + at[:, None]).reshape(-1, 3),
+                       default_params(nl_margin=5.0))
+
+
+def test_pool_counts_what_a_large_job_steps_with():
+    """A job above one workgroup's size is charged for the buffers of its
+    step batches (64 B a bead, 7.7 MB here) when it is admitted: as much as
+    an engine of the same system holds after its first steps.  2 MB: the
+    granularity of the card's memory count."""
+    small, big = _lattice(30), _lattice(1200)
+    for _ in range(5):     # what the kernels themselves need, on every queue
+        e = Engine(small, mode="phases", no_graph=True)
+        e.neighbor_list(0)
+        e.step(20)
+        e.close()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    e = Engine(big, mode="phases", no_graph=True)
+    e.neighbor_list(0)
+    e.init_velocities()
+    e.step(20)
+    held = free - torch.cuda.mem_get_info()[0]
+    e.close()
+    with JobPool(quantum_bead_steps=big["xyz"].size) as pool:
+        j = pool.submit(big, 10 ** 6, seed=3)
+        until = time.time() + 60
+        while pool.poll(j)[1][3] < 10 and time.time() < until:
+            time.sleep(0.01)
+        assert pool.poll(j)[0] == RUNNING
+        charged = pool.stats()["bytes"]
+    print(f"[case] large job: engine holds {held}, pool charges {charged}", flush=True)
+    assert charged > held - (2 << 20)
