@@ -194,68 +194,10 @@ template <typename T, typename S>
 __device__ __forceinline__ V3<T> cvt(const V3<S> &v) { return V3<T>{(T)v.x, (T)v.y, (T)v.z}; }
 
 // ---------------------------------------------------------------------
-// Bonded terms.  Each returns the force on every bead of the term, in the
-// reference's expressions (src/force_bond.F90:42-50,
-// src/force_angl_ReB.F90:43-59, src/force_angl.F90:42-66,
-// src/force_dih_exp.F90:44-79, src/force_dih_cos.F90:28-54).
-template <typename T>
-__device__ __forceinline__ void bond_force(const Params &P, const V3<T> &v, V3<T> f[2]) {
-  T d = m_sqrt(dot(v, v));
-  T delta = d - (T)P.bond_r0;
-  V3<T> fv = ((T)P.bond_k * delta / d) * v;   // v = x1 - x2
-  f[0] = -fv;
-  f[1] = fv;
-}
-template <typename T>
-__device__ __forceinline__ void angle_force(const Params &P, const V3<T> &v12, const V3<T> &v32,
-                                            V3<T> f[3]) {
-  if (P.angl_reb) {
-    T d12 = dot(v12, v12), d32 = dot(v32, v32), a1232 = m_sqrt(d12 * d32);
-    T cosine = dot(v12, v32) / a1232;
-    T co0 = (T)P.angl_co0;
-    T den = (T)1 - cosine * cosine;
-    T ff = -(T)P.angl_k * (cosine - co0) * ((T)1 - cosine * co0) / (den * den);
-    V3<T> f1 = ff * ((T(1) / a1232) * v32 - (cosine / d12) * v12);
-    V3<T> f3 = ff * ((T(1) / a1232) * v12 - (cosine / d32) * v32);
-    f[0] = f1; f[1] = -(f1 + f3); f[2] = f3;
-  } else {
-    V3<T> v21 = -v12;  // x2 - x1
-    T d21 = dot(v21, v21), d32 = dot(v32, v32), d2132 = dot(v32, v21);
-    T cosine = -d2132 / m_sqrt(d21 * d32);
-    if (cosine > (T)1) cosine = (T)1;
-    if (cosine < (T)-1) cosine = (T)-1;
-    T delta = m_acos(cosine) - (T)P.angl_t0;
-    T t = d21 * d32 - d2132 * d2132;
-    if (t <= (T)1) t = (T)1;
-    T ff = (T)P.angl_k * delta / m_sqrt(t);
-    V3<T> f21 = ff * ((d2132 / d21) * v21 - v32);
-    V3<T> f32 = ff * ((d2132 / d32) * v32 - v21);
-    f[0] = -f21; f[1] = f21 - f32; f[2] = f32;
-  }
-}
-template <typename T>
-__device__ __forceinline__ void dih_force(const Params &P, const V3<T> &vij, const V3<T> &vkj,
-                                          const V3<T> &vkl, V3<T> f[4]) {
-  V3<T> m = cross(vij, vkj), n = cross(vkj, vkl);
-  T akj2 = dot(vkj, vkj), akj = m_sqrt(akj2);
-  T dih = m_atan2(akj * dot(vij, n), dot(m, n));
-  T pre;
-  if (P.dih_type == 2) {
-    T dd = dih - (T)P.dih_p0;
-    pre = (T)(P.dih_k * P.dih_w) * dd * m_exp((T)(-0.5 * P.dih_w) * (dd * dd)) * akj;
-  } else {
-    pre = -(T)P.dih_k * m_sin(dih + (T)P.dih_p0) * akj;
-  }
-  V3<T> fi = (-pre / dot(m, m)) * m;
-  V3<T> fl = (pre / dot(n, n)) * n;
-  T a = dot(vij, vkj) / akj2, b = dot(vkl, vkj) / akj2;
-  f[0] = fi;
-  f[1] = ((T)-1 + a) * fi + (-b) * fl;
-  f[2] = (-a) * fi + ((T)-1 + b) * fl;
-  f[3] = fl;
-}
-
-// Force on position p of a bonded term only (owner-computes).
+// Bonded terms: the force on position p of a term, in the reference's
+// expressions (src/force_bond.F90:42-50, src/force_angl_ReB.F90:43-59,
+// src/force_angl.F90:42-66, src/force_dih_exp.F90:44-79,
+// src/force_dih_cos.F90:28-54).
 __device__ __forceinline__ V3<double> bond_force_p(const Params &P, const V3<double> &v, int p) {
   double d = sqrt(dot(v, v));
   double delta = d - P.bond_r0;
