@@ -241,6 +241,7 @@ struct sis_gpu_ctx {
   // the per-phase form's captured steps (phases_graph_steps), one graph
   // for each of the two position buffers a replay can start from
   hipGraphExec_t pg_exec[2] = {nullptr, nullptr};
+  bool time_steps = true;  // events around the steps of directly issued batches (SIS_OPT_NO_GRAPH); not in the job pool
   bool pg_eager = false;   // the same batches of steps issued directly instead (the autotuner's choice)
   PhaseGraphKey pg_key[2]{};
   int dx_graph_key[4] = {0, 0, 0, 0};   // block, precision, exchange cadence, dynamic LDS of the captured graph
@@ -1164,6 +1165,8 @@ bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
   return huge;
 }
 
+constexpr size_t STEP_MARKS = 4096;
+
 inline int pad8(int64_t n) { return (int)((n + 7) / 8 * 8); }
 
 // blocks per replica of a batch's last launch
@@ -1246,9 +1249,17 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     if (c->precision == 1) kernels(0.0f, part, j);
     else kernels(0.0, part, j);
   };
+  // sis_gpu_last_kernel_ms: events around each step issued directly by a
+  // context that asked for that, for the first STEP_MARKS of a call
+  const bool marks = (c->opt.flags & SIS_OPT_NO_GRAPH) && c->time_steps;
   auto launch_batch = [&](int n) {
     A.nj = n;
-    for (int j = 0; j < n; j++) launch_step(0, j);
+    for (int j = 0; j < n; j++) {
+      const bool m = marks && c->tev_used < 2 * STEP_MARKS;
+      if (m) c->tmark();
+      launch_step(0, j);
+      if (m) c->tmark();
+    }
   };
   while (c->istep < stop) {
     // a rebuild due from the last skin test, or lists not built yet
@@ -1293,7 +1304,11 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     // which pays for large systems (a graph launch costs more per node
     // than a kernel launch here)
     if (c->pg_eager || (c->opt.flags & SIS_OPT_NO_GRAPH)) {
+      const size_t mark0 = c->tev_used;
+      const int64_t at = c->istep;
       wait_huge = run_phase_batches(c, stop, true, launch_batch);
+      // steps issued after a halt did nothing
+      c->tev_used = std::min(c->tev_used, mark0 + 2 * (size_t)(c->istep - at));
     } else {
       int slot = -1;
       for (int q = 0; q < 2; q++)

@@ -140,6 +140,7 @@ bool job_admit(sis_pool *p, PoolJob &j) {
   sis_gpu_ctx *c = nullptr;
   if (sis_gpu_create(&t, &j.prm, &o, &c) != SIS_OK) { job_fail(p, j, g_err); return false; }
   j.c = c;
+  c->time_steps = false;
   if (!p->have_P0) {
     p->P0 = c->P;
     std::memcpy(p->bpp0, c->bpp_h, sizeof p->bpp0);
