@@ -917,29 +917,34 @@ __device__ __forceinline__ void batched_body(const Params &P, const Ptrs &D, con
         for (int k = tid; k < nbr; k += B) D.bp_status_mc[r * J.capb + k] = D.bp_status[r * J.capb + k];
     }
     if (J.energy_mode) {
-      // energy_sumup: per-bead terms summed as k_energy and k_energy_reduce
-      // do (blocks of 256 beads, tree sum, blocks in order), so the result
-      // equals the per-phase evaluation's
-      // (128 threads: each holds beads t and t + 128, the tree's first level)
-      static_assert(B == 128 || B >= 256, "energy sums need 128 or at least 256 threads");
-      constexpr int H = B < 256 ? B : 256;
+      // energy_sumup: terms summed as k_energy and k_energy_reduce do
+      // (ENE_LPB lanes a bead, blocks of 256 beads, tree sum, blocks in
+      // order), so the result equals the per-phase evaluation's
+      static_assert((B / 64) * MCB_LDS * sizeof(int) >= 6 * 256 * sizeof(double), "the sums share the MC scratch");
+      double *se = reinterpret_cast<double *>(s_mcws);
+      const int l4 = tid % ENE_LPB;
       __syncthreads();
       double acc[7] = {0, 0, 0, 0, 0, 0, 0};
       for (int a0 = 0; a0 < N; a0 += 256) {
-        double e[7] = {0, 0, 0, 0, 0, 0, 0}, e2[7] = {0, 0, 0, 0, 0, 0, 0};
-        if (tid < H && a0 + tid < N) bead_energy(P, D, r, a0 + tid, J.e_coef, 1.0 / J.e_lam, mc, xr, e);
-        if (B < 256 && tid < H && a0 + tid + 128 < N)
-          bead_energy(P, D, r, a0 + tid + 128, J.e_coef, 1.0 / J.e_lam, mc, xr, e2);
-        for (int k = 1; k < 7; k++) {
-          if (tid < H) s1[tid] = B < 256 ? e[k] + e2[k] : e[k];
-          __syncthreads();
-          for (int off = H / 2; off > 0; off >>= 1) {
-            if (tid < off) s1[tid] += s1[tid + off];
-            __syncthreads();
+        for (int t = tid / ENE_LPB; t < 256; t += B / ENE_LPB) {
+          double e[7] = {0, 0, 0, 0, 0, 0, 0};
+          if (a0 + t < N) bead_energy(P, D, r, a0 + t, J.e_coef, 1.0 / J.e_lam, mc, xr, e, l4, ENE_LPB);
+          for (int k = 1; k < 7; k++) {
+            for (int off = 1; off < ENE_LPB; off <<= 1) e[k] += __shfl_xor(e[k], off);
+            if (l4 == 0) se[(k - 1) * 256 + t] = e[k];
           }
-          if (tid == 0) acc[k] += s1[0];
+        }
+        __syncthreads();
+        for (int off = 128; off > 0; off >>= 1) {
+          for (int q = tid; q < 6 * off; q += B) {
+            double *p = se + q / off * 256 + q % off;
+            p[0] += p[off];
+          }
           __syncthreads();
         }
+        if (tid == 0)
+          for (int k = 1; k < 7; k++) acc[k] += se[(k - 1) * 256];
+        __syncthreads();
       }
       if (tid == 0) {
         double t = 0.0;
