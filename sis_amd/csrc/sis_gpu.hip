@@ -1165,6 +1165,13 @@ bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
   return huge;
 }
 
+// Beads from which the state is packed on the device (k_state_in / _out).
+// Below, the launch and the copy it is followed by cost more than one core's
+// packing: state in / out of 64 beads 43 / 45 us by the host, 52 / 77 by the
+// device, of 9,400 73 / 90 and 90 / 112, of 16,000 102 / 132 and 107 / 139,
+// of 32,000 182 / 234 and 142 / 201.
+constexpr size_t STATE_ON_DEVICE = 20000;
+
 constexpr size_t STEP_MARKS = 4096;
 
 inline int pad8(int64_t n) { return (int)((n + 7) / 8 * 8); }
@@ -1591,7 +1598,8 @@ int sis_gpu_create(const sis_topo *topo, const sis_params *prm, const sis_option
     c->bpp_d.alloc(7);
     HIPCHK(hipMemcpy(c->bpp_d.p, c->bpp_h, sizeof c->bpp_h, hipMemcpyHostToDevice));
     c->ecT_d.alloc(R); c->eCoef_d.alloc(R); c->eLam_d.alloc(R);
-    c->pos_d.alloc(RN); c->pos2_d.alloc(RN); c->fbond_d.alloc(RN); c->vel_d.alloc(RN); c->acc_d.alloc(RN); c->move_d.alloc(RN); c->frc_d.alloc(RN); c->state3_d.alloc(3 * RN);
+    c->pos_d.alloc(RN); c->pos2_d.alloc(RN); c->fbond_d.alloc(RN); c->vel_d.alloc(RN); c->acc_d.alloc(RN); c->move_d.alloc(RN); c->frc_d.alloc(RN);
+    if ((size_t)RN >= STATE_ON_DEVICE) c->state3_d.alloc(3 * RN);
     c->n_ele_d.alloc(RN); c->n_wca_d.alloc(RN); c->n_bp_tmp_d.alloc(RN); c->bp_off_d.alloc(RN + 1);
     c->n_bp_d.alloc(R); c->n_inc_d.alloc(RN); c->nt_cnt_d.alloc(RN); c->comp_d.alloc(RN);
     c->flags_d.alloc(8);
@@ -1642,7 +1650,14 @@ int sis_gpu_set_state(sis_gpu_ctx *c, const double *xyz, const double *velos, co
   API_BEGIN
   if (!c) return fail(SIS_ERR_ARG, "null context");
   const size_t RN = (size_t)c->R * c->N;
+  std::vector<double4> h(RN < STATE_ON_DEVICE ? RN : 0);
+  HIPCHK(hipStreamSynchronize(c->stream));
   auto up = [&](const double *src, DevBuf<double4> &dst) {
+    if (double4 *b = h.data()) {
+      for (size_t g = 0, n = RN; g < n; g++) b[g] = double4{src[3 * g], src[3 * g + 1], src[3 * g + 2], 0.0};
+      HIPCHK(hipMemcpy(dst.p, b, RN * sizeof(double4), hipMemcpyHostToDevice));
+      return;
+    }
     HIPCHK(hipMemcpyAsync(c->state3_d.p, src, 3 * RN * sizeof(double), hipMemcpyHostToDevice, c->stream));
     hipLaunchKernelGGL(k_state_in, dim3((unsigned)((RN + 255) / 256)), dim3(256), 0, c->stream, c->state3_d.p, dst.p, RN);
     HIPCHK(hipStreamSynchronize(c->stream));
@@ -1687,7 +1702,14 @@ int sis_gpu_get_state(sis_gpu_ctx *c, double *xyz, double *velos, double *accels
   API_BEGIN
   if (!c) return fail(SIS_ERR_ARG, "null context");
   const size_t RN = (size_t)c->R * c->N;
+  std::vector<double4> h(RN < STATE_ON_DEVICE ? RN : 0);
+  HIPCHK(hipStreamSynchronize(c->stream));
   auto down = [&](double *dst, DevBuf<double4> &src) {
+    if (double4 *b = h.data()) {
+      HIPCHK(hipMemcpy(b, src.p, RN * sizeof(double4), hipMemcpyDeviceToHost));
+      for (size_t g = 0, n = RN; g < n; g++) { dst[3 * g] = b[g].x; dst[3 * g + 1] = b[g].y; dst[3 * g + 2] = b[g].z; }
+      return;
+    }
     hipLaunchKernelGGL(k_state_out, dim3((unsigned)((RN + 255) / 256)), dim3(256), 0, c->stream, src.p, c->state3_d.p, RN);
     HIPCHK(hipMemcpyAsync(dst, c->state3_d.p, 3 * RN * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(hipStreamSynchronize(c->stream));
