@@ -87,6 +87,14 @@ struct TwzOut;
 
 // What captured per-phase steps take by value: their graph is replayed only
 // while all of it is unchanged.
+// Pinned host words of the step batches (a copy from or to pageable memory
+// would make the host wait for it)
+struct StepPin {
+  StepWords back[2];   // of the last two batches
+  StepWords up;
+  int rep[1];          // R: rebuild flags down, limit-MC flags up
+};
+
 struct PhaseGraphKey {
   Params P;
   Ptrs D;
@@ -225,7 +233,7 @@ struct sis_gpu_ctx {
   int dev = 0;   // the HIP device current when the context was created
   // replayed per-phase steps (phases_graph_steps)
   DevBuf<StepWords> g_step_d;
-  void *step_pin = nullptr;     // pinned copies of it, two batches' worth
+  struct StepPin *step_pin = nullptr;   // pinned: what goes up to it and comes back
   hipEvent_t step_ev[2] = {nullptr, nullptr};
   DevBuf<int> g_int_d;
   DevBuf<double4> step_fpair_d, step_noise_d;
@@ -1132,7 +1140,7 @@ bool graph_steps_ok(sis_gpu_ctx *c) { return !c->parity && !c->ext_on && c->opt.
 // component above the bucket capacity (k_step_huge).
 template <typename F>
 bool run_phase_batches(sis_gpu_ctx *c, int64_t stop, bool exact, F &&launch) {
-  StepWords *pin = static_cast<StepWords *>(c->step_pin);
+  StepWords *pin = c->step_pin->back;
   const int64_t base = c->istep;
   double4 *const pos0 = c->pos_d.p;
   int64_t issued = 0, nb = 0, nread = 0;
@@ -1191,7 +1199,8 @@ void step_buffers(sis_gpu_ctx *c) {
   if (c->step_top2_d.n < top2) c->step_top2_d.alloc(top2);
   if (c->P.nstep_bp_mc > 0 && c->seg_d.n < RN * SEGCAP) c->seg_d.alloc(RN * SEGCAP);
   if (c->P.nstep_bp_mc > 0 && c->exc_list_d.n < RN + 1) c->exc_list_d.alloc(RN + 1);
-  if (!c->step_pin) HIPCHK(hipHostMalloc(&c->step_pin, 2 * sizeof(StepWords), hipHostMallocDefault));
+  if (!c->step_pin)
+    HIPCHK(hipHostMalloc((void **)&c->step_pin, sizeof(StepPin) + c->R * sizeof(int), hipHostMallocDefault));
   for (auto &e : c->step_ev)
     if (!e) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
 }
@@ -1271,28 +1280,30 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
   while (c->istep < stop) {
     // a rebuild due from the last skin test, or lists not built yet
     // (src/job_md.F90:376-395); the rebuilt replicas do the limit MC first
+    StepPin *pin = c->step_pin;
     if (!c->lists_valid) {
       std::fill(flag.begin(), flag.end(), 1);
     } else {
-      HIPCHK(hipMemcpyAsync(flag.data(), c->rebuild_flag_d.p, R * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+      HIPCHK(hipMemcpyAsync(pin->rep, c->rebuild_flag_d.p, R * sizeof(int), hipMemcpyDeviceToHost, c->stream));
       HIPCHK(hipStreamSynchronize(c->stream));
+      flag.assign(pin->rep, pin->rep + R);
     }
     bool any = false;
     for (int r = 0; r < R; r++) any = any || flag[r];
-    std::vector<int> fmc(R, 0);
     if (any) {
       rebuild(c, flag);
       c->rebuilds++;
-      for (int r = 0; r < R; r++) fmc[r] = c->rebuilt[r] && mc_on ? 1 : 0;
+      for (int r = 0; r < R; r++) pin->rep[r] = c->rebuilt[r] && mc_on ? 1 : 0;
+      HIPCHK(hipMemcpyAsync(c->g_int_d.p, pin->rep, R * sizeof(int), hipMemcpyHostToDevice, c->stream));
     }
-    const StepWords w0{c->istep, stop, 0, any ? c->istep + 1 : -1, 0, 0, 0};
-    HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w0, sizeof w0, hipMemcpyHostToDevice, c->stream));
-    HIPCHK(hipMemcpyAsync(c->g_int_d.p, fmc.data(), R * sizeof(int), hipMemcpyHostToDevice, c->stream));
+    // (read by the device before the batches end, which the host waits for)
+    const int64_t force_step = any ? c->istep + 1 : -1;
+    pin->up = StepWords{c->istep, stop, 0, force_step, 0, 0, 0};
+    HIPCHK(hipMemcpyAsync(c->g_step_d.p, &pin->up, sizeof pin->up, hipMemcpyHostToDevice, c->stream));
     // no skin test before the first step: the rebuild above was its answer
     HIPCHK(hipMemsetAsync(c->step_top2_d.p, 0, (size_t)R * nblk * 2 * sizeof(double), c->stream));
     hipLaunchKernelGGL(k_mc_reset, grid_beads(N, R, 256), dim3(256), 0, c->stream, c->P, c->ptrs(), c->exc_cnt_d.p,
                        c->exc_fill_d.p, c->exc_list_d.p, nullptr);
-    HIPCHK(hipStreamSynchronize(c->stream));
     A.seg = c->seg_d.p;
     A.ncand = pad8(std::max<int64_t>(1, (c->D.maxbp + B - 1) / B));   // the capacity; the count is read on the device
     A.sep_huge = c->step_sep_huge ? 1 : 0;
@@ -1350,8 +1361,8 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
       // launch in every step
       c->step_sep_huge = true;
       A.sep_huge = 1;
-      const StepWords w1{c->istep, stop, 0, w0.force_step, 0, 0, 0};
-      HIPCHK(hipMemcpyAsync(c->g_step_d.p, &w1, sizeof w1, hipMemcpyHostToDevice, c->stream));
+      pin->up = StepWords{c->istep, stop, 0, force_step, 0, 0, 0};
+      HIPCHK(hipMemcpyAsync(c->g_step_d.p, &pin->up, sizeof pin->up, hipMemcpyHostToDevice, c->stream));
       A.nj = 1;
       launch_step(1, 0);
       HIPCHK(hipStreamSynchronize(c->stream));
