@@ -252,11 +252,17 @@ struct WaveSearch {
       D.n_ele[g] = o.ne;
       D.n_wca[g] = o.nw;
       D.n_bp_tmp[g] = nb;
+      // the sizes to grow to.  A first search may overflow at every bead: a
+      // maximum already there is only read (an atomic for each of 32,768
+      // beads on one word took 2.4 ms)
+      auto grow = [&](int k, int n) {
+        if (__hip_atomic_load(&D.flags[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < n) atomicMax(&D.flags[k], n);
+      };
       if (o.ne > D.maxnb || o.nw > D.maxw || o.nb > D.maxbpb) {
-        D.flags[0] = 1;
-        atomicMax(&D.flags[2], o.ne);
-        atomicMax(&D.flags[3], o.nw);
-        atomicMax(&D.flags[4], o.nb);
+        grow(0, 1);
+        grow(2, o.ne);
+        grow(3, o.nw);
+        grow(4, o.nb);
       }
     }
     if (!sorted && nb > 64) {
