@@ -1227,9 +1227,7 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
   A.nbead = bd ? 0 : pad8((int64_t)R * ((N + BEAD_TILE - 1) / BEAD_TILE));
   A.npair = (N + PAIR_TILE - 1) / PAIR_TILE;
   A.circ = c->circular ? 1 : 0;
-  // pair tiles of the three launches that carry them
   const int ntile = bd ? 0 : R * A.npair;
-  const int t1 = mc_on ? (int)(ntile * STEP_SHARE_BP) : ntile, t2 = mc_on ? (int)(ntile * (STEP_SHARE_BP + STEP_SHARE_SEG)) : ntile;
   std::vector<int> flag(R, 0);
   const int64_t stop = c->istep + nsteps;
   auto kernels = [&](auto zero, int part, int j) {
@@ -1237,17 +1235,14 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     A.j = j;
     const Ptrs D = c->ptrs();
     if (part == 0) {
-      A.p0 = 0; A.p1 = t1;
-      hipLaunchKernelGGL(k_step_bp<T>, dim3(A.ncand + A.nbead + t1), dim3(B), 0, c->stream, c->P, D, A);
+      A.ntile = mc_on ? 0 : ntile;
+      hipLaunchKernelGGL(k_step_bp<T>, dim3(A.ncand + A.nbead + A.ntile), dim3(B), 0, c->stream, c->P, D, A);
       if (mc_on) {
-        A.p0 = t1; A.p1 = t2;
-        A.nlist = A.ncand;
-        hipLaunchKernelGGL(k_step_seg<T>, dim3(A.nlist + t2 - t1), dim3(B), 0, c->stream, c->P, D, A);
-        A.p0 = t2; A.p1 = ntile;
-        // a wavefront for each component there may be, as far as the
-        // device holds them at once
-        A.nlist = pad8(std::min<int64_t>(2048, (int64_t)(RN + 63) / 64));
-        hipLaunchKernelGGL(k_step_mc<T>, dim3(A.nlist + ntile - t2), dim3(B), 0, c->stream, c->P, D, A);
+        hipLaunchKernelGGL(k_step_seg, dim3(A.ncand), dim3(B), 0, c->stream, c->P, D, A);
+        // a wavefront for each component there may be, up to the cap
+        A.nlist = pad8(std::min<int64_t>(STEP_MC_BLOCKS, (int64_t)(RN + 63) / 64));
+        A.ntile = ntile;
+        hipLaunchKernelGGL(k_step_mc<T>, dim3(A.nlist + ntile), dim3(B), 0, c->stream, c->P, D, A);
       }
     }
     if (A.sep_huge && mc_on) hipLaunchKernelGGL(k_step_huge, dim3(R), dim3(64), 0, c->stream, c->P, D, A);

@@ -4,10 +4,10 @@
 //
 //   k_step_bp    skin decision of the step; base-pair evaluation per
 //                candidate (+ union of formed pairs); bonded forces and noise
-//                of every bead; the first part of the pair forces
-//   k_step_seg   formed pairs bucketed by conflict component; more pair forces
-//   k_step_mc    limit MC, one wavefront per component with excess; the rest
-//                of the pair forces
+//                of every bead; the pair forces when the limit MC is off
+//   k_step_seg   formed pairs bucketed by conflict component
+//   k_step_mc    limit MC, one wavefront per component with excess; the pair
+//                forces
 //   k_step_move  base-pair forces gathered, GJF-2GJ (or Brownian) update,
 //                displacement top-2, reset of the step's scratch
 //
@@ -35,9 +35,21 @@ constexpr int PAIR_LPB = 8;                 // lanes per bead of a pair tile
 constexpr int PAIR_TILE = STEP_B / PAIR_LPB;
 constexpr int GRAPH_STEPS = 16;   // steps of a batch; even: the positions end in the buffer they started in
 
-// Shares of the pair tiles that run beside the evaluation and beside the
-// buckets; the rest runs beside the deletion chains.
-constexpr double STEP_SHARE_BP = 0.40, STEP_SHARE_SEG = 0.15;
+// Where the pair tiles run: beside the deletion chains of k_step_mc, or beside
+// the evaluation in k_step_bp when the limit MC is off and there is no
+// k_step_mc.  Microseconds a step with a share of them beside the evaluation
+// and beside the buckets instead (0.4 and 0.15, then 1 and 0, then none):
+// 94,000 beads FP32 119, 149, 106, FP64 130, 158, 116; 9,400 beads FP64 71.7,
+// 70.9, 69.7; 397 nt FP32 61.1, 60.4, 60.2; 64 x 128 nt FP32 90.0, 91.5, 90.4.
+// The evaluation needs 198 VGPRs and its blocks run two waves a SIMD, a pair
+// tile among them too; k_step_mc needs 133 and waits for few long chains.
+//
+// Blocks of k_step_mc that take components (a wavefront each): a cap, as the
+// listed ones are far fewer than the wavefronts there may be.  94,000 beads
+// (about 3,400 listed a step) FP32 / FP64: 256 blocks 106.6 / 113.7, 512 104.3
+// / 114.1, 1,024 105.4 / 115.9, 2,048 106.8 / 117.2, 4,096 107.0 / 117.2;
+// smaller systems the same with any of them.
+constexpr int STEP_MC_BLOCKS = 512;
 
 // Device words that steer the batches (written back to the host as they are).
 struct StepWords {
@@ -61,9 +73,9 @@ struct StepArgs {
   uint64_t seed;
   int nblk;                  // blocks of k_step_move per replica
   int ncand, nbead;          // leading blocks of k_step_bp: candidates, then bead tiles (multiples of 8)
-  int nlist;                 // leading blocks of k_step_seg / k_step_mc (a multiple of 8)
+  int nlist;                 // leading blocks of k_step_mc (a multiple of 8)
   int npair;                 // pair tiles per replica
-  int p0, p1;                // pair tiles of this launch, of R * npair
+  int ntile;                 // pair tiles of this launch: all R * npair or none
   int circ;                  // 1: some chain is circular (bonded terms per bead)
   int sep_huge;              // 1: k_step_huge runs in every step
   int j, nj;
@@ -221,8 +233,8 @@ __device__ __forceinline__ void pair_tile(const Params &P, const Ptrs &D, const 
 // xcd_tile)
 template <typename T>
 __device__ __forceinline__ void pair_block(const Params &P, const Ptrs &D, const StepArgs &A, int first) {
-  const int n = A.p1 - A.p0, id = blockIdx.x - first;
-  if (id < n) pair_tile<T>(P, D, A, A.p0 + xcd_tile(id, n));
+  const int id = blockIdx.x - first;
+  if (id < A.ntile) pair_tile<T>(P, D, A, xcd_tile(id, A.ntile));
 }
 
 template <typename T>
@@ -250,13 +262,8 @@ __global__ void __launch_bounds__(STEP_B) k_step_bp(Params P, Ptrs D, StepArgs A
   }
 }
 
-template <typename T>
 __global__ void __launch_bounds__(STEP_B) k_step_seg(Params P, Ptrs D, StepArgs A) {
   if (A.w->halt) return;
-  if ((int)blockIdx.x >= A.nlist) {
-    pair_block<T>(P, D, A, A.nlist);
-    return;
-  }
   const int gb = blockIdx.x * STEP_B + threadIdx.x;
   if (gb >= bp_count(P, D, -1) || !D.bp_status[gb]) return;
   const int r = D.bp_mp[(size_t)gb * 8 + 7];
