@@ -485,8 +485,8 @@ int sis_gpu_get_info(sis_gpu_ctx *ctx, int64_t *out, int32_t n);
  * launch of the step's dominant kernel during the last sis_gpu_step call
  * (the persistent / batched step kernel; the force + integrator kernel of
  * steps launched one by one, as with external terms; with SIS_OPT_NO_GRAPH
- * the few launches that share a step's work, taken together, of up to 4,096
- * steps), 4 = number of such launches (0: batches replayed from a graph). */
+ * the few launches that share a step's work, taken together, of one step in
+ * 16), 4 = number of launches timed (0: batches replayed from a graph). */
 double sis_gpu_last_kernel_ms(sis_gpu_ctx *ctx, int32_t which);
 
 /* ---- Job pool: the serving form -------------------------------------

@@ -1260,17 +1260,21 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     if (c->precision == 1) kernels(0.0f, part, j);
     else kernels(0.0, part, j);
   };
-  // sis_gpu_last_kernel_ms: events around each step issued directly by a
-  // context that asked for that, for the first STEP_MARKS of a call
+  // sis_gpu_last_kernel_ms: events around one step of every directly issued
+  // batch, in its middle, where the device has launches to go on with (around
+  // every step they took 9 us each)
   const bool marks = (c->opt.flags & SIS_OPT_NO_GRAPH) && c->time_steps;
+  std::vector<int64_t> marked;   // the steps timed here
+  int64_t issued = 0;
   auto launch_batch = [&](int n) {
     A.nj = n;
     for (int j = 0; j < n; j++) {
-      const bool m = marks && c->tev_used < 2 * STEP_MARKS;
-      if (m) c->tmark();
+      const bool m = marks && j == n / 2 && c->tev_used < 2 * STEP_MARKS;
+      if (m) { c->tmark(); marked.push_back(issued + j + 1); }
       launch_step(0, j);
       if (m) c->tmark();
     }
+    issued += n;
   };
   while (c->istep < stop) {
     // a rebuild due from the last skin test, or lists not built yet
@@ -1317,11 +1321,10 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     // which pays for large systems (a graph launch costs more per node
     // than a kernel launch here)
     if (c->pg_eager || (c->opt.flags & SIS_OPT_NO_GRAPH)) {
-      const size_t mark0 = c->tev_used;
-      const int64_t at = c->istep;
+      issued = c->istep;
       wait_huge = run_phase_batches(c, stop, true, launch_batch);
       // steps issued after a halt did nothing
-      c->tev_used = std::min(c->tev_used, mark0 + 2 * (size_t)(c->istep - at));
+      for (; !marked.empty() && marked.back() > c->istep; marked.pop_back()) c->tev_used -= 2;
     } else {
       int slot = -1;
       for (int q = 0; q < 2; q++)
