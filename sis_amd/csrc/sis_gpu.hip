@@ -1235,8 +1235,13 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
     A.j = j;
     const Ptrs D = c->ptrs();
     if (part == 0) {
-      A.ntile = mc_on ? 0 : ntile;
+      const bool own = !mc_on && ntile >= PAIR_OWN_LAUNCH;
+      A.ntile = mc_on || own ? 0 : ntile;
       hipLaunchKernelGGL(k_step_bp<T>, dim3(A.ncand + A.nbead + A.ntile), dim3(B), 0, c->stream, c->P, D, A);
+      if (own) {
+        A.ntile = ntile;
+        hipLaunchKernelGGL(k_step_pair<T>, dim3(ntile), dim3(B), 0, c->stream, c->P, D, A);
+      }
       if (mc_on) {
         hipLaunchKernelGGL(k_step_seg, dim3(A.ncand), dim3(B), 0, c->stream, c->P, D, A);
         // a wavefront for each component there may be, up to the cap

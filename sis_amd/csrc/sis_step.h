@@ -4,7 +4,8 @@
 //
 //   k_step_bp    skin decision of the step; base-pair evaluation per
 //                candidate (+ union of formed pairs); bonded forces and noise
-//                of every bead; the pair forces when the limit MC is off
+//                of every bead; the pair forces of a small system when the
+//                limit MC is off (k_step_pair after it: of a large one)
 //   k_step_seg   formed pairs bucketed by conflict component
 //   k_step_mc    limit MC, one wavefront per component with excess; the pair
 //                forces
@@ -35,8 +36,7 @@ constexpr int PAIR_LPB = 8;                 // lanes per bead of a pair tile
 constexpr int PAIR_TILE = STEP_B / PAIR_LPB;
 constexpr int GRAPH_STEPS = 16;   // steps of a batch; even: the positions end in the buffer they started in
 
-// Where the pair tiles run: beside the deletion chains of k_step_mc, or beside
-// the evaluation in k_step_bp when the limit MC is off and there is no
+// Where the pair tiles run with the limit MC: beside the deletion chains of
 // k_step_mc.  Microseconds a step with a share of them beside the evaluation
 // and beside the buckets instead (0.4 and 0.15, then 1 and 0, then none):
 // 94,000 beads FP32 119, 149, 106, FP64 130, 158, 116; 9,400 beads FP64 71.7,
@@ -44,6 +44,14 @@ constexpr int GRAPH_STEPS = 16;   // steps of a batch; even: the positions end i
 // The evaluation needs 198 VGPRs and its blocks run two waves a SIMD, a pair
 // tile among them too; k_step_mc needs 133 and waits for few long chains.
 //
+// Without the limit MC there is no k_step_mc.  Few tiles run beside the
+// evaluation in k_step_bp, which spares a launch; from PAIR_OWN_LAUNCH on they
+// have one to themselves (k_step_pair) and with it more waves a SIMD.
+// Microseconds a step in k_step_bp / alone, FP64 and FP32: 256 tiles 30.5 /
+// 34.8 and 27.4 / 32.0, 588 tiles 35.1 / 36.1 and 32.0 / 31.7, 940 tiles 44.2 /
+// 39.7 and 41.0 / 34.5, 2,938 tiles (94,000 beads) 103 / 75 and 92 / 64.
+constexpr int PAIR_OWN_LAUNCH = 640;
+
 // Blocks of k_step_mc that take components (a wavefront each): a cap, as the
 // listed ones are far fewer than the wavefronts there may be.  94,000 beads
 // (about 3,400 listed a step) FP32 / FP64: 256 blocks 106.6 / 113.7, 512 104.3
@@ -268,6 +276,13 @@ __global__ void __launch_bounds__(STEP_B) k_step_seg(Params P, Ptrs D, StepArgs 
   if (gb >= bp_count(P, D, -1) || !D.bp_status[gb]) return;
   const int r = D.bp_mp[(size_t)gb * 8 + 7];
   if (step_mc(P, A, r, A.w->step0 + A.j + 1)) seg_fill_one(P, D, gb, A.seg_n, A.seg, A.has_exc, A.exc_list);
+}
+
+// the pair tiles alone
+template <typename T>
+__global__ void __launch_bounds__(STEP_B) k_step_pair(Params P, Ptrs D, StepArgs A) {
+  if (A.w->halt) return;
+  pair_block<T>(P, D, A, 0);
 }
 
 template <typename T>

@@ -151,6 +151,28 @@ def _lattice(nch, n=100):
                        default_params(nl_margin=5.0))
 
 
+@pytest.mark.parametrize("nch,prec", [(204, 0), (205, 0), (205, 1)])
+def test_pair_tiles_without_limit_mc(nch, prec):
+    """Both sides of the rule that gives the pair tiles a launch of their own
+    when the limit MC is off (640 tiles of 32 beads)."""
+    print(f"[case] pair tiles without limit MC, {100 * nch} beads, prec {prec}", flush=True)
+    s = _lattice(nch)
+    s["params"]["nstep_bp_mc"] = 0
+    out = []
+    for general in (True, False):
+        e = Engine(s, mode="phases", precision=prec, seed=4)
+        if general:
+            e.set_external(dict(rg=1, rg_k=0.0, rg_0=10.0))
+        e.init_velocities()
+        e.neighbor_list(0)
+        e.step(20)
+        out.append(e.get_state())
+        e.close()
+    np.testing.assert_array_equal(out[0][2], out[1][2])
+    assert np.abs(out[0][0] - out[1][0]).max() < 1e-9
+    assert np.abs(out[0][1] - out[1][1]).max() < 1e-12
+
+
 def test_pool_counts_what_a_large_job_steps_with():
     """A job above one workgroup's size is charged for the buffers of its
     step batches (64 B a bead, 7.7 MB here) when it is admitted: as much as
