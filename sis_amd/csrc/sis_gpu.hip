@@ -1371,7 +1371,10 @@ void phases_graph_steps(sis_gpu_ctx *c, int64_t nsteps) {
       HIPCHK(hipStreamSynchronize(c->stream));
       c->istep++;
     }
-    hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(), c->step_top2_d.p, nblk);
+    if (nblk > 1024)
+      hipLaunchKernelGGL(k_skin<1024>, dim3(R), dim3(1024), 0, c->stream, c->P, c->ptrs(), c->step_top2_d.p, nblk);
+    else
+      hipLaunchKernelGGL(k_skin<256>, dim3(R), dim3(256), 0, c->stream, c->P, c->ptrs(), c->step_top2_d.p, nblk);
   }
 }
 

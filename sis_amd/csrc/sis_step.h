@@ -96,14 +96,95 @@ __device__ __forceinline__ bool step_mc(const Params &P, const StepArgs &A, int 
   return step % P.nstep_bp_mc == 0 || (step == A.w->force_step && A.force_mc[r]);
 }
 
+// The skin test of the last step for replica r, of all R in turn
+// (src/job_md.F90:376-395: sqrt(d2max) + sqrt(d2max_2nd) > nl_margin), from the
+// maxima that k_step_move left.  The maxima meet in the order of k_skin's tree,
+// which matters for a run that has blown up: a NaN maximum gives way to what it
+// is compared with, and that order lets every other block count.  Returns
+// whether one fires, to some threads of the block.  s: 2 x STEP_B doubles.
+__device__ __forceinline__ bool skin_fires(const Params &P, const StepArgs &A, double *s) {
+  const int t = threadIdx.x, L = t & 63, n = A.nblk;
+  // blocks b, b + stride, ... of replica r
+  auto take = [&](int r, int b, int stride, double &m1, double &m2) {
+    m1 = m2 = 0.0;
+    for (; b < n; b += stride) {
+      const double *q = A.top2 + ((size_t)r * n + b) * 2;
+      top2_merge(m1, m2, q[0], q[1]);
+    }
+  };
+  bool fire = false;
+  double m1, m2, x1, x2;
+  if (n <= 4) {
+    // a thread for each replica
+    for (int r = t; r < P.R; r += STEP_B) {
+      double m[4][2];
+#pragma unroll
+      for (int b = 0; b < 4; b++) {
+        take(r, b, 4, m[b][0], m[b][1]);
+        top2_merge(m[b][0], m[b][1], 0.0, 0.0);   // the empty rest of the tree
+      }
+      top2_merge(m[0][0], m[0][1], m[2][0], m[2][1]);
+      top2_merge(m[1][0], m[1][1], m[3][0], m[3][1]);
+      top2_merge(m[0][0], m[0][1], m[1][0], m[1][1]);
+      if (sqrt(m[0][0]) + sqrt(m[0][1]) > P.nl_margin) fire = true;
+    }
+    return fire;
+  }
+  if (n <= 64) {
+    // a wavefront for each replica
+    for (int r = t >> 6; r < P.R; r += STEP_B / 64) {
+      take(r, L, 64, m1, m2);
+      top2_merge(m1, m2, 0.0, 0.0);
+      for (int off = 32; off > 0; off >>= 1) {
+        x1 = __shfl_xor(m1, off);
+        x2 = __shfl_xor(m2, off);
+        top2_merge(m1, m2, x1, x2);
+      }
+      if (L == 0 && sqrt(m1) + sqrt(m2) > P.nl_margin) fire = true;
+    }
+    return fire;
+  }
+  for (int r = 0; r < P.R; r++) {
+    if (n <= 1024) {
+      take(r, t, STEP_B, m1, m2);
+    } else {   // k_skin<1024>
+      take(r, t, 1024, m1, m2);
+      take(r, t + 512, 1024, x1, x2);
+      top2_merge(m1, m2, x1, x2);
+      double y1, y2;
+      take(r, t + 256, 1024, x1, x2);
+      take(r, t + 768, 1024, y1, y2);
+      top2_merge(x1, x2, y1, y2);
+      top2_merge(m1, m2, x1, x2);
+    }
+    s[t] = m1;
+    s[STEP_B + t] = m2;
+    __syncthreads();
+    if (t < 64) {
+      top2_merge(m1, m2, s[t + 128], s[STEP_B + t + 128]);
+      x1 = s[t + 64];
+      x2 = s[STEP_B + t + 64];
+      top2_merge(x1, x2, s[t + 192], s[STEP_B + t + 192]);
+      top2_merge(m1, m2, x1, x2);
+      for (int off = 32; off > 0; off >>= 1) {
+        x1 = __shfl_xor(m1, off);
+        x2 = __shfl_xor(m2, off);
+        top2_merge(m1, m2, x1, x2);
+      }
+      if (t == 0 && sqrt(m1) + sqrt(m2) > P.nl_margin) fire = true;
+    }
+    __syncthreads();
+  }
+  return fire;
+}
+
 // Whether step j does nothing: an earlier step of the batch halted, the
 // stop is reached, a component waits for k_step_huge, or the skin test of
-// the last step (src/job_md.F90:376-395: sqrt(d2max) + sqrt(d2max_2nd) >
-// nl_margin) asks for a rebuild.  Every block of k_step_bp works it out from
+// the last step asks for a rebuild.  Every block of k_step_bp works it out from
 // the maxima k_step_move left (a few KB; a launch of its own took longer);
 // block 0 notes it for the other launches and the host.  Called by every
 // thread.
-__device__ __forceinline__ bool step_halted(const Params &P, const StepArgs &A, double (*s)[2]) {
+__device__ __forceinline__ bool step_halted(const Params &P, const StepArgs &A, double *s) {
   // (a block that starts late may see the word block 0 has just written:
   // its own answer would be the same)
   const bool before = A.w->halt != 0;
@@ -117,37 +198,7 @@ __device__ __forceinline__ bool step_halted(const Params &P, const StepArgs &A, 
     done = A.w->huge_step - 1;
   }
   h = __syncthreads_or(h || at >= A.w->stop) != 0;   // one answer for the block
-  if (!h) {
-    const int t = threadIdx.x;
-    int fire = 0;
-    if (A.nblk <= 4) {
-      // few blocks a replica: a thread for each replica
-      for (int r = t; r < P.R; r += STEP_B) {
-        double m1 = 0.0, m2 = 0.0;
-        for (int b = 0; b < A.nblk; b++) {
-          const double *q = A.top2 + ((size_t)r * A.nblk + b) * 2;
-          top2_merge(m1, m2, q[0], q[1]);
-        }
-        if (sqrt(m1) + sqrt(m2) > P.nl_margin) fire = 1;
-      }
-    } else {
-      for (int r = 0; r < P.R; r++) {
-        double m1 = 0.0, m2 = 0.0;
-        for (int b = t; b < A.nblk; b += STEP_B) {
-          const double *q = A.top2 + ((size_t)r * A.nblk + b) * 2;
-          top2_merge(m1, m2, q[0], q[1]);
-        }
-        for (int off = 32; off > 0; off >>= 1) top2_merge(m1, m2, __shfl_xor(m1, off), __shfl_xor(m2, off));
-        if ((t & 63) == 0) { s[t >> 6][0] = m1; s[t >> 6][1] = m2; }
-        __syncthreads();
-        m1 = s[0][0]; m2 = s[0][1];
-        for (int w = 1; w < STEP_B / 64; w++) top2_merge(m1, m2, s[w][0], s[w][1]);
-        if (sqrt(m1) + sqrt(m2) > P.nl_margin) fire = 1;
-        __syncthreads();
-      }
-    }
-    h = __syncthreads_or(fire) != 0;
-  }
+  if (!h) h = __syncthreads_or(skin_fires(P, A, s)) != 0;
   if (blockIdx.x == 0 && threadIdx.x == 0 && h && !before) {
     A.w->done = done;
     A.w->halt = 1;
@@ -248,7 +299,7 @@ __device__ __forceinline__ void pair_block(const Params &P, const Ptrs &D, const
 template <typename T>
 __global__ void __launch_bounds__(STEP_B) k_step_bp(Params P, Ptrs D, StepArgs A) {
   __shared__ double sf[9][STEP_B];
-  if (step_halted(P, A, reinterpret_cast<double(*)[2]>(sf[0]))) return;
+  if (step_halted(P, A, sf[0])) return;   // (two rows of it)
   const int64_t step = A.w->step0 + A.j + 1;
   const int blk = blockIdx.x;
   if (blk < A.ncand) {
@@ -342,6 +393,7 @@ __global__ void __launch_bounds__(STEP_B) k_step_move(Params P, Ptrs D, StepArgs
       A.has_exc[g] = 0;
     }
     m1 = move_bead(P, D, g, a, F, nz.x, nz.y, nz.z);
+    if (!(m1 > 0.0)) m1 = 0.0;   // a bead gone to NaN does not hide the others
   }
   for (int off = 32; off > 0; off >>= 1) top2_merge(m1, m2, __shfl_xor(m1, off), __shfl_xor(m2, off));
   if ((t & 63) == 0) { s[t >> 6][0] = m1; s[t >> 6][1] = m2; }

@@ -220,3 +220,37 @@ def test_step_time_without_graph():
     e.step(1)
     assert e.last_ms(4) == 1
     e.close()
+
+
+@pytest.mark.parametrize("integrator", [1, 2])
+@pytest.mark.parametrize("pairs,bad", [(64, 47), (512, 383), (1200, 1151), (9000, 8959)])
+def test_a_nan_bead_does_not_hide_the_others(integrator, pairs, bad):
+    """Two-bead chains out of each other's reach, the first ones stretched
+    (Brownian) or fast (Langevin) so that they move furthest by far, one in
+    the middle with a NaN coordinate (the last bead of a block of 32 and of
+    256, whose maximum stays NaN): the run rebuilds where it does with that
+    chain at rest, over few, tens and hundreds of blocks of maxima."""
+    print(f"[case] NaN bead, {pairs} pairs, integrator {integrator}", flush=True)
+    k = np.arange(pairs)
+    x = np.zeros((pairs, 2, 3))
+    x[:, 0] = np.stack([90.0 * (k % 30), 90.0 * (k // 30 % 30), 90.0 * (k // 900)], 1)
+    x[:, 1] = x[:, 0] + [5.9, 0.0, 0.0]
+    v = np.zeros_like(x)
+    if integrator == 2:
+        x[:3, 1, 0] += 40.0
+    else:
+        v[:3] = 10.0
+    out = []
+    for nan in (False, True):
+        if nan:
+            x[bad, 1, 0] = np.nan
+        s = configs._mk("pairs", ["AA"] * pairs, x.reshape(-1, 3),
+                        default_params(nl_margin=10.0, integrator=integrator, dt=0.05 if integrator == 1 else 0.005, ele_on=0))
+        e = Engine(s, mode="phases", seed=4)
+        e.set_state(None, v.reshape(1, -1, 3), 0.0 * v.reshape(1, -1, 3))
+        e.neighbor_list(0)
+        out.append([e.step(6) for _ in range(10)])
+        e.close()
+    print(f"[case] rebuilds {out}", flush=True)
+    assert sum(out[0]) > 0
+    assert out[0] == out[1]
