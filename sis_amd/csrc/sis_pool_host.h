@@ -157,8 +157,15 @@ bool job_admit(sis_pool *p, PoolJob &j) {
     job_release(p, j);
     return false;
   }
-  if (c->seg_d.n < (size_t)c->N * SEGCAP) c->seg_d.alloc((size_t)c->N * SEGCAP);
-  if (j.nmp > POOL_WG_MAX) step_buffers(c);
+  try {
+    if (c->seg_d.n < (size_t)c->N * SEGCAP) c->seg_d.alloc((size_t)c->N * SEGCAP);
+    if (j.nmp > POOL_WG_MAX) step_buffers(c);
+  } catch (const HipError &e) {   // out of memory: this job's matter alone
+    (void)hipGetLastError();
+    job_fail(p, j, e.msg);
+    job_release(p, j);
+    return false;
+  }
   j.slot = p->free_slots.back();
   p->free_slots.pop_back();
   int io[4] = {0, c->nbp_total, 0, 0};
