@@ -429,7 +429,7 @@ def main():
                     exchange_every=int(sysd.get("exchange_every", 0)))
         pe.set_state(x, v, a)
         pe.neighbor_list(0)
-        pe.step(min(steps, 50))
+        pe.step(min(steps, 200))
         dom_ms, dom_n = pe.last_ms(3), int(pe.last_ms(4))
         pe.close()
     eng.close()
