@@ -23,8 +23,8 @@
 // active, and the noise once per bead with every lane active.  With the
 // skin test, the resets and the large-component pass inside these launches
 // a step takes four launches where it took seven.  Before and after, one
-// MI355X, microseconds a step: 64 nt FP64 50 -> 33, 397 nt FP32 75 -> 62,
-// 9,400 beads FP64 79 -> 61, 94,000 beads FP32 139 -> 111.
+// MI355X, microseconds a step: 64 nt FP64 45 -> 28, 397 nt FP32 72 -> 54,
+// 9,400 beads FP64 82 -> 61, 94,000 beads FP32 141 -> 100.
 #pragma once
 #include "sis_kernels.h"
 
